@@ -77,6 +77,7 @@ rf_status sortpass_plan(Device& d, SortPass& S, hipStream_t s, uint64_t* counter
         }
         *err_out = e;
         S.n_f = misc[32];
+        P.fan_cnt = nullptr;  // the counts are known: later passes leave them
         break;
     }
     S.off.assign(nd, 0);

@@ -2108,14 +2108,9 @@ uint32_t raster_wg_per_cu(uint32_t tile_w, uint32_t chunk, uint32_t tile_h) {
 // gather writes into the main batch, whose descriptors of these draws hold
 // the fan counts the planning run found.
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ void put_fan(const BatchDesc& B, const DrawDesc* D, uint32_t di, const CV& a,
+// Fan f of the pass: its key, draw and clip-space vertices.
+__device__ __forceinline__ void put_fan(const BatchDesc& B, const DrawDesc* D, uint32_t di, uint32_t f, const CV& a,
                                         const CV& b, const CV& c, uint64_t g, uint32_t j) {
-    const uint32_t f = atomicAdd(B.fan_count, 1u);
-    if (B.fan_cnt) atomicAdd(&B.fan_cnt[di], 1u);
-    if (f >= B.fan_cap) {
-        atomicOr(B.err, ERRB_EXTRA);
-        return;
-    }
     const float z = ((a.p[2] + b.p[2]) + c.p[2]) / 3.0f;
     uint32_t k = (uint32_t)total_key(z) ^ 0x80000000u;  // ascending total order as unsigned
     if (D->sort == 2) k = ~k;                           // back to front
@@ -2130,34 +2125,68 @@ __device__ __forceinline__ void put_fan(const BatchDesc& B, const DrawDesc* D, u
     }
 }
 
+// Bound by the fan counter when every fan takes its index with an atomic of
+// its own: atomics on one address serialise in L2 (640,000 triangles in 4
+// draws: 6.71 ms, with one atomic a block 0.07). A block counts its fans first
+// and takes one range of indices; the order of the indices is of no account,
+// the sort keys are distinct. The per-draw counts, wanted by the planning run only, take one
+// atomic a wave where the wave's triangles are of one draw.
 __global__ __launch_bounds__(256) void k_fans(BatchDesc B) {
+    __shared__ uint32_t s_tot[4], s_base;
     const uint64_t g = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (g >= B.n_tris) return;
-    const uint32_t di = draw_of_tri(B.draws, B.n_draws, B.group_draw[g / WAVE], g);
-    if (B.any_cull && !B.draw_vis[di]) return;  // a draw the bounding-box test hid
-    const DrawDesc* D = &B.draws[di];
-    const uint64_t t = g - D->tri_base;
-    const uint32_t i0 = D->tris[3 * t], i1 = D->tris[3 * t + 1], i2 = D->tris[3 * t + 2];
-    if (i0 >= D->n_verts || i1 >= D->n_verts || i2 >= D->n_verts) {
-        atomicOr(B.err, ERRB_INDEX);
-        return;
-    }
+    const uint32_t lane = lane_id(), wave = threadIdx.x / WAVE;
+    uint32_t cnt = 0, di = 0;
+    const DrawDesc* D = nullptr;
     CV poly[CLIP_MAX], tmp[CLIP_MAX];
-    const uint64_t ix[3] = {D->vert_base + i0, D->vert_base + i1, D->vert_base + i2};
-    for (int k = 0; k < 3; ++k) {
-        const float4 p = B.cv[ix[k]], a = B.ca[ix[k]];
-        const float pp[4] = {p.x, p.y, p.z, p.w}, aa[3] = {a.x, a.y, a.z};
-        cv_make(poly[k], pp, aa);
+    if (g < B.n_tris) {
+        di = draw_of_tri(B.draws, B.n_draws, B.group_draw[g / WAVE], g);
+        D = &B.draws[di];
+        const uint64_t t = g - D->tri_base;
+        if (B.any_cull && !B.draw_vis[di]) {
+            // a draw the bounding-box test hid
+        } else if (D->tris[3 * t] >= D->n_verts || D->tris[3 * t + 1] >= D->n_verts ||
+                   D->tris[3 * t + 2] >= D->n_verts) {
+            atomicOr(B.err, ERRB_INDEX);
+        } else {
+            uint32_t all_out = ~0u, any_out = 0;
+            for (int k = 0; k < 3; ++k) {
+                const uint64_t ix = D->vert_base + D->tris[3 * t + k];
+                const float4 p = B.cv[ix], a = B.ca[ix];
+                const float pp[4] = {p.x, p.y, p.z, p.w}, aa[3] = {a.x, a.y, a.z};
+                cv_make(poly[k], pp, aa);
+                all_out &= poly[k].oc;
+                any_out |= poly[k].oc;
+            }
+            int n = 0;                                             // Hidden
+            if (all_out == 0) n = any_out == 0 ? 3 : clip_polygon(poly, 3, tmp);  // Visible or Clipped
+            if (n < 0) atomicOr(B.err, ERRB_CLIP);
+            cnt = n >= 3 ? (uint32_t)(n - 2) : 0u;
+        }
     }
-    const uint32_t all_out = poly[0].oc & poly[1].oc & poly[2].oc, any_out = poly[0].oc | poly[1].oc | poly[2].oc;
-    if (all_out != 0) return;  // Hidden
-    if (any_out == 0) {        // Visible
-        put_fan(B, D, di, poly[0], poly[1], poly[2], g, 0);
+    uint32_t tot;
+    const uint32_t pre = wave_excl_scan(cnt, &tot);
+    if (lane == 0) s_tot[wave] = tot;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        const uint32_t all = s_tot[0] + s_tot[1] + s_tot[2] + s_tot[3];
+        s_base = all ? atomicAdd(B.fan_count, all) : 0u;
+    }
+    __syncthreads();
+    if (B.fan_cnt) {
+        const uint32_t d0 = wave_min_u32(cnt ? di : 0xFFFFFFFFu), d1 = ~wave_min_u32(cnt ? ~di : 0xFFFFFFFFu);
+        if (d0 == d1) {
+            if (lane == 0) atomicAdd(&B.fan_cnt[d0], tot);
+        } else if (cnt) {
+            atomicAdd(&B.fan_cnt[di], cnt);
+        }
+    }
+    uint32_t f = s_base + pre;
+    for (uint32_t k = 0; k < wave; ++k) f += s_tot[k];
+    if (cnt && f + cnt > B.fan_cap) {
+        atomicOr(B.err, ERRB_EXTRA);
         return;
     }
-    const int n = clip_polygon(poly, 3, tmp);
-    if (n < 0) atomicOr(B.err, ERRB_CLIP);
-    for (int k = 1; k + 1 < n; ++k) put_fan(B, D, di, poly[0], poly[k], poly[k + 1], g, (uint32_t)(k - 1));
+    for (uint32_t k = 0; k < cnt; ++k) put_fan(B, D, di, f + k, poly[0], poly[k + 1], poly[k + 2], g, k);
 }
 
 // The second sort's keys: the draw of each fan in the first sort's order.
