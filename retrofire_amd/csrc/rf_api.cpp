@@ -105,15 +105,12 @@ static void scratch_arrays(BatchDesc& B, Fn&& fn) {
     const uint64_t ntl = std::max<uint64_t>(B.n_tiles, 1), nf = std::max<uint64_t>(B.n_frames, 1);
     void* misc = nullptr;
     fn(MISC_BYTES, &misc);
-    fn(nv * sizeof(float4), (void**)&B.cv);
-    fn(nv * sizeof(float4), (void**)&B.ca);
     fn(nv * 6 * sizeof(float), (void**)&B.sv);
     fn(nt * sizeof(uint32_t), (void**)&B.hdr);
     fn(nt * sizeof(ScrTri), (void**)&B.scr);
     fn(std::max<uint64_t>(B.extra_cap, 1) * sizeof(ScrTri), (void**)&B.extra);
     fn(nt * 2 * sizeof(uint32_t), (void**)&B.rect);
     fn((nt / 64 + 1) * sizeof(uint32_t), (void**)&B.group_draw);
-    fn((nv / 256 + 1) * sizeof(uint32_t), (void**)&B.vblock_draw);
     fn(ntl * sizeof(uint32_t), (void**)&B.run_count);
     fn((ntl + 1) * sizeof(uint32_t), (void**)&B.run_off);
     fn(ntl * sizeof(uint32_t), (void**)&B.run_cursor);
@@ -388,7 +385,6 @@ void plain_descs(const rf_draw* draw, const rf_target* target, const rf_ctx* ctx
     B.frames = (const FrameDesc*)((uint8_t*)P.desc + 256 * ((sizeof(DrawDesc) + 255) / 256));
     B.n_draws = 1;
     B.n_frames = 1;
-    B.n_verts = draw->n_verts;
     B.n_tris = draw->n_tris;
     B.n_groups = (uint32_t)((draw->n_tris + WAVE_SIZE - 1) / WAVE_SIZE);
     B.n_tiles = tile_base;

@@ -122,7 +122,7 @@ static rf_status build_descs(Batch& b, uint32_t tile_w, uint32_t tile_h, uint32_
             dd.vert_base = vbase;
             dd.tri_base = tbase;
             any_cull |= md.cull;
-            vbase += dd.n_verts;
+            vbase += dd.pre ? dd.n_verts : 0;
             tbase += dd.n_tris;
             b.frame_calls[fi] += 1;
             b.frame_objs[fi] += md.cull;

@@ -25,13 +25,11 @@ static void point_fans(SortPass& S) {
 rf_status sortpass_plan(Device& d, SortPass& S, hipStream_t s, uint64_t* counter, uint32_t* err_out) {
     *err_out = 0;
     const uint32_t nd = (uint32_t)S.draws.size();
-    uint64_t nv = 0, nt = 0;
+    uint64_t nt = 0;
     uint32_t any_cull = 0;
     for (DrawDesc& dd : S.draws) {
-        dd.vert_base = nv;
         dd.tri_base = nt;
         dd.pre = 0;
-        nv += dd.n_verts;
         nt += dd.n_tris;
         any_cull |= dd.cull;
     }
@@ -46,7 +44,6 @@ rf_status sortpass_plan(Device& d, SortPass& S, hipStream_t s, uint64_t* counter
     P.frames = S.frames;
     P.n_draws = nd;
     P.n_frames = S.frames_n;
-    P.n_verts = nv;
     P.n_tris = nt;
     P.n_groups = (uint32_t)((nt + WAVE_SIZE - 1) / WAVE_SIZE);
     P.any_cull = any_cull;

@@ -1,11 +1,9 @@
 // HIP kernels of the render path for gfx950 (CDNA4, wave64).
 //
-//   k_vertex   one thread per vertex slot: the built-in vertex shader
-//              (ProjMat3::apply, mat.rs:965-969), the outcode (clip.rs:303-309)
-//              and the screen-space vertex (prim.rs:62-88) used when the
-//              triangle needs no clipping.
 //   k_setup    one wave per group of 64 consecutive triangles: primitive
-//              assembly (prim.rs:17-19), frustum clipping (clip.rs:350-400),
+//              assembly (prim.rs:17-19), the built-in vertex shader at each
+//              corner (ProjMat3::apply, mat.rs:965-969), outcodes
+//              (clip.rs:303-309), frustum clipping (clip.rs:350-400),
 //              to_screen, face culling (render.rs:185-196), the tile rectangle
 //              of each triangle, and the per-tile count of bin runs.
 //   k_scan     exclusive scan of the run counts.
@@ -132,64 +130,6 @@ __device__ __forceinline__ uint32_t draw_of_tri(const DrawDesc* d, uint32_t n, u
     while (k + 1 < n && d[k + 1].tri_base <= g) ++k;
     return k;
 }
-__device__ __forceinline__ uint32_t draw_of_vert(const DrawDesc* d, uint32_t n, uint32_t hint, uint64_t s) {
-    uint32_t k = hint;
-    while (k + 1 < n && d[k + 1].vert_base <= s) ++k;
-    return k;
-}
-__device__ __forceinline__ uint32_t find_draw_vert(const DrawDesc* d, uint32_t n, uint64_t s) {
-    uint32_t lo = 0, hi = n;
-    while (hi - lo > 1) {
-        uint32_t mid = (lo + hi) >> 1;
-        if (d[mid].vert_base <= s) lo = mid; else hi = mid;
-    }
-    return lo;
-}
-
-// ---------------------------------------------------------------------------
-// k_vertex
-// ---------------------------------------------------------------------------
-#ifndef RF_RASTER_TU
-__global__ __launch_bounds__(256) void k_vertex(BatchDesc B) {
-    const uint64_t slot = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (slot >= B.n_verts) return;
-    const uint32_t di = draw_of_vert(B.draws, B.n_draws, B.vblock_draw[slot / 256], slot);
-    if (B.any_cull && !B.draw_vis[di]) return;  // a draw the bounding-box test hid: nothing reads these slots
-    const DrawDesc* D = &B.draws[di];
-    if (D->pre) return;  // filled by k_fan_gather
-    const uint64_t i = slot - D->vert_base;
-    const float px = D->pos[3 * i + 0], py = D->pos[3 * i + 1], pz = D->pos[3 * i + 2];
-    // vertex(mvp.apply(&v.pos), v.attrib): ProjMat3::apply, to_hom w = 1
-    const float* m = D->mvp;
-    const float x = dot4(m + 0, px, py, pz, 1.0f);
-    const float y = dot4(m + 4, px, py, pz, 1.0f);
-    const float z = dot4(m + 8, px, py, pz, 1.0f);
-    const float w = dot4(m + 12, px, py, pz, 1.0f);
-    const int na = kind_attrs(D->kind);
-    const uint64_t as = D->attr_stride;
-    float a0 = 0.0f, a1 = 0.0f, a2 = 0.0f;
-    if (na >= 2) {
-        a0 = D->attr[as * i + 0];
-        a1 = D->attr[as * i + 1];
-    }
-    if (na == 3) a2 = D->attr[as * i + 2];
-    const uint32_t oc = outcode(x, y, z, w);
-    B.cv[slot] = make_float4(x, y, z, w);
-    B.ca[slot] = make_float4(a0, a1, a2, u2f(oc));
-    // to_screen (prim.rs:62-88): (x/w, y/w, 1/w), viewport, attribute z_div
-    const float nx = x / w, ny = y / w, nz = 1.0f / w;
-    const float* v = D->vp;
-    float* s = B.sv + 6 * slot;
-    s[0] = dot4(v + 0, nx, ny, nz, 1.0f);
-    s[1] = dot4(v + 4, nx, ny, nz, 1.0f);
-    s[2] = dot4(v + 8, nx, ny, nz, 1.0f);
-    const bool persp = kind_persp(D->kind);
-    s[3] = persp ? a0 / w : a0;
-    s[4] = persp ? a1 / w : a1;
-    s[5] = persp ? a2 / w : a2;
-}
-#endif  // RF_RASTER_TU
-
 // ---------------------------------------------------------------------------
 // k_setup helpers: clipping in registers
 // ---------------------------------------------------------------------------
@@ -203,6 +143,35 @@ __device__ __forceinline__ void cv_make(CV& o, const float* p, const float* a) {
     for (int k = 0; k < 4; ++k) o.p[k] = p[k];
     for (int k = 0; k < 3; ++k) o.a[k] = a[k];
     o.oc = outcode(p[0], p[1], p[2], p[3]);
+}
+
+// vertex(mvp.apply(&v.pos), v.attrib) of the built-in vertex shader: the
+// clip position of a draw's vertex i (ProjMat3::apply, mat.rs:965-969, to_hom
+// w = 1) and its attributes. Shaded at each corner that names the vertex:
+// the same operations on the same inputs give the same bits, and a triangle's
+// corners cost less than writing every vertex of the mesh to HBM (56 bytes
+// each) and reading it back: 8 frames of 3.2M triangles took 0.36 ms in a
+// vertex kernel and 1.22 in k_setup, and take 1.25 in k_setup alone; 32 mixed
+// frames whose draws use a part of their mesh 1.27 + 2.67, now 2.80.
+__device__ __forceinline__ void shade_pos(const float* m, const float* pos, uint32_t i, float* p) {
+    const float x = pos[3ull * i], y = pos[3ull * i + 1], z = pos[3ull * i + 2];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) p[r] = dot4(m + 4 * r, x, y, z, 1.0f);
+}
+__device__ __forceinline__ void fetch_attr(const DrawDesc* D, uint32_t i, float* a) {
+    const int na = kind_attrs(D->kind);
+    const float* src = D->attr + (uint64_t)D->attr_stride * i;
+    a[0] = a[1] = a[2] = 0.0f;
+    if (na >= 2) {
+        a[0] = src[0];
+        a[1] = src[1];
+    }
+    if (na == 3) a[2] = src[2];
+}
+__device__ __forceinline__ void shade_vertex(const DrawDesc* D, uint32_t i, CV& o) {
+    shade_pos(D->mvp, D->pos, i, o.p);
+    fetch_attr(D, i, o.a);
+    o.oc = outcode(o.p[0], o.p[1], o.p[2], o.p[3]);
 }
 
 // Screen vertex of a clip vertex (to_screen, prim.rs:62-88).
@@ -241,6 +210,12 @@ __device__ int clip_polygon(CV* poly, int n, CV* tmp) {
     CV* out = tmp;
     for (int p = 0; p < 6; ++p) {
         const uint32_t bit = 1u << p;
+        // a plane that every vertex is inside of keeps them all and cuts no
+        // edge (no distance is > 0, so no product of two is < 0): most
+        // polygons meet one plane of the six
+        uint32_t any = 0;
+        for (int k = 0; k < n; ++k) any |= in[k].oc;
+        if ((any & bit) == 0) continue;
         int m = 0;
         for (int k = 0; k < n; ++k) {
             const CV& v0 = in[k];
@@ -400,25 +375,13 @@ __device__ uint32_t edge_setup(const BatchDesc& B, const DrawDesc* D, const Fram
         atomicOr(B.err, ERRB_INDEX);
         return 0;
     }
-    const uint64_t s0 = D->vert_base + i0, s1 = D->vert_base + i1;
-    const uint32_t o0 = f2u(B.ca[s0].w), o1 = f2u(B.ca[s1].w);
-    if (o0 & o1) return 0;  // both ends outside one plane
+    CV ea, eb;
+    shade_vertex(D, i0, ea);
+    shade_vertex(D, i1, eb);
+    if (ea.oc & eb.oc) return 0;  // both ends outside one plane
     const bool persp = kind_persp(D->kind);
     float a[6], b[6];
-    if ((o0 | o1) == 0) {
-        for (int c = 0; c < 6; ++c) {
-            a[c] = B.sv[6 * s0 + c];
-            b[c] = B.sv[6 * s1 + c];
-        }
-    } else {
-        CV ea, eb;
-        {
-            const float4 p0 = B.cv[s0], q0 = B.ca[s0], p1 = B.cv[s1], q1 = B.ca[s1];
-            const float pa[4] = {p0.x, p0.y, p0.z, p0.w}, aa[3] = {q0.x, q0.y, q0.z};
-            const float pb[4] = {p1.x, p1.y, p1.z, p1.w}, ab[3] = {q1.x, q1.y, q1.z};
-            cv_make(ea, pa, aa);
-            cv_make(eb, pb, ab);
-        }
+    if ((ea.oc | eb.oc) != 0) {
         for (int p = 0; p < 6; ++p) {
             const uint32_t bit = 1u << p;
             const bool a_in = (bit & ea.oc) == 0, b_in = (bit & eb.oc) == 0;
@@ -437,9 +400,9 @@ __device__ uint32_t edge_setup(const BatchDesc& B, const DrawDesc* D, const Fram
                 else if (b_in) ea = v;
             }
         }
-        to_screen(ea, D->vp, persp, a);
-        to_screen(eb, D->vp, persp, b);
     }
+    to_screen(ea, D->vp, persp, a);
+    to_screen(eb, D->vp, persp, b);
     if (F.face_cull == FC_FRONT) return 0;
     if (!(__builtin_isfinite(a[0]) && __builtin_isfinite(a[1]) && __builtin_isfinite(b[0]) &&
           __builtin_isfinite(b[1]))) {
@@ -510,8 +473,31 @@ __device__ uint32_t edge_setup(const BatchDesc& B, const DrawDesc* D, const Fram
 // k_setup
 // ---------------------------------------------------------------------------
 #ifndef RF_RASTER_TU
-// Eight waves per SIMD (at most 64 VGPRs): 0.092 -> 0.089 ms on crates1080.
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_setup(BatchDesc B) {
+// The corners of triangle (i0, i1, i2) of draw D: clip positions, outcodes,
+// and screen positions of a triangle that needs no clipping (prim.rs:62-88).
+// Called with D wave-uniform (the matrices come through scalar loads) or not.
+__device__ __forceinline__ void corners(const DrawDesc* D, const uint32_t* ix, float (&p)[3][4], uint32_t (&oc)[3],
+                                        float (&s)[3][3]) {
+    const float* const pos = D->pos;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        shade_pos(D->mvp, pos, ix[k], p[k]);
+        oc[k] = outcode(p[k][0], p[k][1], p[k][2], p[k][3]);
+    }
+    if ((oc[0] | oc[1] | oc[2]) == 0) {
+        const float* const v = D->vp;
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            const float w = p[k][3];
+            const float nx = p[k][0] / w, ny = p[k][1] / w, nz = 1.0f / w;
+            s[k][0] = dot4(v + 0, nx, ny, nz, 1.0f);
+            s[k][1] = dot4(v + 4, nx, ny, nz, 1.0f);
+            s[k][2] = dot4(v + 8, nx, ny, nz, 1.0f);
+        }
+    }
+}
+
+__global__ __launch_bounds__(256) void k_setup(BatchDesc B) {
     const uint32_t lane = lane_id();
     const uint32_t group = blockIdx.x * (blockDim.x / WAVE) + threadIdx.x / WAVE;
     if (group >= B.n_groups) return;  // whole wave exits together
@@ -521,8 +507,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8))) voi
     uint32_t rect[2] = {0, 0};
     bool has_rect = false;
     uint32_t frame = 0xFFFFFFFFu;
+    const uint32_t d0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)B.group_draw[group]);
+    const uint32_t di = valid ? draw_of_tri(B.draws, B.n_draws, d0, g) : d0;
+    const bool uniform = __ballot(di != d0) == 0ull;
     if (valid) {
-        const uint32_t di = draw_of_tri(B.draws, B.n_draws, B.group_draw[group], g);
         const DrawDesc* D = &B.draws[di];
         const FrameDesc& F = B.frames[D->frame];
         frame = D->frame;
@@ -535,39 +523,56 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8))) voi
                    D->tris[3 * t + 2] >= D->n_verts) {
             atomicOr(B.err, ERRB_INDEX);
         } else {
-            const uint32_t i0 = D->tris[3 * t], i1 = D->tris[3 * t + 1], i2 = D->tris[3 * t + 2];
-            const uint64_t s0 = D->vert_base + i0, s1 = D->vert_base + i1, s2 = D->vert_base + i2;
-            const uint32_t o0 = f2u(B.ca[s0].w), o1 = f2u(B.ca[s1].w), o2 = f2u(B.ca[s2].w);
-            const uint32_t all_out = o0 & o1 & o2, any_out = o0 | o1 | o2;
+            const uint32_t ix[3] = {D->tris[3 * t], D->tris[3 * t + 1], D->tris[3 * t + 2]};
+            float p[3][4], sp[3][3];
+            uint32_t oc[3] = {0, 0, 0};
+            if (!D->pre) {
+                if (uniform) corners(&B.draws[d0], ix, p, oc, sp);
+                else corners(D, ix, p, oc, sp);
+            }
+            const uint32_t all_out = oc[0] & oc[1] & oc[2], any_out = oc[0] | oc[1] | oc[2];
             RectAcc ra;
             ra.init();
             if (all_out != 0) {
                 // Hidden
             } else if (any_out == 0) {
-                // Visible: screen vertices were computed per vertex
-                float v0[6], v1[6], v2[6];
-                for (int c = 0; c < 6; ++c) {
-                    v0[c] = B.sv[6 * s0 + c];
-                    v1[c] = B.sv[6 * s1 + c];
-                    v2[c] = B.sv[6 * s2 + c];
+                // Visible
+                float v[3][6];
+                if (D->pre) {  // a depth-sorted clip fan's screen vertices
+#pragma unroll
+                    for (int k = 0; k < 3; ++k)
+#pragma unroll
+                        for (int c = 0; c < 6; ++c) v[k][c] = B.sv[6 * (D->vert_base + ix[k]) + c];
+                } else {
+#pragma unroll
+                    for (int k = 0; k < 3; ++k)
+#pragma unroll
+                        for (int c = 0; c < 3; ++c) v[k][c] = sp[k][c];
                 }
-                if (!culled(F.face_cull, backface(v0, v1, v2))) {
-                    write_scr(&B.scr[g], v0, v1, v2, di, D->kind);
-                    ra.add(v0);
-                    ra.add(v1);
-                    ra.add(v2);
+                if (!culled(F.face_cull, backface(v[0], v[1], v[2]))) {
+                    if (!D->pre) {
+                        const bool persp = kind_persp(D->kind);
+#pragma unroll
+                        for (int k = 0; k < 3; ++k) {
+                            float a[3];
+                            fetch_attr(D, ix[k], a);
+#pragma unroll
+                            for (int c = 0; c < 3; ++c) v[k][3 + c] = persp ? a[c] / p[k][3] : a[c];
+                        }
+                    }
+                    write_scr(&B.scr[g], v[0], v[1], v[2], di, D->kind);
+                    ra.add(v[0]);
+                    ra.add(v[1]);
+                    ra.add(v[2]);
                     nf = 1;
                 }
             } else {
                 // Clipped
                 CV poly[CLIP_MAX], tmp[CLIP_MAX];
-                const uint64_t ss[3] = {s0, s1, s2};
                 for (int k = 0; k < 3; ++k) {
-                    const float4 p = B.cv[ss[k]];
-                    const float4 a = B.ca[ss[k]];
-                    const float pp[4] = {p.x, p.y, p.z, p.w};
-                    const float aa[3] = {a.x, a.y, a.z};
-                    cv_make(poly[k], pp, aa);
+                    for (int c = 0; c < 4; ++c) poly[k].p[c] = p[k][c];
+                    fetch_attr(D, ix[k], poly[k].a);
+                    poly[k].oc = oc[k];
                 }
                 const int n = clip_polygon(poly, 3, tmp);
                 if (n < 0) atomicOr(B.err, ERRB_CLIP);
@@ -2101,9 +2106,9 @@ uint32_t raster_wg_per_cu(uint32_t tile_w, uint32_t chunk, uint32_t tile_h) {
 //                 stable sort by draw, so each draw's fans are contiguous and
 //                 in order (each render() call sorts its own primitives);
 //   k_fan_gather  fan i of the sorted order becomes vertex slots
-//                 3i'..3i'+2 of its draw, i' its rank in the draw (clip
-//                 position, attributes, outcode 0, screen vertex): the main
-//                 pipeline then draws them as unclipped triangles.
+//                 3i'..3i'+2 of its draw, i' its rank in the draw (screen
+//                 vertices): the main pipeline then draws them as unclipped
+//                 triangles.
 // The sorted draws form a batch of their own (their original meshes); the
 // gather writes into the main batch, whose descriptors of these draws hold
 // the fan counts the planning run found.
@@ -2129,8 +2134,8 @@ __device__ __forceinline__ void put_fan(const BatchDesc& B, const DrawDesc* D, u
 // its own: atomics on one address serialise in L2 (640,000 triangles in 4
 // draws: 6.71 ms, with one atomic a block 0.07). A block counts its fans first
 // and takes one range of indices; the order of the indices is of no account,
-// the sort keys are distinct. The per-draw counts, wanted by the planning run only, take one
-// atomic a wave where the wave's triangles are of one draw.
+// the sort keys are distinct. The per-draw counts, wanted by the planning run
+// only, take one atomic a wave where the wave's triangles are of one draw.
 __global__ __launch_bounds__(256) void k_fans(BatchDesc B) {
     __shared__ uint32_t s_tot[4], s_base;
     const uint64_t g = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -2150,10 +2155,7 @@ __global__ __launch_bounds__(256) void k_fans(BatchDesc B) {
         } else {
             uint32_t all_out = ~0u, any_out = 0;
             for (int k = 0; k < 3; ++k) {
-                const uint64_t ix = D->vert_base + D->tris[3 * t + k];
-                const float4 p = B.cv[ix], a = B.ca[ix];
-                const float pp[4] = {p.x, p.y, p.z, p.w}, aa[3] = {a.x, a.y, a.z};
-                cv_make(poly[k], pp, aa);
+                shade_vertex(D, D->tris[3 * t + k], poly[k]);
                 all_out &= poly[k].oc;
                 any_out |= poly[k].oc;
             }
@@ -2214,8 +2216,6 @@ __global__ __launch_bounds__(256) void k_fan_gather(BatchDesc P, BatchDesc M, co
         CV c;
         for (int e = 0; e < 4; ++e) c.p[e] = src[7 * q + e];
         for (int e = 0; e < 3; ++e) c.a[e] = src[7 * q + 4 + e];
-        M.cv[slot] = make_float4(c.p[0], c.p[1], c.p[2], c.p[3]);
-        M.ca[slot] = make_float4(c.a[0], c.a[1], c.a[2], u2f(0u));  // inside: clipped already
         to_screen(c, D->vp, persp, M.sv + 6 * slot);
         idx[3ull * i + q] = 3u * rank + (uint32_t)q;
     }
@@ -2260,9 +2260,8 @@ __global__ __launch_bounds__(256) void k_cull(BatchDesc B) {
 __global__ void k_reset(BatchDesc B) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < B.n_tiles) B.run_count[i] = 0;
-    // the draw of each group's first triangle and of each block's first vertex
+    // the draw of each group's first triangle
     if (i < B.n_groups) B.group_draw[i] = find_draw_tri(B.draws, B.n_draws, (uint64_t)i * WAVE);
-    if ((uint64_t)i * 256 < B.n_verts) B.vblock_draw[i] = find_draw_vert(B.draws, B.n_draws, (uint64_t)i * 256);
     if (i < B.n_frames * PRIM_PARTS) B.prims_part[(uint64_t)i * PRIM_PART_STRIDE] = 0;
     if (i < B.n_frames) {
         B.stats[i].prims_o = 0;
@@ -2292,8 +2291,6 @@ static hipError_t launch_impl(const BatchDesc& B0, hipStream_t s, uint32_t raste
     B.clear_in_raster = RF_CLEAR_IN_RASTER;
     uint32_t reset_n = B.n_tiles > B.n_frames * PRIM_PARTS ? B.n_tiles : B.n_frames * PRIM_PARTS;
     reset_n = reset_n > B.n_groups ? reset_n : B.n_groups;
-    const uint32_t n_vblocks = (uint32_t)((B.n_verts + 255) / 256);
-    reset_n = reset_n > n_vblocks ? reset_n : n_vblocks;
     auto mark = [&](int i) {
         if (ev) (void)hipEventRecord(ev[i], s);
     };
@@ -2304,8 +2301,6 @@ static hipError_t launch_impl(const BatchDesc& B0, hipStream_t s, uint32_t raste
     mark(0);
     hipLaunchKernelGGL(k_reset, dim3((reset_n + 255) / 256 + 1), dim3(256), 0, s, B);
     if (B.any_cull) hipLaunchKernelGGL(k_cull, dim3((B.n_draws + 255) / 256), dim3(256), 0, s, B);
-    if (B.n_verts)
-        hipLaunchKernelGGL(k_vertex, dim3((uint32_t)((B.n_verts + 255) / 256)), dim3(256), 0, s, B);
     mark(1);
     if (B.n_groups) hipLaunchKernelGGL(k_setup, dim3((B.n_groups + 3) / 4), dim3(256), 0, s, B);
     mark(2);
@@ -2334,11 +2329,8 @@ hipError_t launch_fans(const BatchDesc& B, hipStream_t s) {
     uint32_t reset_n = B.n_tiles > B.n_frames * PRIM_PARTS ? B.n_tiles : B.n_frames * PRIM_PARTS;
     reset_n = reset_n > B.n_groups ? reset_n : B.n_groups;
     reset_n = reset_n > B.n_draws ? reset_n : B.n_draws;
-    const uint32_t n_vblocks = (uint32_t)((B.n_verts + 255) / 256);
-    reset_n = reset_n > n_vblocks ? reset_n : n_vblocks;
     hipLaunchKernelGGL(k_reset, dim3((reset_n + 255) / 256 + 1), dim3(256), 0, s, B);
     if (B.any_cull) hipLaunchKernelGGL(k_cull, dim3((B.n_draws + 255) / 256), dim3(256), 0, s, B);
-    if (B.n_verts) hipLaunchKernelGGL(k_vertex, dim3(n_vblocks), dim3(256), 0, s, B);
     if (B.n_tris) hipLaunchKernelGGL(k_fans, dim3((uint32_t)((B.n_tris + 255) / 256)), dim3(256), 0, s, B);
     return hipGetLastError();
 }
@@ -2349,7 +2341,7 @@ hipError_t launch_fan_draw_keys(const uint32_t* order, const uint32_t* fan_draw,
 }
 hipError_t launch_fan_gather(const BatchDesc& P, const BatchDesc& M, const uint32_t* order, const uint32_t* draws_of,
                              const uint32_t* map, uint32_t n_fans, uint32_t* idx, hipStream_t s) {
-    if (n_fans && (!P.fans || !order || !map || !idx || !M.cv || !M.ca || !M.sv)) return hipErrorInvalidValue;
+    if (n_fans && (!P.fans || !order || !map || !idx || !M.sv)) return hipErrorInvalidValue;
     if (n_fans)
         hipLaunchKernelGGL(k_fan_gather, dim3((n_fans + 255) / 256), dim3(256), 0, s, P, M, order, draws_of, map,
                            n_fans, idx);

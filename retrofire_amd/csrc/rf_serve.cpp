@@ -141,11 +141,10 @@ constexpr uint32_t STAGE_DRAWS = 8;  // draws per frame the staging is sized for
 
 // Counts of a launch: what its block must hold.
 struct Plan {
-    uint64_t n_verts = 0, n_tris = 0, n_draws = 0, n_frames = 0, n_tiles = 0, targets = 0;
+    uint64_t n_tris = 0, n_draws = 0, n_frames = 0, n_tiles = 0, targets = 0;
     bool sorted = false;  // a depth-sorted launch: its scratch is the lane's own
     void add(const Req& q) {
         sorted = sorted || q.sorted;
-        n_verts += q.n_verts;
         n_tris += q.n_tris;
         n_draws += q.draws.size();
         n_frames += 1;
@@ -270,7 +269,6 @@ static uint32_t est_runs(const Serve& s, const Plan& p) {
 static uint64_t block_bytes(const Plan& p, uint32_t extra, uint32_t runs) {
     BatchDesc B;
     std::memset(&B, 0, sizeof(B));
-    B.n_verts = p.n_verts;
     B.n_tris = p.n_tris;
     B.n_draws = (uint32_t)p.n_draws;
     B.n_frames = (uint32_t)p.n_frames;
@@ -388,7 +386,7 @@ static FrameDesc frame_desc(const Req& q, uint8_t*& tgt, uint32_t& tile_base) {
     return f;
 }
 
-// A draw's descriptor (vert_base and tri_base left at 0).
+// A draw's descriptor (tri_base left at 0).
 static DrawDesc draw_desc(const rf_mesh_draw& md, uint32_t fi) {
     const Mesh* m = reinterpret_cast<const Mesh*>(md.mesh);
     const Tex* t = reinterpret_cast<const Tex*>(md.tex);
@@ -496,7 +494,7 @@ static rf_status launch_lane_sorted(Serve& s, Lane& l) {
         dd.vert_base = vbase;
         dd.tri_base = tbase;
         any_cull |= dd.cull;
-        vbase += dd.n_verts;
+        vbase += dd.pre ? dd.n_verts : 0;
         tbase += dd.n_tris;
         dds.push_back(dd);
     }
@@ -556,7 +554,6 @@ static rf_status launch_lane(Serve& s, Lane& l) {
     B.frames = (const FrameDesc*)(blk + db);
     B.n_draws = (uint32_t)p.n_draws;
     B.n_frames = (uint32_t)p.n_frames;
-    B.n_verts = p.n_verts;
     B.n_tris = p.n_tris;
     B.n_groups = (uint32_t)((p.n_tris + WAVE_SIZE - 1) / WAVE_SIZE);
     B.n_tiles = (uint32_t)p.n_tiles;
@@ -574,17 +571,15 @@ static rf_status launch_lane(Serve& s, Lane& l) {
     std::vector<FrameDesc> fds;
     dds.reserve(p.n_draws);
     fds.reserve(p.n_frames);
-    uint64_t vbase = 0, tbase = 0;
+    uint64_t tbase = 0;
     uint32_t tile_base = 0, any_cull = 0;
     for (size_t i = 0; i < l.reqs.size(); ++i) {
         Req& q = l.reqs[i];
         fds.push_back(frame_desc(q, tgt, tile_base));
         for (const rf_mesh_draw& md : q.draws) {
             DrawDesc dd = draw_desc(md, (uint32_t)i);
-            dd.vert_base = vbase;
             dd.tri_base = tbase;
             any_cull |= md.cull;
-            vbase += dd.n_verts;
             tbase += dd.n_tris;
             dds.push_back(dd);
         }

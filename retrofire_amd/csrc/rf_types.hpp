@@ -91,7 +91,7 @@ struct DrawDesc {
     uint32_t pre;                       // 1: vertex slots already filled (depth-sorted clip fans)
     uint32_t sort;                      // depth sort of this render() call: 0 none, 1 front to back, 2 back to front
     uint32_t in_tris, in_verts;         // a pre draw's render() input counts (prims.i, verts.i), for culled draws
-    uint64_t vert_base;                 // first slot in the batch vertex buffers
+    uint64_t vert_base;                 // a pre draw's first slot in the batch's screen vertices
     uint64_t tri_base;                  // first global triangle index
     float mvp[16];                      // row-major ProjMat3 (the uniform)
     float vp[16];                       // row-major Mat4<Ndc, Screen>
@@ -146,7 +146,7 @@ struct BatchDesc {
     const FrameDesc* frames;
     FrameStats* stats;
     uint32_t n_draws, n_frames;
-    uint64_t n_verts;   // total vertex slots
+    uint64_t n_verts;   // vertex slots of the pre draws
     uint64_t n_tris;    // total input triangles
     uint32_t n_groups;  // ceil(n_tris / 64)
     uint32_t n_tiles;   // total tiles over all frames
@@ -154,9 +154,7 @@ struct BatchDesc {
     uint32_t chunk;     // rasterizer span chunk: 6 or 8 pixels (anything else: 8)
     uint32_t sort_tpw;  // tiles per k_binsort wave (1..64; 0: the default, 8)
     // scratch
-    float4* cv;          // clip-space position per vertex slot
-    float4* ca;          // clip attributes (a0, a1, a2, outcode bits)
-    float* sv;           // screen vertex (x, y, z, a0, a1, a2) per slot
+    float* sv;           // screen vertex (x, y, z, a0, a1, a2) per slot of the pre draws
     uint32_t* hdr;       // per triangle: surviving fan count | extra base << 3
     ScrTri* scr;         // per triangle: first surviving fan
     ScrTri* extra;       // further fans of clipped triangles
@@ -172,7 +170,6 @@ struct BatchDesc {
     uint32_t* busy_count;  // their number
     uint32_t clear_in_raster;  // 1: the rasterizer clears the tiles without runs itself
     uint32_t* group_draw;   // per 64-triangle group: the draw of its first triangle
-    uint32_t* vblock_draw;  // per 256 vertex slots: the draw of the first
     Run* runs;
     uint32_t runs_cap;
     uint32_t* tile_counter;  // persistent raster work counters, one per tile partition (TILE_PARTS)
