@@ -110,6 +110,7 @@ static void scratch_arrays(BatchDesc& B, Fn&& fn) {
     fn(nt * sizeof(ScrTri), (void**)&B.scr);
     fn(std::max<uint64_t>(B.extra_cap, 1) * sizeof(ScrTri), (void**)&B.extra);
     fn(nt * 2 * sizeof(uint32_t), (void**)&B.rect);
+    fn(nt * sizeof(float), (void**)&B.zmax);
     fn((nt / 64 + 1) * sizeof(uint32_t), (void**)&B.group_draw);
     fn(ntl * sizeof(uint32_t), (void**)&B.run_count);
     fn((ntl + 1) * sizeof(uint32_t), (void**)&B.run_off);

@@ -275,7 +275,7 @@ struct RectAcc {
     }
 };
 
-// Tile rectangle of a triangle's pixels. Rows are exact: tri_fill covers rows
+// Pixel rectangle that holds a triangle's pixels. Rows are exact: tri_fill covers rows
 // floor(top_y + 0.5) .. floor(bot_y + 0.5) (scan, raster.rs:286-300). Columns
 // are the vertex x range widened by a margin that bounds how far the serially
 // stepped edges drift from the exact edges (the rasterizer checks every span
@@ -302,8 +302,7 @@ __device__ __forceinline__ int32_t bin_margin(const RectAcc& r, float rows) {
 // 0/0) draws no pixel, but its rows whose left edge is NaN are spans
 // `0..x1` (`x0 as usize` of NaN is 0, raster.rs:104-107) that count in
 // frags.i: its columns start at 0.
-__device__ __forceinline__ bool tile_rect(const RectAcc& r, const FrameDesc& F, uint32_t tw, uint32_t th_log2,
-                                          uint32_t* out) {
+__device__ __forceinline__ bool pixel_rect(const RectAcc& r, const FrameDesc& F, uint32_t* out) {
     const float r0 = floorf(r.ymin + 0.5f), r1 = floorf(r.ymax + 0.5f);
     if (!(r1 > r0)) return false;
     int64_t row0 = (int64_t)r0, row1 = (int64_t)r1 - 1;
@@ -317,11 +316,15 @@ __device__ __forceinline__ bool tile_rect(const RectAcc& r, const FrameDesc& F, 
     if (row1 >= (int64_t)F.height) row1 = (int64_t)F.height - 1;
     if (c1 >= (int64_t)F.width) c1 = (int64_t)F.width - 1;
     if (row1 < row0 || c1 < c0) return false;
-    const uint32_t tx0 = (uint32_t)(c0 / tw), tx1 = (uint32_t)(c1 / tw);
-    const uint32_t ty0 = (uint32_t)row0 >> th_log2, ty1 = (uint32_t)row1 >> th_log2;
-    out[0] = tx0 | (ty0 << 16);
-    out[1] = tx1 | (ty1 << 16);
+    out[0] = (uint32_t)c0 | ((uint32_t)row0 << 16);
+    out[1] = (uint32_t)c1 | ((uint32_t)row1 << 16);
     return true;
+}
+
+// The tiles (of 1 << twl columns x 1 << thl rows) a pixel rectangle meets:
+// one corner's tile column | tile row << 16.
+__device__ __forceinline__ uint32_t rect_tile(uint32_t corner, uint32_t twl, uint32_t thl) {
+    return ((corner & 0xFFFFu) >> twl) | ((corner >> 16 >> thl) << 16);
 }
 
 // Visit, over the whole wave, each distinct tile in the union of the lanes'
@@ -349,13 +352,6 @@ __device__ __forceinline__ void for_each_tile(bool valid, uint32_t r0, uint32_t 
             }
         }
     }
-}
-
-// Tile rectangle of an exact pixel rectangle (rows r0..r1, columns c0..c1).
-__device__ __forceinline__ void tile_rect_px(uint32_t r0, uint32_t r1, uint32_t c0, uint32_t c1, uint32_t tw,
-                                             uint32_t th_log2, uint32_t* out) {
-    out[0] = (c0 / tw) | ((r0 >> th_log2) << 16);
-    out[1] = (c1 / tw) | ((r1 >> th_log2) << 16);
 }
 
 // One Edge<usize> primitive (prim.rs:41-60): assembly, edge clipping
@@ -462,11 +458,187 @@ __device__ uint32_t edge_setup(const BatchDesc& B, const DrawDesc* D, const Fram
     d[9] = step;
     d[10] = u2f(wide ? 1u : 0u);
     d[11] = 0.0f;
-    const uint32_t th_log2 = (uint32_t)__builtin_ctz(B.tile_h);
-    if (wide) tile_rect_px((uint32_t)lo, (uint32_t)hi, S, S + n - 1, B.tile_w, th_log2, rect);
-    else tile_rect_px(S, S + n - 1, (uint32_t)lo, (uint32_t)hi, B.tile_w, th_log2, rect);
+    const uint32_t w0 = S, w1 = S + n - 1, t0 = (uint32_t)lo, t1 = (uint32_t)hi;
+    rect[0] = wide ? (w0 | t0 << 16) : (t0 | w0 << 16);
+    rect[1] = wide ? (w1 | t1 << 16) : (t1 | w1 << 16);
     has_rect = true;
     return 1;
+}
+
+struct Trap {
+    float y0i;             // first row (floor(y0 + 0.5))
+    uint32_t n;            // row count
+    float lx, lz, la[3];   // left state at the first row
+    float dlx, dlz, dla[3];
+    float rx, drx;         // right x at the first row, step
+    float dvz, dva[3];     // d(varyings)/dx
+};
+struct Slot {
+    Trap t[2];
+    int32_t ylo, yhi;      // rows covered (absolute)
+};
+
+// scan (raster.rs:248-302) for one trapezoid; y components are not needed by
+// any output and are left out.
+__device__ __forceinline__ void scan_setup(Trap& T, float y0, float y1, const float* l0,
+                                           const float* l1, const float* r0, const float* r1,
+                                           int na) {
+    // l*/r* layout: x, y, z, a0, a1, a2
+    const float recip_dy = 1.0f / (y1 - y0);
+    float dl[6], dr[6];
+    for (int c = 0; c < 6; ++c) {
+        dl[c] = (l1[c] - l0[c]) * recip_dy;
+        dr[c] = (r1[c] - r0[c]) * recip_dy;
+    }
+    float l0s[6], r0s[6];
+    for (int c = 0; c < 6; ++c) {
+        l0s[c] = l0[c] + dl[c];
+        r0s[c] = r0[c] + dr[c];
+    }
+    const float dx = r0s[0] - l0s[0];
+    const float rdx = 1.0f / dx;
+    T.dvz = (r0s[2] - l0s[2]) * rdx;
+    for (int c = 0; c < 3; ++c) T.dva[c] = (c < na) ? (r0s[3 + c] - l0s[3 + c]) * rdx : 0.0f;
+    const float y0r = round_up_to_half(y0);
+    const float y1r = round_up_to_half(y1);
+    const float tweak = y0r - y0;
+    // l0.lerp(&l0.step(&dl_dy), y_tweak) == l0 + ((l0 + dl) - l0) * tweak
+    T.lx = l0[0] + (l0s[0] - l0[0]) * tweak;
+    T.lz = l0[2] + (l0s[2] - l0[2]) * tweak;
+    for (int c = 0; c < 3; ++c) T.la[c] = (c < na) ? l0[3 + c] + (l0s[3 + c] - l0[3 + c]) * tweak : 0.0f;
+    T.dlx = dl[0];
+    T.dlz = dl[2];
+    for (int c = 0; c < 3; ++c) T.dla[c] = (c < na) ? dl[3 + c] : 0.0f;
+    T.rx = r0[0] + dr[0] * tweak;
+    T.drx = dr[0];
+    T.n = as_u32(y1r - y0r);
+    T.y0i = y0r - 0.5f;
+}
+
+// tri_fill (raster.rs:185-224) setup for one screen triangle (vertices as
+// x, y, z, a0, a1, a2; sorted in registers).
+__device__ __forceinline__ void swap6(float* a, float* b) {
+#pragma unroll
+    for (int k = 0; k < 6; ++k) {
+        const float t = a[k];
+        a[k] = b[k];
+        b[k] = t;
+    }
+}
+// The total_cmp order key of a screen y. A NaN y (0/0, the screen position
+// of a w = 0 clip vertex) is keyed as x86-64's default NaN, which has its
+// sign bit set and so sorts before -inf: that is the NaN the reference's
+// arithmetic produces there (the GPU's own NaN has no defined sign).
+__device__ __forceinline__ int32_t y_key(float y) { return total_key(y == y ? y : u2f(0xFFC00000u)); }
+
+__device__ __forceinline__ void tri_setup(Slot& S, float (&va)[6], float (&vb)[6], float (&vc)[6], int na) {
+    // stable sort by total_cmp of y (slice::sort_by is stable)
+    if (y_key(vb[1]) < y_key(va[1])) swap6(va, vb);
+    if (y_key(vc[1]) < y_key(vb[1])) swap6(vb, vc);
+    if (y_key(vb[1]) < y_key(va[1])) swap6(va, vb);
+    const float* top = va;
+    const float* mid0 = vb;
+    const float* bot = vc;
+    const float top_y = top[1], mid_y = mid0[1], bot_y = bot[1];
+    const float tt = (mid_y - top_y) / (bot_y - top_y);
+    float mid1[6];
+#pragma unroll
+    for (int k = 0; k < 6; ++k) mid1[k] = top[k] + (bot[k] - top[k]) * tt;
+    const bool l_is_mid0 = mid0[0] < mid1[0];
+    float left[6], right[6];
+#pragma unroll
+    for (int k = 0; k < 6; ++k) {
+        left[k] = l_is_mid0 ? mid0[k] : mid1[k];
+        right[k] = l_is_mid0 ? mid1[k] : mid0[k];
+    }
+    scan_setup(S.t[0], top_y, mid_y, top, left, top, right, na);
+    scan_setup(S.t[1], mid_y, bot_y, left, bot, right, bot, na);
+    int32_t lo = 0x7FFFFFFF, hi = -0x7FFFFFFF;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        if (S.t[h].n == 0) continue;
+        const int32_t y0 = (int32_t)S.t[h].y0i;
+        const int32_t y1 = y0 + (int32_t)S.t[h].n;
+        lo = y0 < lo ? y0 : lo;
+        hi = y1 > hi ? y1 : hi;
+    }
+    S.ylo = lo;
+    S.yhi = hi;
+}
+
+// ---------------------------------------------------------------------------
+// Small triangles: what the rasterizer needs to pass over one without
+// walking it
+// ---------------------------------------------------------------------------
+// A scene of many small triangles is mostly hidden: of 8 icospheres1080
+// frames' 285M fragments 43M pass the depth test. The rasterizer skips a
+// triangle of a tile whose every fragment must fail (see k_raster), but the
+// fragments still count in frags.i, and rows outside the target still are an
+// error. So k_setup walks the rows of each triangle of up to SMALL_ROWS rows
+// here, once: x only, the same serial sums as the rasterizer's, and an upper
+// bound of its fragments' z. Larger triangles are counted where they are
+// drawn.
+//
+// The walk costs a small launch 4 to 8 us (one 256 x 256 frame of 20 crates:
+// k_setup 8.8 -> 14.2 us; 13 frames of 80 icospheres at 66 triangles a tile: 20
+// -> 28, raster unchanged), so it is made where tiles have more triangles than
+// this on average.
+#ifndef RF_SMALL_TRIS
+#define RF_SMALL_TRIS 128
+#endif
+constexpr uint32_t SMALL_ROWS = 32;
+struct SmallTri {
+    uint32_t frags;  // frags.i of the whole triangle
+    float zmax;      // no fragment's z is above this
+    uint32_t err;
+};
+// The triangle's corners are finite and at or below row 0; cols: the columns
+// of its tiles, first | end << 16. False (nothing counted) if it is too tall
+// or the bound is not finite.
+__device__ __forceinline__ bool small_tri(const float* v0, const float* v1, const float* v2, uint32_t width,
+                                          uint32_t height, uint32_t cols, SmallTri& o) {
+    float va[6], vb[6], vc[6];
+#pragma unroll
+    for (int c = 0; c < 6; ++c) {
+        va[c] = v0[c];
+        vb[c] = v1[c];
+        vc[c] = v2[c];
+    }
+    Slot S;
+    tri_setup(S, va, vb, vc, 0);
+    o.frags = o.err = 0;
+    o.zmax = -__builtin_inff();
+    if (S.t[0].n > SMALL_ROWS || S.t[1].n > SMALL_ROWS || S.t[0].n + S.t[1].n > SMALL_ROWS) return false;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const Trap& T = S.t[h];
+        float lx = T.lx, rx = T.rx, w = 0.0f;
+        uint32_t y = (uint32_t)(int32_t)T.y0i;
+        for (uint32_t k = 0; k < T.n; ++k, ++y) {
+            w = fmaxf(w, rx - lx);
+            const uint32_t xs = cvt_u32(round_up_to_half(lx));
+            uint32_t xe = cvt_u32(round_up_to_half(rx));
+            xe = xe < xs ? xs : xe;
+            if (xe > width || y >= height) {
+                o.err |= ERRB_BOUNDS;
+            } else {
+                if (xe > xs && (xs < (cols & 0xFFFFu) || xe > (cols >> 16))) o.err |= ERRB_MARGIN;
+                o.frags += xe - xs;
+            }
+            lx = lx + T.dlx;
+            rx = rx + T.drx;
+        }
+        if (T.n == 0) continue;
+        // z starts at the left edge (lz + k dlz) and goes on by dvz a pixel,
+        // at most w + 1 pixels: a bound of the exact values, and of the
+        // rounding of rows + w + 8 operations on values up to m (each half an
+        // ulp, 2^-24 relative; taken four times)
+        const float n = (float)T.n, m = fabsf(T.lz) + n * fabsf(T.dlz) + (w + 2.0f) * fabsf(T.dvz);
+        const float z = fmaxf(T.lz, T.lz + n * T.dlz) + (w + 2.0f) * fmaxf(T.dvz, 0.0f) + (n + w + 8.0f) * 0x1p-22f * m;
+        o.zmax = z > o.zmax || z != z ? z : o.zmax;
+        if (z != z) return false;
+    }
+    return o.zmax < __builtin_inff();
 }
 
 // ---------------------------------------------------------------------------
@@ -506,6 +678,9 @@ __global__ __launch_bounds__(256) void k_setup(BatchDesc B) {
     uint32_t nf = 0, extra_base = 0;
     uint32_t rect[2] = {0, 0};
     bool has_rect = false;
+    uint32_t frags = 0;
+    float zmax = __builtin_inff();
+    const uint32_t twl = (uint32_t)__builtin_ctz(B.tile_w), thl = (uint32_t)__builtin_ctz(B.tile_h);
     uint32_t frame = 0xFFFFFFFFu;
     const uint32_t d0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)B.group_draw[group]);
     const uint32_t di = valid ? draw_of_tri(B.draws, B.n_draws, d0, g) : d0;
@@ -560,11 +735,24 @@ __global__ __launch_bounds__(256) void k_setup(BatchDesc B) {
                             for (int c = 0; c < 3; ++c) v[k][3 + c] = persp ? a[c] / p[k][3] : a[c];
                         }
                     }
-                    write_scr(&B.scr[g], v[0], v[1], v[2], di, D->kind);
                     ra.add(v[0]);
                     ra.add(v[1]);
                     ra.add(v[2]);
                     nf = 1;
+                    uint32_t kind = D->kind;
+                    if (B.small_tris && !ra.nan && !ra.inf && ra.ymin >= 0.0f && ra.ymax - ra.ymin <= (float)SMALL_ROWS &&
+                        pixel_rect(ra, F, rect)) {
+                        const uint32_t cols = ((rect[0] & 0xFFFFu) >> twl << twl) |
+                                              ((((rect[1] & 0xFFFFu) >> twl) + 1) << twl << 16);
+                        SmallTri st;
+                        if (small_tri(v[0], v[1], v[2], F.width, F.height, cols, st)) {
+                            kind |= KIND_COUNTED;
+                            frags = st.frags;
+                            zmax = st.zmax;
+                            if (st.err) atomicOr(B.err, st.err);
+                        }
+                    }
+                    write_scr(&B.scr[g], v[0], v[1], v[2], di, kind);
                 }
             } else {
                 // Clipped
@@ -637,7 +825,7 @@ __global__ __launch_bounds__(256) void k_setup(BatchDesc B) {
                     const float rr0 = floorf(ra.ymin + 0.5f), rr1 = floorf(ra.ymax + 0.5f);
                     if (rr1 > rr0 && (rr1 > (float)F.height || floorf(ra.xmin) > (float)F.width + 1.0f))
                         atomicOr(B.err, ERRB_BOUNDS);
-                    has_rect = tile_rect(ra, F, B.tile_w, (uint32_t)__builtin_ctz(B.tile_h), rect);
+                    has_rect = pixel_rect(ra, F, rect);
                 }
             }
         }
@@ -646,25 +834,34 @@ __global__ __launch_bounds__(256) void k_setup(BatchDesc B) {
         B.hdr[g] = nf | (extra_base << 3);
         B.rect[2 * g] = has_rect ? rect[0] : 0xFFFFFFFFu;
         B.rect[2 * g + 1] = rect[1];
+        if (B.small_tris) B.zmax[g] = zmax;
     }
     // prims.o (render.rs:195; verts.o is 3 per primitive, derived in
-    // k_scan_top): one atomic per wave when the wave's triangles all belong to
-    // one frame, else one per lane, into the group's partial counter
+    // k_scan_top) and the small triangles' frags.i: one atomic each per wave
+    // when the wave's triangles all belong to one frame, else one per lane,
+    // into the group's partial counters
     {
         const uint32_t fmin = wave_min_u32(nf > 0 ? frame : 0xFFFFFFFFu);
         const uint32_t fmax = ~wave_min_u32(nf > 0 ? ~frame : 0xFFFFFFFFu);
         const uint32_t part = (group % PRIM_PARTS) * PRIM_PART_STRIDE;
+        unsigned long long* c = B.prims_part + part;
         if (fmin == fmax) {
-            const unsigned long long tot = wave_sum_u64(nf);
-            if (lane == 0 && tot) atomicAdd(&B.prims_part[(uint64_t)fmin * PRIM_PARTS * PRIM_PART_STRIDE + part], tot);
+            c += (uint64_t)fmin * PRIM_PARTS * PRIM_PART_STRIDE;
+            uint32_t tot, ftot;
+            (void)wave_excl_scan(nf, &tot);
+            (void)wave_excl_scan(frags, &ftot);  // at most 64 triangles x 32 rows x 16,384 columns
+            if (lane == 0 && tot) atomicAdd(c, (unsigned long long)tot);
+            if (lane == 0 && ftot) atomicAdd(c + 1, (unsigned long long)ftot);
         } else if (nf > 0) {
-            atomicAdd(&B.prims_part[(uint64_t)frame * PRIM_PARTS * PRIM_PART_STRIDE + part], (unsigned long long)nf);
+            c += (uint64_t)frame * PRIM_PARTS * PRIM_PART_STRIDE;
+            atomicAdd(c, (unsigned long long)nf);
+            if (frags) atomicAdd(c + 1, (unsigned long long)frags);
         }
     }
     // per-tile run counts
     const FrameDesc* F = has_rect ? &B.frames[frame] : nullptr;
     const uint32_t base = has_rect ? F->tile_base : 0, ntx = has_rect ? F->ntx : 0;
-    for_each_tile(has_rect, rect[0], rect[1], base, ntx,
+    for_each_tile(has_rect, rect_tile(rect[0], twl, thl), rect_tile(rect[1], twl, thl), base, ntx,
                   [&](uint32_t tile, unsigned long long) { atomicAdd(&B.run_count[tile], 1u); });
 }
 #endif  // RF_RASTER_TU
@@ -748,13 +945,18 @@ __global__ __launch_bounds__(1024) void k_scan_top(BatchDesc B) {
             for (uint32_t k = 0; k < 16; ++k) carry[tid] += wave_tot[tid][k];
         __syncthreads();
     }
-    // prims.o of every frame from its partial counters; verts.o is 3 per
-    // primitive (render.rs:196)
+    // prims.o and the small triangles' frags.i of every frame from its
+    // partial counters; verts.o is 3 per primitive (render.rs:196)
     for (uint32_t f = tid; f < B.n_frames; f += blockDim.x) {
-        unsigned long long p = 0;
-        for (uint32_t k = 0; k < PRIM_PARTS; ++k) p += B.prims_part[((uint64_t)f * PRIM_PARTS + k) * PRIM_PART_STRIDE];
+        unsigned long long p = 0, fr = 0;
+        for (uint32_t k = 0; k < PRIM_PARTS; ++k) {
+            const unsigned long long* c = &B.prims_part[((uint64_t)f * PRIM_PARTS + k) * PRIM_PART_STRIDE];
+            p += c[0];
+            fr += c[1];
+        }
         B.stats[f].prims_o = p;
         B.stats[f].verts_o = 3ull * p;
+        B.stats[f].frags_i = fr;
     }
     if (tid == 0) {
         B.run_off[B.n_tiles] = carry[0];
@@ -908,107 +1110,6 @@ __global__ __launch_bounds__(64) void k_binsort(BatchDesc B) {
 // ---------------------------------------------------------------------------
 // k_raster
 // ---------------------------------------------------------------------------
-struct Trap {
-    float y0i;             // first row (floor(y0 + 0.5))
-    uint32_t n;            // row count
-    float lx, lz, la[3];   // left state at the first row
-    float dlx, dlz, dla[3];
-    float rx, drx;         // right x at the first row, step
-    float dvz, dva[3];     // d(varyings)/dx
-};
-struct Slot {
-    Trap t[2];
-    int32_t ylo, yhi;      // rows covered (absolute)
-};
-
-// scan (raster.rs:248-302) for one trapezoid; y components are not needed by
-// any output and are left out.
-__device__ __forceinline__ void scan_setup(Trap& T, float y0, float y1, const float* l0,
-                                           const float* l1, const float* r0, const float* r1,
-                                           int na) {
-    // l*/r* layout: x, y, z, a0, a1, a2
-    const float recip_dy = 1.0f / (y1 - y0);
-    float dl[6], dr[6];
-    for (int c = 0; c < 6; ++c) {
-        dl[c] = (l1[c] - l0[c]) * recip_dy;
-        dr[c] = (r1[c] - r0[c]) * recip_dy;
-    }
-    float l0s[6], r0s[6];
-    for (int c = 0; c < 6; ++c) {
-        l0s[c] = l0[c] + dl[c];
-        r0s[c] = r0[c] + dr[c];
-    }
-    const float dx = r0s[0] - l0s[0];
-    const float rdx = 1.0f / dx;
-    T.dvz = (r0s[2] - l0s[2]) * rdx;
-    for (int c = 0; c < 3; ++c) T.dva[c] = (c < na) ? (r0s[3 + c] - l0s[3 + c]) * rdx : 0.0f;
-    const float y0r = round_up_to_half(y0);
-    const float y1r = round_up_to_half(y1);
-    const float tweak = y0r - y0;
-    // l0.lerp(&l0.step(&dl_dy), y_tweak) == l0 + ((l0 + dl) - l0) * tweak
-    T.lx = l0[0] + (l0s[0] - l0[0]) * tweak;
-    T.lz = l0[2] + (l0s[2] - l0[2]) * tweak;
-    for (int c = 0; c < 3; ++c) T.la[c] = (c < na) ? l0[3 + c] + (l0s[3 + c] - l0[3 + c]) * tweak : 0.0f;
-    T.dlx = dl[0];
-    T.dlz = dl[2];
-    for (int c = 0; c < 3; ++c) T.dla[c] = (c < na) ? dl[3 + c] : 0.0f;
-    T.rx = r0[0] + dr[0] * tweak;
-    T.drx = dr[0];
-    T.n = as_u32(y1r - y0r);
-    T.y0i = y0r - 0.5f;
-}
-
-// tri_fill (raster.rs:185-224) setup for one screen triangle (vertices as
-// x, y, z, a0, a1, a2; sorted in registers).
-__device__ __forceinline__ void swap6(float* a, float* b) {
-#pragma unroll
-    for (int k = 0; k < 6; ++k) {
-        const float t = a[k];
-        a[k] = b[k];
-        b[k] = t;
-    }
-}
-// The total_cmp order key of a screen y. A NaN y (0/0, the screen position
-// of a w = 0 clip vertex) is keyed as x86-64's default NaN, which has its
-// sign bit set and so sorts before -inf: that is the NaN the reference's
-// arithmetic produces there (the GPU's own NaN has no defined sign).
-__device__ __forceinline__ int32_t y_key(float y) { return total_key(y == y ? y : u2f(0xFFC00000u)); }
-
-__device__ __forceinline__ void tri_setup(Slot& S, float (&va)[6], float (&vb)[6], float (&vc)[6], int na) {
-    // stable sort by total_cmp of y (slice::sort_by is stable)
-    if (y_key(vb[1]) < y_key(va[1])) swap6(va, vb);
-    if (y_key(vc[1]) < y_key(vb[1])) swap6(vb, vc);
-    if (y_key(vb[1]) < y_key(va[1])) swap6(va, vb);
-    const float* top = va;
-    const float* mid0 = vb;
-    const float* bot = vc;
-    const float top_y = top[1], mid_y = mid0[1], bot_y = bot[1];
-    const float tt = (mid_y - top_y) / (bot_y - top_y);
-    float mid1[6];
-#pragma unroll
-    for (int k = 0; k < 6; ++k) mid1[k] = top[k] + (bot[k] - top[k]) * tt;
-    const bool l_is_mid0 = mid0[0] < mid1[0];
-    float left[6], right[6];
-#pragma unroll
-    for (int k = 0; k < 6; ++k) {
-        left[k] = l_is_mid0 ? mid0[k] : mid1[k];
-        right[k] = l_is_mid0 ? mid1[k] : mid0[k];
-    }
-    scan_setup(S.t[0], top_y, mid_y, top, left, top, right, na);
-    scan_setup(S.t[1], mid_y, bot_y, left, bot, right, bot, na);
-    int32_t lo = 0x7FFFFFFF, hi = -0x7FFFFFFF;
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-        if (S.t[h].n == 0) continue;
-        const int32_t y0 = (int32_t)S.t[h].y0i;
-        const int32_t y1 = y0 + (int32_t)S.t[h].n;
-        lo = y0 < lo ? y0 : lo;
-        hi = y1 > hi ? y1 : hi;
-    }
-    S.ylo = lo;
-    S.yhi = hi;
-}
-
 // 16-byte framebuffer stores. The rasterizer writes every target pixel once
 // and never reads it back in the launch, so with RF_NT_STORE the stores are
 // streaming (non-temporal): a gigabyte of colour and depth per launch then
@@ -1046,9 +1147,6 @@ __device__ __forceinline__ void store_pixel(const FrameDesc& F, uint32_t x, uint
 }
 
 
-#ifndef RF_RUN_MULTI
-#define RF_RUN_MULTI 1  // runs flag groups with several fans per triangle
-#endif
 #ifndef RF_CLEAR_ROWS
 #define RF_CLEAR_ROWS 1  // clear runs of empty tiles row segment by row segment
 #endif
@@ -1154,6 +1252,9 @@ __global__ __launch_bounds__(256) void k_bin(BatchDesc B) {
         r0 = B.rect[2 * g];
         r1 = B.rect[2 * g + 1];
         valid = r0 != 0xFFFFFFFFu;
+        const uint32_t twl = (uint32_t)__builtin_ctz(B.tile_w), thl = (uint32_t)__builtin_ctz(B.tile_h);
+        r0 = rect_tile(r0, twl, thl);
+        r1 = rect_tile(r1, twl, thl);
         if (valid) {
             const uint32_t di = draw_of_tri(B.draws, B.n_draws, B.group_draw[group], g);
             const FrameDesc& F = B.frames[B.draws[di].frame];
@@ -1220,14 +1321,36 @@ struct EdgeRec {
     float lx, rx, lz, l0, l1, l2;
 };
 
-// Edge records per batch of a tile th rows tall (a batch's first triangle
-// has at most th rows in a tile, unless rows above the target fold onto row 0).
-__host__ __device__ constexpr int rec_cap(int th) { return th > 32 ? 384 : 128; }
-constexpr int FQ_CAP = 512;          // fan queue (ring); one run adds at most 64 * 7 fans
+// The tile's queues of fans (rings): those of its runs in order, and of them
+// those to draw (n_slot + 64 at most). A run adds at most 64 fans, or, where triangles have several,
+// 16 triangles at a time, at most 112.
+constexpr int FQ_CAP = 192;
+
 #ifndef RF_CELL_W
 #define RF_CELL_W 8
 #endif
 constexpr int CELL_W = RF_CELL_W;    // pixel columns per ordering cell
+// Triangles and edge records per batch. LDS decides how many one-wave
+// workgroups a CU holds (registers allow eight), so a tile's batch takes what
+// its pixels leave of the smallest share that holds 128 records: 1/8 of the
+// CU's 160 KB, else 1/6, 1/5, 1/4 or 1/3 (in the allocation's 1,280-byte
+// steps); tiles of 64 rows, whose triangles are taller, hold 384. Longer batches start fewer half-empty rounds: at 32 x 32 tiles, 8
+// icospheres1080 frames, 128 records and 32 triangles 2.63 ms, 192 and 64
+// 2.55, 256 and 32 2.35. (A batch's first triangle has at most th rows in a
+// tile, unless rows above the target fold onto row 0.)
+constexpr int REC_BYTES = 25;  // an EdgeRec and its owner
+__host__ __device__ constexpr int lds_fixed(int tw, int th, int slots) {
+    return 9 * tw * (th + 1) + 4 * th * (tw / CELL_W) + 4 * (FQ_CAP + 64) + 4 * (slots + WAVE) + 64 * slots;
+}
+__host__ __device__ constexpr int n_slot(int tw, int th) {
+    return tw * th <= 512 || th > 32 ? 64 : 32;
+}
+__host__ __device__ constexpr int rec_cap(int tw, int th) {
+    const int f = lds_fixed(tw, th, n_slot(tw, th)), min = f + (th > 32 ? 384 : 128) * REC_BYTES;
+    const int share = min <= 20480 ? 20480 : min <= 26880 ? 26880 : min <= 32000 ? 32000 : min <= 40960 ? 40960 : 53760;
+    const int r = (share - f) / REC_BYTES / 32 * 32;
+    return r < 480 ? r : 480;
+}
 #ifndef RF_TILE_GRAB
 #define RF_TILE_GRAB 1
 #endif
@@ -1247,6 +1370,13 @@ constexpr int JSER = RF_JSER;  // pixel steps taken serially; more use the exact
 #ifndef RF_REFILL_MIN
 #define RF_REFILL_MIN 16
 #endif
+#ifndef RF_HIDE_RUNS
+#define RF_HIDE_RUNS 64
+#endif
+// Tiles of more runs than this pass over hidden triangles. Measured at 16, 64
+// and 128 on 14 icosphere and mixed batches: 64 is never behind (10 frames of
+// 1,291 icospheres: raster 621, 674, 720 us, but 13 frames of 80: 220, 209, 210).
+constexpr int HIDE_RUNS = RF_HIDE_RUNS;
 constexpr int REFILL_MIN = RF_REFILL_MIN;  // free lanes that trigger a refill while others still work
 
 // Tile rasterizer. One wave owns one tile (TILE_H rows x TW columns) at a
@@ -1278,9 +1408,14 @@ constexpr int REFILL_MIN = RF_REFILL_MIN;  // free lanes that trigger a refill w
 // passing fragment, so the fetches run once per written pixel at the end of
 // the tile, all pixels in parallel, and colour and depth go straight to the
 // target.
-constexpr uint16_t TAG_NONE = 0xFFFFu;   // no fragment wrote colour
-constexpr uint16_t TAG_COLOR = 0xFFFEu;  // payload is the colour; else tag = draw - base, payload = texel
+constexpr uint8_t TAG_NONE = 0xFFu;   // no fragment wrote colour
+constexpr uint8_t TAG_COLOR = 0xFEu;  // payload is the colour; else tag = index in the tile's draws, payload = texel
+// Draws a tile's colour sources can name at a time. One byte a pixel for the
+// tag: at two, a 64 x 32 tile's workgroup holds 29 KB and five fit a CU; at
+// one, with 32 slots, 26.6 KB and six (32 crates1080 frames: 0.680 -> 0.621 ms).
+constexpr int N_TAGS = 62;
 constexpr uint32_t LINE_TAG = 0x8000u;   // SlotP::kind_tag bit of a line primitive
+constexpr uint32_t COUNTED_TAG = 0x4000u;  // and of a triangle whose frags.i k_setup counted
 
 __device__ __forceinline__ uint32_t texel_pixel(const BatchDesc& B, uint32_t fmt, uint32_t draw, uint32_t texel) {
     const uint32_t t = ((const uint32_t*)B.draws[draw].tex)[texel];
@@ -1329,7 +1464,9 @@ __device__ __forceinline__ bool depth_pass_u(int32_t dt, float nz, float cur) {
 template <int TW, int CH, int TH>
 __global__ __launch_bounds__(64, 2) void k_raster(BatchDesc B) {
     constexpr int TILE_H = TH;  // tile rows
-    constexpr int REC_CAP = rec_cap(TH);
+    constexpr int REC_CAP = rec_cap(TW, TH);
+    constexpr int NSLOT = n_slot(TW, TH);
+    constexpr int DQ_CAP = NSLOT + WAVE;
     constexpr int LD = TILE_H + 1;  // padded column stride in LDS (bank spread)
     constexpr int NPX = TW * LD;
     constexpr int CW = CELL_W < TW ? CELL_W : TW;  // ordering cell width in this tile
@@ -1341,11 +1478,13 @@ __global__ __launch_bounds__(64, 2) void k_raster(BatchDesc B) {
     float* const s_dep = s_px;
     uint32_t* const s_pay = reinterpret_cast<uint32_t*>(s_px + NPX);  // the pixel's colour source: payload
     static_assert((CH - 1) * LD + TILE_H <= NPX, "depth over-reads stay in the array");
-    __shared__ __align__(16) uint16_t s_tag[NPX];   //   and tag
-    static_assert((NPX * 4) % 16 == 0 && (NPX * 2) % 16 == 0, "16-byte LDS fills");
-    __shared__ SlotP s_slot[WAVE];
+    __shared__ __align__(16) uint8_t s_tag[NPX];   //   and tag
+    static_assert((NPX * 4) % 16 == 0 && NPX % 16 == 0, "16-byte LDS fills");
+    __shared__ SlotP s_slot[NSLOT];
     __shared__ EdgeRec s_rec[REC_CAP];
     __shared__ uint32_t s_fq[FQ_CAP];  // g << 3 | fan
+    __shared__ uint32_t s_dq[DQ_CAP];
+    __shared__ uint32_t s_draws[N_TAGS];
     __shared__ int8_t s_own[REC_CAP];  // slot whose records start here, or -1
     __shared__ __align__(16) uint32_t s_cell[TILE_H * NCG];
 
@@ -1483,7 +1622,7 @@ __global__ __launch_bounds__(64, 2) void k_raster(BatchDesc B) {
             if (has_depth)
                 for (uint32_t i = lane; i < (uint32_t)NPX / 4; i += WAVE)
                     reinterpret_cast<float4*>(s_dep)[i] = make_float4(cd, cd, cd, cd);
-            for (uint32_t i = lane; i < (uint32_t)NPX / 8; i += WAVE)
+            for (uint32_t i = lane; i < (uint32_t)NPX / 16; i += WAVE)
                 reinterpret_cast<uint4*>(s_tag)[i] = make_uint4(0xFFFFFFFFu, 0xFFFFFFFFu, 0xFFFFFFFFu, 0xFFFFFFFFu);
         } else {
             constexpr uint32_t LPR = WAVE / TILE_H;  // lanes per row
@@ -1501,9 +1640,13 @@ __global__ __launch_bounds__(64, 2) void k_raster(BatchDesc B) {
         unsigned long long fi_acc = 0, fo_acc = 0;
         uint32_t errs = 0;
         uint32_t fq_head = 0, fq_tail = 0;  // ring indices (wave-uniform)
+        uint32_t dq_head = 0, dq_tail = 0;
+        // Triangles that cannot pass the depth test anywhere in the tile are
+        // passed over (see below) once a batch has been drawn.
+        const bool hide = B.small_tris && dtest == (int32_t)DT_LESS && nruns > (uint32_t)HIDE_RUNS;
+        bool drawn = false;
         uint32_t head_skip = 0;             // rows of the head triangle already taken (wave-uniform)
-        uint32_t dbase = 0;                 // draw of the tile's first triangle
-        bool dbase_set = false;
+        uint32_t n_tags = 0, last_draw = 0;  // draws in s_draws, and the last of them
 
         // the tile's runs in group order: lists of up to 64 are loaded one per
         // lane and sorted here; longer ones were sorted by k_binsort
@@ -1522,7 +1665,7 @@ __global__ __launch_bounds__(64, 2) void k_raster(BatchDesc B) {
         // batch has handed out its last record, the next one is set up while
         // the items in flight finish (an item keeps in registers all it needs
         // of its slot and record). Order keys run on across the batches.
-        uint32_t ri = 0;          // next run to append
+        uint32_t ri = 0, rquarter = 0;  // next run to queue, and its next 16 triangles if they have several fans
         uint32_t next = 0;        // next record of the current batch to hand out
         uint32_t nrec = 0;        // records of the current batch
         uint32_t key_base = 0;    // order key of the current batch's first record
@@ -1533,34 +1676,92 @@ __global__ __launch_bounds__(64, 2) void k_raster(BatchDesc B) {
         int32_t xs = 0, jc = 0, j1 = 0;
         for (;;) {
             if (next >= nrec) {
-                // append runs until a full batch of fans is queued (or none are left)
-                while (ri < nruns && fq_tail - fq_head < (uint32_t)WAVE) {
-                    Run run;
-                    if (nruns <= (uint32_t)WAVE) {
-                        run.group = __shfl(lrun_g, ri, WAVE);
-                        run.mask = __shfl(lrun_m, ri, WAVE);
-                        run.multi = __shfl(lrun_x, ri, WAVE);
-                    } else {
-                        run = B.runs[off + ri];
+                // The least depth of each of 4 x 4 blocks of the tile, four lanes
+                // a block. Depths under the Less test only grow, so items in
+                // flight can only raise it: a triangle whose fragments' z is
+                // nowhere above its blocks' least depth fails at every pixel.
+                // 8 icospheres1080 frames: 6.66 -> 2.35 ms (42.9M of 285M
+                // fragments pass).
+                float bmin = 0.0f;
+                const bool test = hide && drawn && ri < nruns;
+                if (test) {
+                    constexpr uint32_t BW = TW / 4, BH = TILE_H / 4;
+                    const uint32_t bx = (lane >> 2 & 3u) * BW, by = (lane >> 4) * BH;
+                    bmin = __builtin_inff();
+#pragma unroll 4
+                    for (uint32_t i = 0; i < BW * BH / 4; ++i) {
+                        const uint32_t c = bx + (i * 4 + (lane & 3u)) / BH, r = by + (i * 4 + (lane & 3u)) % BH;
+                        const float d = s_dep[c * LD + r];
+                        bmin = c < ncols && r < nrows ? fminf(bmin, d) : bmin;
                     }
-                    const uint64_t g = (uint64_t)run.group * WAVE + lane;
-                    const bool has = (run.mask >> lane) & 1ull;
-                    // a triangle in the mask has at least one fan; only groups
-                    // with clipped triangles need their headers
-                    const uint32_t nf = has ? (RF_RUN_MULTI && !run.multi ? 1u : (B.hdr[g] & 7u)) : 0u;
-                    uint32_t tot;
-                    const uint32_t pre = wave_excl_scan(nf, &tot);
-                    for (uint32_t j = 0; j < nf; ++j) s_fq[(fq_tail + pre + j) % FQ_CAP] = ((uint32_t)g << 3) | j;
-                    fq_tail += tot;
-                    ++ri;
+                    bmin = fminf(bmin, u2f(dpp_u32<DPP_QUAD_1032>(f2u(bmin), f2u(bmin))));
+                    bmin = fminf(bmin, u2f(dpp_u32<DPP_QUAD_2301>(f2u(bmin), f2u(bmin))));
+                }
+                // queue fans until a full batch is to be drawn (or none are left)
+                while (!hide || dq_tail - dq_head < (uint32_t)NSLOT) {
+                    while (ri < nruns && fq_tail - fq_head < (uint32_t)WAVE) {
+                        Run run;
+                        if (nruns <= (uint32_t)WAVE) {
+                            run.group = __shfl(lrun_g, ri, WAVE);
+                            run.mask = __shfl(lrun_m, ri, WAVE);
+                            run.multi = __shfl(lrun_x, ri, WAVE);
+                        } else {
+                            run = B.runs[off + ri];
+                        }
+                        const uint64_t g = (uint64_t)run.group * WAVE + lane;
+                        bool has = (run.mask >> lane) & 1ull;
+                        if (run.multi) has = has && lane / 16 == rquarter;
+                        // a triangle in the mask has at least one fan; only groups
+                        // with clipped triangles need their headers
+                        const uint32_t nf = has ? (!run.multi ? 1u : (B.hdr[g] & 7u)) : 0u;
+                        uint32_t tot;
+                        const uint32_t pre = wave_excl_scan(nf, &tot);
+                        for (uint32_t j = 0; j < nf; ++j) s_fq[(fq_tail + pre + j) % FQ_CAP] = ((uint32_t)g << 3) | j;
+                        fq_tail += tot;
+                        if (!run.multi || ++rquarter == 4) {
+                            ++ri;
+                            rquarter = 0;
+                        }
+                        __syncthreads();
+                    }
+                    const uint32_t nq = min(fq_tail - fq_head, (uint32_t)WAVE);
+                    if (!hide || nq == 0) break;
+                    bool take = lane < nq;
+                    const uint32_t e = take ? s_fq[(fq_head + lane) % FQ_CAP] : 0u;
+                    if (test) {
+                        float z = -__builtin_inff(), m = __builtin_inff();
+                        uint32_t blocks = 0;
+                        if (take) {
+                            constexpr uint32_t BWL = __builtin_ctz(TW / 4), BHL = __builtin_ctz(TILE_H / 4);
+                            const uint64_t gg = e >> 3;
+                            z = B.zmax[gg];
+                            const uint32_t r0 = B.rect[2 * gg], r1 = B.rect[2 * gg + 1];
+                            const uint32_t cx0 = max(r0 & 0xFFFFu, x0) - x0, cx1 = min(r1 & 0xFFFFu, x0 + TW - 1) - x0;
+                            const uint32_t cy0 = max(r0 >> 16, y0) - y0, cy1 = min(r1 >> 16, y0 + TILE_H - 1) - y0;
+                            const uint32_t xm = (2u << (cx1 >> BWL)) - (1u << (cx0 >> BWL));
+                            const uint32_t ym = (16u << 4 * (cy1 >> BHL)) - (1u << 4 * (cy0 >> BHL));
+                            blocks = xm * 0x1111u & ym;
+                        }
+#pragma unroll 2
+                        for (int k = 0; k < 16; ++k) {
+                            const float bm = u2f((uint32_t)__builtin_amdgcn_readlane((int)f2u(bmin), 4 * k));
+                            m = blocks >> k & 1u ? fminf(m, bm) : m;
+                        }
+                        take = take && z > m;
+                    }
+                    const unsigned long long tm = __ballot(take);
+                    if (take) s_dq[(dq_tail + __popcll(tm & ((1ull << lane) - 1))) % DQ_CAP] = e;
+                    dq_tail += __popcll(tm);
+                    fq_head += nq;
                     __syncthreads();
                 }
-                const uint32_t avail = fq_tail - fq_head;
+                drawn = true;
+                const uint32_t avail = hide ? dq_tail - dq_head : fq_tail - fq_head;
                 if (avail == 0) {
                     if (__ballot(have) == 0ull) break;  // the tile is done
                     goto rounds;
                 }
-                const uint32_t nb = avail < (uint32_t)WAVE ? avail : (uint32_t)WAVE;
+                const uint32_t nb = avail < (uint32_t)NSLOT ? avail : (uint32_t)NSLOT;
                 // ---- setup: lane = triangle
                 const bool act = lane < nb;
                 Slot S;
@@ -1570,11 +1771,11 @@ __global__ __launch_bounds__(64, 2) void k_raster(BatchDesc B) {
                 int na = 0;
                 // a line (KIND_LINE): one record per pixel of its walk that lies in
                 // the tile's columns (wide) or rows (tall), from step lka on
-                bool is_line = false, lwide = false;
+                bool is_line = false, lwide = false, counted = false;
                 uint32_t lS = 0, lka = 0;
                 float lbase = 0.0f, lstep = 0.0f, lz = 0.0f, la0 = 0.0f, la1 = 0.0f, la2 = 0.0f;
                 if (act) {
-                    const uint32_t e = s_fq[(fq_head + lane) % FQ_CAP];
+                    const uint32_t e = hide ? s_dq[(dq_head + lane) % DQ_CAP] : s_fq[(fq_head + lane) % FQ_CAP];
                     const uint64_t gg = e >> 3;
                     const uint32_t j = e & 7u;
                     const ScrTri* st = (j == 0) ? &B.scr[gg] : &B.extra[(B.hdr[gg] >> 3) + j - 1];
@@ -1588,6 +1789,7 @@ __global__ __launch_bounds__(64, 2) void k_raster(BatchDesc B) {
                     di = st->draw;
                     kind = st->kind & 0xFFu;
                     is_line = (st->kind & KIND_LINE) != 0u;
+                    counted = (st->kind & KIND_COUNTED) != 0u;
                     na = kind_attrs(kind);
                     if (is_line) {
                         lS = f2u(vb[0]);
@@ -1612,8 +1814,8 @@ __global__ __launch_bounds__(64, 2) void k_raster(BatchDesc B) {
                     } else {
                         tri_setup(S, va, vb, vc, na);
                         const uint32_t rr0 = B.rect[2 * gg], rr1 = B.rect[2 * gg + 1];
-                        rx0b = (rr0 & 0xFFFF) * TW;
-                        rx1b = ((rr1 & 0xFFFF) + 1) * TW;
+                        rx0b = (rr0 & 0xFFFFu) / TW * TW;
+                        rx1b = ((rr1 & 0xFFFFu) / TW + 1) * TW;
                         // rows of the triangle in this tile; in the first tile
                         // row, the rows above the target too: `self.y as
                         // usize` folds each onto row 0 as a span of its own
@@ -1634,38 +1836,39 @@ __global__ __launch_bounds__(64, 2) void k_raster(BatchDesc B) {
                 const bool head_split = __ballot(split) != 0ull;
                 uint32_t rec_tot;
                 const uint32_t rec_base = wave_excl_scan(rows_in, &rec_tot);
-                // take the leading triangles whose records fit (lane 0 always
-                // fits: it has at most REC_CAP rows)
-                const bool fits = rec_base + rows_in <= (uint32_t)REC_CAP;
-                const unsigned long long nf_mask = ~__ballot(act && fits && !head_split);
-                const uint32_t nuse = head_split ? 1u
-                                    : nf_mask == 0ull ? (uint32_t)WAVE : (uint32_t)(__ffsll((long long)nf_mask) - 1);
-                const bool use = lane < nuse;
-                const uint32_t nrec_new = __shfl(rec_base + rows_in, nuse - 1, WAVE);
-                // draw tags are relative to the tile's first draw (draws only grow
-                // along the triangle order); resolve pending texels before the
-                // range would overflow
-                const uint32_t dfirst = __shfl(di, 0, WAVE), dlast = __shfl(di, nuse - 1, WAVE);
-                const bool rebase = dbase_set && dlast - dbase >= (uint32_t)TAG_COLOR;
-                if (rebase && __ballot(have) != 0ull) {
-                    // items in flight still tag with the old base: let them finish first
-                    goto rounds;
-                }
-                if (!dbase_set) {
-                    dbase = dfirst;
-                    dbase_set = true;
-                } else if (rebase) {
+                // the draws' tags (draws only grow along the triangle order)
+                const uint32_t prev = __shfl_up(di, 1, WAVE);
+                const bool fresh = act && (lane == 0 ? n_tags == 0 || di != last_draw : di != prev);
+                const unsigned long long fm = __ballot(fresh);
+                uint32_t tag = n_tags + (uint32_t)__popcll(fm & ((2ull << lane) - 1)) - 1;
+                const uint32_t tag0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)tag);
+                if (tag0 >= (uint32_t)N_TAGS) {
+                    // no tag left for the first triangle: pending texels are
+                    // resolved to colours, and the tags start over
+                    if (__ballot(have) != 0ull) goto rounds;  // after the items in flight, which use the old ones
                     for (uint32_t i = lane; i < npx; i += WAVE) {
                         const uint32_t r = i / ncols, c = i - r * ncols;
                         const uint32_t li = c * LD + r;
                         const uint32_t tg = s_tag[li];
                         if (tg < TAG_COLOR) {
-                            s_pay[li] = texel_pixel(B, F.fmt, dbase + tg, s_pay[li]);
+                            s_pay[li] = texel_pixel(B, F.fmt, s_draws[tg], s_pay[li]);
                             s_tag[li] = TAG_COLOR;
                         }
                     }
-                    dbase = dfirst;
+                    __syncthreads();
+                    tag -= tag0;
                 }
+                // take the leading triangles whose records and tags fit (lane
+                // 0 always does: it has at most REC_CAP rows)
+                const bool fits = rec_base + rows_in <= (uint32_t)REC_CAP && tag < (uint32_t)N_TAGS;
+                const unsigned long long nf_mask = ~__ballot(act && fits && !head_split);
+                const uint32_t nuse = head_split ? 1u
+                                    : nf_mask == 0ull ? (uint32_t)WAVE : (uint32_t)(__ffsll((long long)nf_mask) - 1);
+                const bool use = lane < nuse;
+                const uint32_t nrec_new = __shfl(rec_base + rows_in, nuse - 1, WAVE);
+                if (use && (fresh || lane == 0)) s_draws[tag] = di;
+                n_tags = __shfl(tag, nuse - 1, WAVE) + 1;
+                last_draw = __shfl(di, nuse - 1, WAVE);
                 for (uint32_t i = lane; i < nrec_new; i += WAVE) s_own[i] = -1;
                 __syncthreads();
                 if (use) {
@@ -1675,7 +1878,7 @@ __global__ __launch_bounds__(64, 2) void k_raster(BatchDesc B) {
                         P.dv[h][0] = S.t[h].dvz;
                         for (int c = 0; c < 3; ++c) P.dv[h][1 + c] = S.t[h].dva[c];
                     }
-                    P.kind_tag = kind | (is_line ? LINE_TAG : 0u) | ((di - dbase) << 16);
+                    P.kind_tag = kind | (is_line ? LINE_TAG : 0u) | (counted ? COUNTED_TAG : 0u) | (tag << 16);
                     const DrawDesc& D = B.draws[di];
                     if (kind == KIND_FLAT) {
                         const uint32_t fc = D.flat_rgba;
@@ -1740,7 +1943,8 @@ __global__ __launch_bounds__(64, 2) void k_raster(BatchDesc B) {
                 if (head_split) {
                     head_skip += REC_CAP;  // the same triangle heads the next batch
                 } else {
-                    fq_head += nuse;
+                    if (hide) dq_head += nuse;
+                    else fq_head += nuse;
                     head_skip = 0;
                 }
             }
@@ -1813,7 +2017,7 @@ __global__ __launch_bounds__(64, 2) void k_raster(BatchDesc B) {
                         // frags.i: the part of [xs, xe) inside this tile
                         const uint32_t pa = xs32 > x0 ? xs32 : x0;
                         const uint32_t pb = xe < x0 + TW ? xe : x0 + TW;
-                        if (pb > pa) fi_acc += pb - pa;
+                        if (pb > pa && !(P.kind_tag & COUNTED_TAG)) fi_acc += pb - pa;
                         const uint32_t nfrag = cnt_f < xe - xs32 ? cnt_f : xe - xs32;
                         xs = (int32_t)xs32;
                         jj0 = (int32_t)x0 - xs > 0 ? (int32_t)x0 - xs : 0;
@@ -1965,7 +2169,7 @@ __global__ __launch_bounds__(64, 2) void k_raster(BatchDesc B) {
 #pragma unroll
                     for (int p = 0; p < CH; ++p) {
                         if (ps[p]) {
-                            s_tag[li + p * LD] = (uint16_t)tg;
+                            s_tag[li + p * LD] = (uint8_t)tg;
                             s_pay[li + p * LD] = pay[p];
                         }
                     }
@@ -2002,7 +2206,7 @@ __global__ __launch_bounds__(64, 2) void k_raster(BatchDesc B) {
                 }
 #pragma unroll
                 for (int k = 0; k < 4; ++k)
-                    tp[k] = tg[k] < TAG_COLOR ? (const uint32_t*)B.draws[dbase + tg[k]].tex : nullptr;
+                    tp[k] = tg[k] < TAG_COLOR ? (const uint32_t*)B.draws[s_draws[tg[k]]].tex : nullptr;
                 uint4 old = make_uint4(0, 0, 0, 0);
                 const bool keep = !F.clear_color && (tg[0] == TAG_NONE || tg[1] == TAG_NONE || tg[2] == TAG_NONE ||
                                                      tg[3] == TAG_NONE);
@@ -2032,7 +2236,7 @@ __global__ __launch_bounds__(64, 2) void k_raster(BatchDesc B) {
                 if (tg == TAG_COLOR) {
                     store_pixel(F, x0 + c, y0 + r, s_pay[li]);
                 } else if (tg != TAG_NONE) {
-                    store_pixel(F, x0 + c, y0 + r, texel_pixel(B, F.fmt, dbase + tg, s_pay[li]));
+                    store_pixel(F, x0 + c, y0 + r, texel_pixel(B, F.fmt, s_draws[tg], s_pay[li]));
                 } else if (F.clear_color) {
                     store_pixel(F, x0 + c, y0 + r, F.clear_pixel);
                 }
@@ -2262,7 +2466,10 @@ __global__ void k_reset(BatchDesc B) {
     if (i < B.n_tiles) B.run_count[i] = 0;
     // the draw of each group's first triangle
     if (i < B.n_groups) B.group_draw[i] = find_draw_tri(B.draws, B.n_draws, (uint64_t)i * WAVE);
-    if (i < B.n_frames * PRIM_PARTS) B.prims_part[(uint64_t)i * PRIM_PART_STRIDE] = 0;
+    if (i < B.n_frames * PRIM_PARTS) {
+        B.prims_part[(uint64_t)i * PRIM_PART_STRIDE] = 0;
+        B.prims_part[(uint64_t)i * PRIM_PART_STRIDE + 1] = 0;
+    }
     if (i < B.n_frames) {
         B.stats[i].prims_o = 0;
         B.stats[i].verts_o = 0;
@@ -2289,6 +2496,7 @@ static hipError_t launch_impl(const BatchDesc& B0, hipStream_t s, uint32_t raste
     // the rasterizer's waves clear the tiles without runs at their end (faster,
     // measured, than k_bin's extra blocks doing it beside the binning)
     B.clear_in_raster = RF_CLEAR_IN_RASTER;
+    B.small_tris = B.n_tris > (uint64_t)RF_SMALL_TRIS * B.n_tiles;
     uint32_t reset_n = B.n_tiles > B.n_frames * PRIM_PARTS ? B.n_tiles : B.n_frames * PRIM_PARTS;
     reset_n = reset_n > B.n_groups ? reset_n : B.n_groups;
     auto mark = [&](int i) {

@@ -38,6 +38,9 @@ enum PrimType : uint32_t {
 // end (its z and varyings hold for every pixel) and v[1] its pixel walk
 // (see k_setup).
 constexpr uint32_t KIND_LINE = 0x100;
+// ScrTri::kind bit of a triangle whose frags.i k_setup has counted (see
+// small_tri): the rasterizer leaves it alone.
+constexpr uint32_t KIND_COUNTED = 0x200;
 
 __host__ __device__ inline int kind_attrs(uint32_t k) {
     return k == KIND_FLAT ? 0 : (k == KIND_GOURAUD ? 3 : 2);
@@ -114,11 +117,12 @@ struct FrameDesc {
 };
 
 // Per-frame statistics (stats.rs:16-40), accumulated by the kernels.
-// prims.o is counted in this many partial counters per frame, each on its
-// own 128-byte line: atomics on one address serialise, and a frame of 3.2M
-// small triangles has 50,000 setup waves adding to it.
+// prims.o, and frags.i of the small triangles, are counted in this many
+// partial counters per frame, each pair on its own 128-byte line: atomics on
+// one address serialise, and a frame of 3.2M small triangles has 50,000 setup
+// waves adding to it.
 constexpr uint32_t PRIM_PARTS = 16;
-constexpr uint32_t PRIM_PART_STRIDE = 16;  // u64 words between partial counters
+constexpr uint32_t PRIM_PART_STRIDE = 16;  // u64 words between partial counters (prims.o, frags.i)
 
 struct FrameStats {
     unsigned long long prims_o, verts_o, frags_i, frags_o;
@@ -160,7 +164,8 @@ struct BatchDesc {
     ScrTri* extra;       // further fans of clipped triangles
     uint32_t* extra_count;
     uint32_t extra_cap;
-    uint32_t* rect;      // per triangle: tile rect (tx0 | ty0 << 16, tx1 | ty1 << 16), 2 words
+    uint32_t* rect;      // per triangle: pixel rect (c0 | r0 << 16, c1 | r1 << 16; all ones: none), 2 words
+    float* zmax;         // per triangle: no fragment's z is above it (+inf: not known)
     uint32_t* run_count; // per tile
     uint32_t* run_off;   // per tile + 1 (exclusive scan)
     uint32_t* run_cursor;
@@ -168,13 +173,14 @@ struct BatchDesc {
     uint32_t* tile_frame;  // per tile: its frame
     uint32_t* tile_list;   // tiles with runs, in tile order
     uint32_t* busy_count;  // their number
+    uint32_t small_tris;       // 1: k_setup counts and bounds the small triangles, the rasterizer passes over hidden ones
     uint32_t clear_in_raster;  // 1: the rasterizer clears the tiles without runs itself
     uint32_t* group_draw;   // per 64-triangle group: the draw of its first triangle
     Run* runs;
     uint32_t runs_cap;
     uint32_t* tile_counter;  // persistent raster work counters, one per tile partition (TILE_PARTS)
     uint32_t* err;
-    unsigned long long* prims_part;  // per frame: PRIM_PARTS partial prims.o counters
+    unsigned long long* prims_part;  // per frame: PRIM_PARTS partial counters (prims.o, frags.i)
     uint32_t* draw_vis;  // per draw: 0 if the bounding-box test hid it, else 1
     uint32_t any_cull;   // some draw asks for the bounding-box test
     // depth sort (render.rs:180-183, 209-219): clip fans in clip space, their keys

@@ -11,7 +11,19 @@ from test_gpu_parity import random_soup
 pytestmark = pytest.mark.gpu
 
 
-def check_frame(w, h, draws, ctx, octx):
+def small_soup(rng, n, w, h, kind):
+    """Triangles a few pixels wide, slivers among them, at random depths: most
+    are hidden once some layers are drawn."""
+    pos, attr, tris, mvp, vp = random_soup(rng, n, w, h, kind)
+    pos = pos.reshape(n, 3, 3)
+    size = rng.choice([0.0, 0.02, 0.1, 0.3], n).astype(np.float32)
+    pos[:, 1:] = pos[:, :1] + (pos[:, 1:] - pos[:, :1]) * size[:, None, None]
+    thin = rng.random(n) < 0.2
+    pos[thin, 2] = pos[thin, 0] + (pos[thin, 1] - pos[thin, 0]) * np.float32(0.999)
+    return pos.reshape(-1, 3), attr, tris, mvp, vp
+
+
+def check_frame(w, h, draws, ctx, octx, soup=random_soup, tile_w=32):
     """One batched frame of (kind, n) random draws equals the oracle's."""
     rng = np.random.default_rng([w, h] + [n for _, n in draws])
     fb = RB.DeviceFramebuf(w, h, 0, True)
@@ -24,13 +36,13 @@ def check_frame(w, h, draws, ctx, octx):
     shaders = {0: rf.shader.Flat((9, 200, 77, 255)), 1: rf.shader.Gouraud(), 3: rf.shader.TexRepeatPot(tex)}
     meshes, mds = [], []
     for kind, n in draws:
-        pos, attr, tris, mvp, vp = random_soup(rng, n, w, h, kind)
+        pos, attr, tris, mvp, vp = soup(rng, n, w, h, kind)
         meshes.append(RB.Mesh(pos, tris, attr))
         mds.append(RB.mesh_draw(meshes[-1], shaders[kind], mvp, vp, texture=dtex if kind == 3 else None))
         err, _ = O.render(kind, tris, pos, attr, mvp, vp, ocol, depth=odep, flat=(9, 200, 77, 255),
                           tex=tex if kind == 3 else None, ctx=octx, stats=ost)
         assert err == 0
-    b = RB.Batch([(fb, ctx, mds)], tile_w=32)
+    b = RB.Batch([(fb, ctx, mds)], tile_w=tile_w)
     for _ in range(2):
         b.run()
         s = b.wait()[0]
@@ -52,3 +64,33 @@ def test_sorted_draws_of_every_size(sizes):
     kinds = [1, 0, 3, 1, 3]
     check_frame(150, 90, [(kinds[i], n) for i, n in enumerate(sizes)],
                 rf.Context(clear=True, depth_test=None, face_cull=None, depth_sort="back_to_front"), (0, 0, 1, 1, 2))
+
+
+@pytest.mark.parametrize("tw,th", [(16, 16), (32, 32), (64, 32), (32, 64), (64, 64)])
+@pytest.mark.parametrize("w,h", [(64, 64), (101, 67)])
+def test_hidden_small_triangles(w, h, tw, th):
+    """Thousands of small triangles a tile, most of them behind others: the
+    tiles pass over those (whole and partial tiles, clipped triangles and
+    large ones among them), and every counter still is the oracle's."""
+    dev = rf.default_device()
+    dev.set_tile_height(th)
+    try:
+        check_frame(w, h, [(1, 4000), (3, 3000), (0, 2000)], rf.Context(clear=True, face_cull=None), (1, 0, 1, 1, 0),
+                    small_soup, tw)
+    finally:
+        dev.set_tile_height(0)
+
+
+@pytest.mark.parametrize("dt,dw", [("less", False), ("greater", True), ("equal", True), (None, True)])
+def test_small_triangles_under_other_tests(dt, dw):
+    """As above where nothing may be passed over, or depth never changes."""
+    check_frame(64, 48, [(3, 3000), (1, 3000)], rf.Context(clear=True, face_cull=None, depth_test=dt, depth_write=dw),
+                ({None: 0, "less": 1, "equal": 2, "greater": 3}[dt], 0, 1, int(dw), 0), small_soup)
+
+
+@pytest.mark.parametrize("n", [61, 62, 63, 130, 300])
+def test_tiles_of_many_draws(n):
+    """More draws meet in one tile than its colour sources can name at a time."""
+    kinds = [3, 1, 3, 0]
+    check_frame(40, 40, [(kinds[i % 4], 1 + i % 3) for i in range(n)], rf.Context(clear=True, face_cull=None),
+                (1, 0, 1, 1, 0))
