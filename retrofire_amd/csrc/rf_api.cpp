@@ -112,12 +112,13 @@ static void scratch_arrays(BatchDesc& B, Fn&& fn) {
     fn(nt * 2 * sizeof(uint32_t), (void**)&B.rect);
     fn(nt * sizeof(float), (void**)&B.zmax);
     fn((nt / 64 + 1) * sizeof(uint32_t), (void**)&B.group_draw);
-    fn(ntl * sizeof(uint32_t), (void**)&B.run_count);
+    fn(run_slot(ntl) * sizeof(uint32_t), (void**)&B.run_count);
     fn((ntl + 1) * sizeof(uint32_t), (void**)&B.run_off);
-    fn(ntl * sizeof(uint32_t), (void**)&B.run_cursor);
+    fn(run_slot(ntl) * sizeof(uint32_t), (void**)&B.run_cursor);
     fn(2 * (ntl / 1024 + 2) * sizeof(uint32_t), (void**)&B.scan_blk);
-    fn(ntl * sizeof(uint32_t), (void**)&B.tile_list);
-    fn(ntl * sizeof(uint32_t), (void**)&B.tile_frame);
+    fn(ntl * sizeof(TileRec), (void**)&B.tiles);
+    fn(ntl * sizeof(uint32_t), (void**)&B.long_list);
+    fn(ntl * sizeof(uint32_t), (void**)&B.heavy_list);
     fn(std::max<uint64_t>(B.runs_cap, 1) * sizeof(Run), (void**)&B.runs);
     fn(nf * sizeof(FrameStats), (void**)&B.stats);
     fn(std::max<uint64_t>(B.n_draws, 1) * sizeof(uint32_t), (void**)&B.draw_vis);
@@ -125,8 +126,8 @@ static void scratch_arrays(BatchDesc& B, Fn&& fn) {
     uint32_t* m = (uint32_t*)misc;
     B.extra_count = m;
     B.err = m ? m + 2 : nullptr;
-    B.busy_count = m ? m + 8 : nullptr;
-    B.tile_counter = m ? m + 16 : nullptr;  // TILE_PARTS + 1 words (busy partitions, empty tiles)
+    B.tile_counts = m ? m + 64 : nullptr;    // TileCount words
+    B.tile_counter = m ? m + 128 : nullptr;  // N_TILE_COUNTERS, TC_STRIDE words apart
 }
 
 uint64_t scratch_bytes(const BatchDesc& B0) {
@@ -391,7 +392,6 @@ void plain_descs(const rf_draw* draw, const rf_target* target, const rf_ctx* ctx
     B.n_tiles = tile_base;
     B.tile_w = tile_w;
     B.chunk = chunk;
-    B.sort_tpw = 1;  // one frame: one tile per binsort wave costs little and spreads dense tiles
     B.tile_h = tile_h;
 }
 

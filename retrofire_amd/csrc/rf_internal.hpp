@@ -40,7 +40,9 @@ struct DevBuf {
 // per-triangle, per-tile and per-frame arrays, each 256-byte aligned).
 // scratch_bytes gives the block's size for B's counts and capacities;
 // scratch_carve sets B's pointers into a block of at least that size.
-constexpr uint64_t MISC_BYTES = 256;  // counters: extra count, error word, busy count, tile counters, fan count
+// Counters: extra count, error word, fan count; from 256 B the tile counts, from
+// 512 B the work counters, each on a line of its own.
+constexpr uint64_t MISC_BYTES = 512 + 4 * N_TILE_COUNTERS * TC_STRIDE;
 uint64_t scratch_bytes(const BatchDesc& B);
 void scratch_carve(BatchDesc& B, uint8_t* base);
 inline uint32_t* misc_words(const BatchDesc& B) { return B.extra_count; }

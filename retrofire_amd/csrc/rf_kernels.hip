@@ -6,10 +6,10 @@
 //              (clip.rs:303-309), frustum clipping (clip.rs:350-400),
 //              to_screen, face culling (render.rs:185-196), the tile rectangle
 //              of each triangle, and the per-tile count of bin runs.
-//   k_scan     exclusive scan of the run counts.
+//   k_scan     exclusive scan of the run counts, the lists of tiles.
 //   k_bin      one wave per group again: writes one run (group, 64-bit mask)
 //              per distinct tile the group touches.
-//   k_binsort  one workgroup per tile: sorts the tile's runs by group, which
+//   k_binsort  sorts the long run lists by group, which
 //              restores primitive submission order inside the tile.
 //   k_raster   one wave per tile (persistent): the tile's depth and colour
 //              sources live in LDS; a lane walks a triangle's edges, then
@@ -29,6 +29,8 @@
 // varying stepping per pixel) are reproduced as serial sums; no closed forms.
 #include <hip/hip_runtime.h>
 
+#include <cstddef>
+
 #include "rf_ff.hpp"
 #include "rf_math.hpp"
 #include "rf_types.hpp"
@@ -37,6 +39,7 @@
 namespace rf {
 
 constexpr int WAVE = 64;
+typedef uint32_t rf_u32x4 __attribute__((ext_vector_type(4)));
 constexpr int BIN_MARGIN = 2;  // pixels around a triangle's bounding box, besides the drift bound
 // Rows above the target (y < 0) that a triangle may fold onto row 0; more is
 // RF_E_VIEWPORT (the row counter y0 + k, a float in the reference, stays
@@ -862,7 +865,7 @@ __global__ __launch_bounds__(256) void k_setup(BatchDesc B) {
     const FrameDesc* F = has_rect ? &B.frames[frame] : nullptr;
     const uint32_t base = has_rect ? F->tile_base : 0, ntx = has_rect ? F->ntx : 0;
     for_each_tile(has_rect, rect_tile(rect[0], twl, thl), rect_tile(rect[1], twl, thl), base, ntx,
-                  [&](uint32_t tile, unsigned long long) { atomicAdd(&B.run_count[tile], 1u); });
+                  [&](uint32_t tile, unsigned long long) { atomicAdd(&B.run_count[run_slot(tile)], 1u); });
 }
 #endif  // RF_RASTER_TU
 
@@ -876,18 +879,135 @@ __device__ __forceinline__ uint32_t find_frame_tile(const FrameDesc* f, uint32_t
 }
 
 // ---------------------------------------------------------------------------
-// k_scan_*: exclusive scan of the run counts over all tiles, in three steps
-// (blocks of 1024 tiles; the block totals; their offsets added back)
+// k_scan*: exclusive scan of the run counts over all tiles (the offsets of
+// their run lists) and the lists of tiles the later kernels work through
 // ---------------------------------------------------------------------------
-// Two scans side by side: run counts (offsets of the tiles' run lists) and
-// "has runs" flags: B.tile_list lists the tiles with runs first, then the
-// others (which the rasterizer only clears).
+// Launches are what a small frame waits for: up to SCAN_ONE tiles, one block
+// does it all (k_scan: a 256 x 256 frame 11.9 -> 8.2 us); above, a block per
+// 1024 tiles, the block totals, and their offsets added back (k_scan_local,
+// k_scan_top, k_scan_add: 14 us at 16,320 tiles, where one block, two steps of
+// 8 tiles a thread, took 47).
 #ifndef RF_RASTER_TU
+constexpr uint32_t SCAN_PER = 4;  // consecutive tiles a thread of k_scan takes
+constexpr uint32_t SCAN_ONE = 1024 * SCAN_PER;
+
+// Appends to a list: the place of each lane that wants one.
+__device__ __forceinline__ uint32_t wave_append(uint32_t* count, bool want) {
+    const unsigned long long m = __ballot(want);
+    if (m == 0ull) return 0;
+    const uint32_t first = (uint32_t)(__ffsll((long long)m) - 1);
+    uint32_t at = 0;
+    if (lane_id() == first) at = atomicAdd(count, (uint32_t)__popcll(m));
+    at = (uint32_t)__builtin_amdgcn_readlane((int)at, (int)first);
+    return at + (uint32_t)__popcll(m & ((1ull << lane_id()) - 1));
+}
+
+// A tile is heavy with 3 times the mean number of runs of the tiles with any,
+// one of the heaviest with 12 times. The rasterizer takes these first, the
+// heaviest before the others, so that no wave is left with one at the end (32
+// mixed frames, in list order 7.2 ms, so 5.1).
+struct HeavyMin {
+    uint32_t heavy, heaviest;
+    __device__ HeavyMin(uint32_t runs, uint32_t busy) {
+        const unsigned long long r = runs, n = busy ? busy : 1u;
+        heavy = (uint32_t)max(min(3ull * r / n, 0xFFFFFFFFull), (unsigned long long)WAVE);
+        heaviest = (uint32_t)max(min(12ull * r / n, 0xFFFFFFFFull), (unsigned long long)WAVE);
+    }
+};
+
+// Tile i's entries: n runs from off, `busy` tiles with runs before it. Called
+// by whole waves (`in`: the lane has a tile); `c` counts the lists' entries
+// (TileCount words).
+__device__ __forceinline__ void place_tile(const BatchDesc& B, uint32_t* c, bool in, uint32_t i, uint32_t n, uint32_t off,
+                                           uint32_t busy, uint32_t frame, const HeavyMin& h) {
+    const uint32_t at = n ? busy : B.n_tiles - 1 - (i - busy);
+    if (in) {
+        B.run_off[i] = off;
+        B.run_cursor[run_slot(i)] = off;
+        B.tiles[at] = TileRec{i, frame, off, n};
+    }
+    const bool huge = in && n > HUGE_RUNS, is_long = in && n > LONG_RUNS && !huge;
+    const bool top = in && n > h.heaviest, heavy = in && n > h.heavy && !top;
+    uint32_t k = wave_append(c + TN_LONG, is_long);
+    if (is_long) B.long_list[k] = at;
+    k = wave_append(c + TN_HUGE, huge);
+    if (huge) B.long_list[B.n_tiles - 1 - k] = at;
+    k = wave_append(c + TN_HEAVIEST, top);
+    if (top) B.heavy_list[k] = at;
+    k = wave_append(c + TN_HEAVY, heavy);
+    if (heavy) B.heavy_list[B.n_tiles - 1 - k] = at;
+}
+
+// Totals known: prims.o and the small triangles' frags.i of every frame from
+// its partial counters (verts.o is 3 per primitive, render.rs:196), and the
+// counters of the kernels that follow.
+__device__ __forceinline__ void scan_totals(const BatchDesc& B, uint32_t runs, uint32_t busy, const HeavyMin& h) {
+    for (uint32_t f = threadIdx.x; f < B.n_frames; f += blockDim.x) {
+        unsigned long long p = 0, fr = 0;
+        for (uint32_t k = 0; k < PRIM_PARTS; ++k) {
+            const unsigned long long* c = &B.prims_part[((uint64_t)f * PRIM_PARTS + k) * PRIM_PART_STRIDE];
+            p += c[0];
+            fr += c[1];
+        }
+        B.stats[f].prims_o = p;
+        B.stats[f].verts_o = 3ull * p;
+        B.stats[f].frags_i = fr;
+    }
+    if (threadIdx.x == 0) {
+        B.run_off[B.n_tiles] = runs;
+        B.tile_counts[TN_BUSY] = busy;
+        B.tile_counts[TN_HEAVY_MIN] = h.heavy;
+        if (runs > B.runs_cap) atomicOr(B.err, ERRB_RUNS);
+    }
+}
+
+__global__ __launch_bounds__(1024) void k_scan(BatchDesc B) {
+    __shared__ uint32_t wave_tot[2][16];
+    __shared__ uint32_t counts[TN_HEAVY_MIN];
+    const uint32_t tid = threadIdx.x, w = tid / WAVE, i0 = tid * SCAN_PER;
+    if (tid < TN_HEAVY_MIN) counts[tid] = 0;
+    uint32_t n[SCAN_PER], v = 0, f = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < SCAN_PER; ++k) {
+        n[k] = i0 + k < B.n_tiles ? B.run_count[run_slot(i0 + k)] : 0u;
+        v += n[k];
+        f += n[k] ? 1u : 0u;
+    }
+    uint32_t frame = i0 < B.n_tiles ? find_frame_tile(B.frames, B.n_frames, i0) : 0u;
+    uint32_t wt, wf, off = wave_excl_scan(v, &wt), busy = wave_excl_scan(f, &wf);
+    if (lane_id() == 0) {
+        wave_tot[0][w] = wt;
+        wave_tot[1][w] = wf;
+    }
+    __syncthreads();
+    uint32_t tot = 0, ftot = 0;
+    for (uint32_t k = 0; k < 16; ++k) {
+        if (k == w) {
+            off += tot;
+            busy += ftot;
+        }
+        tot += wave_tot[0][k];
+        ftot += wave_tot[1][k];
+    }
+    const HeavyMin h(tot, ftot);
+    for (uint32_t k = 0; k < SCAN_PER; ++k) {
+        const uint32_t i = i0 + k;
+        const bool in = i < B.n_tiles;
+        while (in && frame + 1 < B.n_frames && B.frames[frame + 1].tile_base <= i) ++frame;
+        place_tile(B, counts, in, i, n[k], off, busy, frame, h);
+        off += n[k];
+        busy += n[k] ? 1u : 0u;
+    }
+    __syncthreads();
+    if (tid > TN_BUSY && tid < TN_HEAVY_MIN) B.tile_counts[tid] = counts[tid];
+    scan_totals(B, tot, ftot, h);
+}
+
 __global__ __launch_bounds__(1024) void k_scan_local(BatchDesc B) {
     __shared__ uint32_t wave_tot[2][16];
     const uint32_t tid = threadIdx.x, lane = lane_id(), w = tid / WAVE;
     const uint32_t i = blockIdx.x * 1024 + tid;
-    const uint32_t v = i < B.n_tiles ? B.run_count[i] : 0u;
+    const uint32_t v = i < B.n_tiles ? B.run_count[run_slot(i)] : 0u;
     const uint32_t f = v != 0 ? 1u : 0u;
     uint32_t tot, ftot;
     const uint32_t ex = wave_excl_scan(v, &tot);
@@ -903,9 +1023,8 @@ __global__ __launch_bounds__(1024) void k_scan_local(BatchDesc B) {
         foff += wave_tot[1][k];
     }
     if (i < B.n_tiles) {
-        B.run_off[i] = off + ex;
-        B.run_cursor[i] = foff + fex;  // block-local list position until k_scan_add
-        B.tile_frame[i] = find_frame_tile(B.frames, B.n_frames, i);
+        B.run_off[i] = off + ex;        // within the block until k_scan_add
+        B.run_cursor[run_slot(i)] = foff + fex;
     }
     if (tid == 1023) {
         B.scan_blk[2 * blockIdx.x] = off + ex + v;
@@ -945,52 +1064,20 @@ __global__ __launch_bounds__(1024) void k_scan_top(BatchDesc B) {
             for (uint32_t k = 0; k < 16; ++k) carry[tid] += wave_tot[tid][k];
         __syncthreads();
     }
-    // prims.o and the small triangles' frags.i of every frame from its
-    // partial counters; verts.o is 3 per primitive (render.rs:196)
-    for (uint32_t f = tid; f < B.n_frames; f += blockDim.x) {
-        unsigned long long p = 0, fr = 0;
-        for (uint32_t k = 0; k < PRIM_PARTS; ++k) {
-            const unsigned long long* c = &B.prims_part[((uint64_t)f * PRIM_PARTS + k) * PRIM_PART_STRIDE];
-            p += c[0];
-            fr += c[1];
-        }
-        B.stats[f].prims_o = p;
-        B.stats[f].verts_o = 3ull * p;
-        B.stats[f].frags_i = fr;
-    }
-    if (tid == 0) {
-        B.run_off[B.n_tiles] = carry[0];
-        *B.busy_count = carry[1];
-        if (carry[0] > B.runs_cap) atomicOr(B.err, ERRB_RUNS);
-        for (uint32_t k = 0; k <= TILE_PARTS; ++k) B.tile_counter[k] = 0;
-    }
+    scan_totals(B, carry[0], carry[1], HeavyMin(carry[0], carry[1]));
 }
 
 __global__ __launch_bounds__(1024) void k_scan_add(BatchDesc B) {
     const uint32_t i = blockIdx.x * 1024 + threadIdx.x;
-    if (i >= B.n_tiles) return;
-    if (blockIdx.x > 0) B.run_off[i] += B.scan_blk[2 * blockIdx.x];
-    const uint32_t busy_before = B.run_cursor[i] + B.scan_blk[2 * blockIdx.x + 1];
-    B.tile_list[B.run_count[i] != 0 ? busy_before : *B.busy_count + (i - busy_before)] = i;
-    B.run_cursor[i] = 0;
+    const bool in = i < B.n_tiles;
+    const uint32_t off = (in ? B.run_off[i] : 0u) + B.scan_blk[2 * blockIdx.x];
+    const uint32_t busy = (in ? B.run_cursor[run_slot(i)] : 0u) + B.scan_blk[2 * blockIdx.x + 1];
+    place_tile(B, B.tile_counts, in, i, in ? B.run_count[run_slot(i)] : 0u, off, busy, in ? find_frame_tile(B.frames, B.n_frames, i) : 0u,
+               HeavyMin(B.run_off[B.n_tiles], B.tile_counts[TN_BUSY]));
 }
 #endif  // RF_RASTER_TU
 
-#ifndef RF_SORT_LDS
-#define RF_SORT_LDS 1024
-#endif
-#ifndef RF_SORT_TPW
-#define RF_SORT_TPW 8
-#endif
-constexpr int SORT_LDS = RF_SORT_LDS;  // bins up to this many runs sort in LDS
-constexpr int SORT_TPW = RF_SORT_TPW;  // default tiles per k_binsort wave (their sorts run one after another)
-static_assert(SORT_TPW >= 1 && SORT_TPW <= 64, "one lane per tile");
-// Tiles per k_binsort wave of this batch (1..64; 0: the default). One tile a
-// wave spreads dense scenes' long run lists over many waves; 8 a wave costs
-// fewer waves where lists are short.
-__host__ __device__ __forceinline__ uint32_t sort_tpw(const BatchDesc& B) {
-    return B.sort_tpw >= 1 && B.sort_tpw <= 64 ? B.sort_tpw : (uint32_t)SORT_TPW;
-}
+constexpr uint32_t SORT_LDS = 4096;  // run lists up to this long sort in LDS, a block each
 
 // Sorts the runs held one per lane (lanes >= n hold none) by group: a bitonic
 // network over the 64 lanes; lane i ends with the i-th run. Groups are
@@ -1015,82 +1102,89 @@ __device__ __forceinline__ void wave_sort_runs(uint32_t n, uint32_t& group, unsi
     group = (uint32_t)(kk >> 6);
 }
 
-// Orders the runs of each tile with more than 64 of them by group (k_bin
-// appends them in arrival order; the rasterizer sorts lists of up to 64 runs
-// itself, in registers). One wave per sort_tpw(B) tiles, whose long lists it
-// sorts one after another: bins of up to SORT_LDS runs in LDS, larger ones in
-// place in global memory.
+// Orders the runs of each tile with more than LONG_RUNS of them by group
+// (k_bin appends them in arrival order; the rasterizer sorts shorter lists
+// itself, in registers). Each block takes huge lists (more than HUGE_RUNS)
+// until none is left, then its waves take long ones: keys sort in LDS, and the
+// records move once, through registers; lists beyond SORT_LDS sort in place in
+// global memory. Bound by the longest lists: 32 mixed frames, whose lists
+// exceed 1,024 runs, took 0.72 to 1.0 ms with a wave for every list and 1,024
+// keys in LDS, and take 0.37.
 #ifndef RF_RASTER_TU
-__global__ __launch_bounds__(64) void k_binsort(BatchDesc B) {
-    __shared__ unsigned long long key[SORT_LDS];
-    __shared__ unsigned long long msk[SORT_LDS];
-    const uint32_t lane = lane_id();
-    const uint32_t tpw = sort_tpw(B);
-    const uint32_t t0 = blockIdx.x * tpw;
-    const uint32_t t = t0 + lane;
-    uint32_t off = 0, n = 0;
-    if (lane < tpw && t < B.n_tiles) {
-        off = B.run_off[t];
-        n = B.run_off[t + 1] - off;
-        if (off >= B.runs_cap) n = 0;
-        else if (off + n > B.runs_cap) n = B.runs_cap - off;
-    }
-    unsigned long long todo = __ballot(n > (uint32_t)WAVE);
-    while (todo) {
-        const uint32_t j = (uint32_t)(__ffsll((long long)todo) - 1);
-        todo &= todo - 1;
-        const uint32_t o = __shfl(off, j, WAVE), nn = __shfl(n, j, WAVE);
-        Run* runs = B.runs + o;
-        if (nn <= (uint32_t)SORT_LDS) {
-            bool unsorted = false;
-            for (uint32_t i = lane; i + 1 < nn; i += WAVE) unsorted |= runs[i].group > runs[i + 1].group;
-            if (!__ballot(unsorted)) continue;
-            uint32_t p2 = 1;
-            while (p2 < nn) p2 <<= 1;
-            for (uint32_t i = lane; i < nn; i += WAVE) {
-                // groups are distinct in a tile, so the flag and index below
-                // the group never decide the order
-                key[i] = ((unsigned long long)runs[i].group << 32) | ((unsigned long long)runs[i].multi << 31) | i;
-                msk[i] = runs[i].mask;
-            }
-            __syncthreads();
-            // all-ascending bitonic network: the first step of each merge
-            // compares i with i ^ (k - 1), later steps i with i ^ j; indices
-            // >= nn act as +inf keys
-            for (uint32_t ksz = 2; ksz <= p2; ksz <<= 1) {
-                for (uint32_t js = ksz >> 1; js > 0; js >>= 1) {
-                    const uint32_t x = (js == (ksz >> 1)) ? (ksz - 1) : js;
-                    for (uint32_t i = lane; i < nn; i += WAVE) {
-                        const uint32_t l = i ^ x;
-                        if (l > i && l < nn) {
-                            const unsigned long long a = key[i], c = key[l];
-                            if (a > c) {
-                                key[i] = c;
-                                key[l] = a;
-                            }
-                        }
+// Sorts keys [0, n) in LDS by `threads` threads, tid among them: an
+// all-ascending bitonic network. The first step of each merge compares i with
+// i ^ (k - 1), later steps i with i ^ j; indices >= n act as +inf keys.
+template <class Barrier>
+__device__ __forceinline__ void bitonic_lds(unsigned long long* key, uint32_t n, uint32_t tid, uint32_t threads,
+                                            Barrier&& barrier) {
+    uint32_t p2 = 1;
+    while (p2 < n) p2 <<= 1;
+    for (uint32_t ksz = 2; ksz <= p2; ksz <<= 1) {
+        for (uint32_t js = ksz >> 1; js > 0; js >>= 1) {
+            const uint32_t x = (js == (ksz >> 1)) ? (ksz - 1) : js;
+            // the q-th index with bit js clear, and its partner
+            for (uint32_t q = tid; q < p2 / 2; q += threads) {
+                const uint32_t i = ((q & ~(js - 1)) << 1) | (q & (js - 1)), l = i ^ x;
+                if (l < n) {
+                    const unsigned long long a = key[i], c = key[l];
+                    if (a > c) {
+                        key[i] = c;
+                        key[l] = a;
                     }
-                    __syncthreads();
                 }
             }
-            for (uint32_t i = lane; i < nn; i += WAVE) {
-                Run w;
-                w.group = (uint32_t)(key[i] >> 32);
-                w.multi = (uint32_t)(key[i] >> 31) & 1u;
-                w.mask = msk[(uint32_t)key[i] & 0x7FFFFFFFu];
-                runs[i] = w;
-            }
-            __syncthreads();
+            barrier();
+        }
+    }
+}
+// Orders a list of n <= threads * 16 runs: keys in LDS, then the records. (A
+// list without room, n = 0, has no first record either.)
+template <class Barrier>
+__device__ __forceinline__ void sort_runs(rf_u32x4* runs, uint32_t n, unsigned long long* key, uint32_t tid,
+                                          uint32_t threads, Barrier&& barrier) {
+    static_assert(sizeof(Run) == sizeof(rf_u32x4) && offsetof(Run, group) == 0, "a run moves as one 16-byte access");
+    if (n < 2) return;
+    for (uint32_t i = tid; i < n; i += threads) key[i] = ((unsigned long long)runs[i][0] << 32) | i;
+    barrier();
+    bitonic_lds(key, n, tid, threads, barrier);
+    rf_u32x4 mine[16];
+#pragma unroll
+    for (uint32_t k = 0; k < 16; ++k) {
+        const uint32_t i = tid + threads * k;
+        if (threads * k < n) mine[k] = runs[i < n ? (uint32_t)key[i] : 0u];
+    }
+    barrier();
+#pragma unroll
+    for (uint32_t k = 0; k < 16; ++k)
+        if (tid + threads * k < n) runs[tid + threads * k] = mine[k];
+}
+
+__global__ __launch_bounds__(256) void k_binsort(BatchDesc B) {
+    __shared__ unsigned long long key[SORT_LDS];
+    __shared__ uint32_t s_next;
+    static_assert(HUGE_RUNS * 4 <= SORT_LDS && HUGE_RUNS <= 16 * WAVE && SORT_LDS <= 16 * 256, "see sort_runs");
+    const uint32_t tid = threadIdx.x, lane = lane_id(), wave = tid / WAVE;
+    const uint32_t n_huge = B.tile_counts[TN_HUGE], n_long = B.tile_counts[TN_LONG];
+    // a block's (wave's) first list is the one of its number; more come by a counter
+    auto runs_of = [&](uint32_t place, uint32_t& n) {
+        const TileRec T = B.tiles[place];
+        n = T.off >= B.runs_cap ? 0u : min(T.nruns, B.runs_cap - T.off);
+        return B.runs + T.off;
+    };
+    for (uint32_t k = blockIdx.x; k < n_huge;) {
+        uint32_t n;
+        Run* const runs = runs_of(B.long_list[B.n_tiles - 1 - k], n);
+        if (n <= SORT_LDS) {
+            sort_runs(reinterpret_cast<rf_u32x4*>(runs), n, key, tid, 256u, [] { __syncthreads(); });
         } else {
-            // very large bin: the same network in place on the run records
             uint32_t p2 = 1;
-            while (p2 < nn) p2 <<= 1;
+            while (p2 < n) p2 <<= 1;
             for (uint32_t ksz = 2; ksz <= p2; ksz <<= 1) {
                 for (uint32_t js = ksz >> 1; js > 0; js >>= 1) {
                     const uint32_t x = (js == (ksz >> 1)) ? (ksz - 1) : js;
-                    for (uint32_t i = lane; i < nn; i += WAVE) {
-                        const uint32_t l = i ^ x;
-                        if (l > i && l < nn) {
+                    for (uint32_t q = tid; q < p2 / 2; q += 256) {
+                        const uint32_t i = ((q & ~(js - 1)) << 1) | (q & (js - 1)), l = i ^ x;
+                        if (l < n) {
                             const Run a = runs[i], c = runs[l];
                             if (a.group > c.group) {
                                 runs[i] = c;
@@ -1103,6 +1197,20 @@ __global__ __launch_bounds__(64) void k_binsort(BatchDesc B) {
                 }
             }
         }
+        if (tid == 0) s_next = gridDim.x + atomicAdd(&B.tile_counter[TC_HUGE * TC_STRIDE], 1u);
+        __syncthreads();
+        k = s_next;
+        __syncthreads();
+    }
+    for (uint32_t k = blockIdx.x * 4 + wave; k < n_long;) {
+        uint32_t n;
+        Run* const runs = runs_of(B.long_list[k], n);
+        // a wave's LDS accesses are performed in order
+        sort_runs(reinterpret_cast<rf_u32x4*>(runs), n, key + wave * HUGE_RUNS, lane, (uint32_t)WAVE,
+                  [] { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); });
+        uint32_t c = 0;
+        if (lane == 0) c = atomicAdd(&B.tile_counter[TC_LONG * TC_STRIDE], 1u);
+        k = gridDim.x * 4 + (uint32_t)__builtin_amdgcn_readfirstlane((int)c);
     }
 }
 #endif  // RF_RASTER_TU
@@ -1118,7 +1226,6 @@ __global__ __launch_bounds__(64) void k_binsort(BatchDesc B) {
 #ifndef RF_NT_STORE
 #define RF_NT_STORE 1
 #endif
-typedef uint32_t rf_u32x4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ void st16(void* p, uint32_t a, uint32_t b, uint32_t c, uint32_t d) {
 #if RF_NT_STORE
     __builtin_nontemporal_store(rf_u32x4{a, b, c, d}, (rf_u32x4*)p);
@@ -1147,17 +1254,8 @@ __device__ __forceinline__ void store_pixel(const FrameDesc& F, uint32_t x, uint
 }
 
 
-#ifndef RF_CLEAR_ROWS
-#define RF_CLEAR_ROWS 1  // clear runs of empty tiles row segment by row segment
-#endif
-#ifndef RF_EARLY_CLEAR
-#define RF_EARLY_CLEAR 0  // workgroups that clear the tiles without runs first
-#endif
 #ifndef RF_VEC_INIT
 #define RF_VEC_INIT 1  // tile init of a cleared frame with 16-byte LDS fills
-#endif
-#ifndef RF_CLEAR_IN_RASTER
-#define RF_CLEAR_IN_RASTER 1
 #endif
 #ifndef RF_EMPTY_GRAB
 #define RF_EMPTY_GRAB 32
@@ -1196,53 +1294,9 @@ __device__ __forceinline__ void clear_tile(const FrameDesc& F, uint32_t tile, ui
     }
 }
 
-// Clears tiles without runs (listed after the others in B.tile_list): wave
-// `w` takes EMPTY_GRAB list entries.
-__device__ __forceinline__ void clear_empty_tiles(const BatchDesc& B, uint32_t w, uint32_t lane) {
-    const uint32_t n_busy = *B.busy_count, n_empty = B.n_tiles - n_busy;
-    const uint32_t e0 = w * EMPTY_GRAB;
-    if (e0 >= n_empty) return;
-    const uint32_t ne = min((uint32_t)EMPTY_GRAB, n_empty - e0);
-    uint32_t my_tile = 0, my_fi = 0;
-    if (lane < ne) {
-        my_tile = B.tile_list[n_busy + e0 + lane];
-        my_fi = B.tile_frame[my_tile];
-    }
-    uint32_t cur_fi = 0xFFFFFFFFu;
-    FrameDesc F;
-    for (uint32_t j = 0; j < ne; ++j) {
-        const uint32_t tile = (uint32_t)__builtin_amdgcn_readlane((int)my_tile, (int)j);
-        const uint32_t fi = (uint32_t)__builtin_amdgcn_readlane((int)my_fi, (int)j);
-        if (fi != cur_fi) {
-            F = B.frames[fi];
-            cur_fi = fi;
-        }
-        if (B.tile_h == 16) {
-            if (B.tile_w == 16) clear_tile<16, 16>(F, tile, lane);
-            else if (B.tile_w == 32) clear_tile<32, 16>(F, tile, lane);
-            else clear_tile<64, 16>(F, tile, lane);
-        } else if (B.tile_h == 64) {
-            if (B.tile_w == 16) clear_tile<16, 64>(F, tile, lane);
-            else if (B.tile_w == 32) clear_tile<32, 64>(F, tile, lane);
-            else clear_tile<64, 64>(F, tile, lane);
-        } else {
-            if (B.tile_w == 16) clear_tile<16, 32>(F, tile, lane);
-            else if (B.tile_w == 32) clear_tile<32, 32>(F, tile, lane);
-            else clear_tile<64, 32>(F, tile, lane);
-        }
-    }
-}
-
-// Blocks past the groups' clear the tiles without runs: binning waits on
-// atomics and loads while the clears only store, so they share the GPU well.
 #ifndef RF_RASTER_TU
 __global__ __launch_bounds__(256) void k_bin(BatchDesc B) {
     const uint32_t lane = lane_id();
-    const uint32_t bin_blocks = (B.n_groups + 3) / 4;
-    if (blockIdx.x >= bin_blocks) {
-        if (!B.clear_in_raster) clear_empty_tiles(B, (blockIdx.x - bin_blocks) * 4 + threadIdx.x / WAVE, lane);
-        return;
-    }
     const uint32_t group = blockIdx.x * (blockDim.x / WAVE) + threadIdx.x / WAVE;
     if (group >= B.n_groups) return;
     const uint64_t g = (uint64_t)group * WAVE + lane;
@@ -1274,7 +1328,7 @@ __global__ __launch_bounds__(256) void k_bin(BatchDesc B) {
     unsigned long long my_mask = 0;
     auto flush = [&]() {
         if (lane < k) {
-            const uint32_t pos = B.run_off[my_tile] + atomicAdd(&B.run_cursor[my_tile], 1u);
+            const uint32_t pos = atomicAdd(&B.run_cursor[run_slot(my_tile)], 1u);
             if (pos < cap) {
                 Run r;
                 r.group = group;
@@ -1351,14 +1405,6 @@ __host__ __device__ constexpr int rec_cap(int tw, int th) {
     const int r = (share - f) / REC_BYTES / 32 * 32;
     return r < 480 ? r : 480;
 }
-#ifndef RF_TILE_GRAB
-#define RF_TILE_GRAB 1
-#endif
-constexpr int TILE_GRAB = RF_TILE_GRAB;  // tiles a wave takes from the shared counter at once
-#ifndef RF_TILE_TAIL
-#define RF_TILE_TAIL 512
-#endif
-constexpr int TILE_TAIL = RF_TILE_TAIL;  // the last tiles of a partition are taken one at a time
 #ifndef RF_KMAX
 #define RF_KMAX 600
 #endif
@@ -1490,32 +1536,33 @@ __global__ __launch_bounds__(64, 2) void k_raster(BatchDesc B) {
 
     const uint32_t lane = lane_id();
     for (uint32_t i = lane; i < (uint32_t)(TILE_H * NCG); i += WAVE) s_cell[i] = 0xFFFFFFFFu;
-    // Tiles come from TILE_PARTS contiguous partitions with a counter each.
-    // Workgroups are dispatched round-robin over the XCDs, so a workgroup
-    // starts on partition blockIdx.x % TILE_PARTS: neighbouring tiles (which
-    // share triangles) meet in one XCD's L2. A wave takes TILE_GRAB tiles per
-    // atomic and moves on to the next partition when its own is done.
-    const uint32_t n_busy = *B.busy_count;  // tiles with runs, listed in B.tile_list
-    // The tiles without runs, EMPTY_GRAB per atomic: their fused clear is the
-    // only write. The first EARLY_CLEAR workgroups start with them, so these
-    // stores overlap the busy tiles' work; every wave takes what is left at
-    // its end.
-    const uint32_t n_empty = B.clear_in_raster ? B.n_tiles - n_busy : 0u;
+    // Tiles come from the heavy list, then from TILE_PARTS contiguous
+    // partitions of all tiles with runs, with a counter each. Workgroups are
+    // dispatched round-robin over the XCDs, so a workgroup starts on partition
+    // blockIdx.x % TILE_PARTS: neighbouring tiles (which share triangles) meet
+    // in one XCD's L2. A wave takes one tile per atomic and moves on to the
+    // next partition when its own is done.
+    // (The lists' lengths are read again for each tile: kept, they take scalar
+    // registers that spill.)
+    // The tiles without runs, EMPTY_GRAB per atomic, at the waves' end: their
+    // fused clear is the only write.
     auto clear_empties = [&]() {
+        const uint32_t n_empty = B.n_tiles - B.tile_counts[TN_BUSY];
         uint32_t ecur_fi = 0xFFFFFFFFu;
         FrameDesc E;
         for (;;) {
             uint32_t e0 = 0;
-            if (lane == 0) e0 = atomicAdd(&B.tile_counter[TILE_PARTS], (uint32_t)EMPTY_GRAB);
+            if (lane == 0) e0 = atomicAdd(&B.tile_counter[TC_EMPTY * TC_STRIDE], (uint32_t)EMPTY_GRAB);
             e0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)e0);
             if (e0 >= n_empty) break;
             const uint32_t ne = min((uint32_t)EMPTY_GRAB, n_empty - e0);
             uint32_t my_tile = 0, my_fi = 0;
             if (lane < ne) {
-                my_tile = B.tile_list[n_busy + e0 + lane];
-                my_fi = B.tile_frame[my_tile];
+                const TileRec T = B.tiles[B.n_tiles - 1 - (e0 + lane)];
+                my_tile = T.tile;
+                my_fi = T.frame;
             }
-            if (RF_CLEAR_ROWS) {
+            {
                 // ne consecutive full tiles of one tile row of one frame (the
                 // common case: the list is in tile order): clear the row
                 // segment they make, each store instruction 1 KB of one pixel row
@@ -1563,38 +1610,51 @@ __global__ __launch_bounds__(64, 2) void k_raster(BatchDesc B) {
             }
         }
     };
-    if (blockIdx.x < (uint32_t)RF_EARLY_CLEAR) clear_empties();
-    uint32_t part = blockIdx.x % TILE_PARTS, parts_left = TILE_PARTS;
-    uint32_t tcur = 0, tend = 0;
-    bool tail_near = false;
+    // The wave's next tile: its atomic is in flight while the tile before is
+    // written back.
+    uint32_t stage = 0;  // 0: the heavy list, else the partitions in turn from the wave's own
+    uint32_t claim = 0;
+    auto take = [&]() {
+        const uint32_t part = (blockIdx.x + stage - 1) % TILE_PARTS;
+        if (lane == 0) claim = atomicAdd(&B.tile_counter[(stage ? part : TC_HEAVY) * TC_STRIDE], 1u);
+    };
+    if (B.tile_counts[TN_HEAVIEST] + B.tile_counts[TN_HEAVY] == 0) stage = 1;
+    take();
     for (;;) {
-        while (tcur >= tend && parts_left) {
-            const uint32_t pb = (uint32_t)(((uint64_t)n_busy * part) / TILE_PARTS);
-            const uint32_t pe = (uint32_t)(((uint64_t)n_busy * (part + 1)) / TILE_PARTS);
-            // near a partition's end single tiles keep the tail short
-            const uint32_t grab = tail_near ? 1u : (uint32_t)TILE_GRAB;
-            uint32_t t0 = 0;
-            if (lane == 0) t0 = atomicAdd(&B.tile_counter[part], grab);
-            t0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)t0);
-            if (t0 < pe - pb) {
-                tcur = pb + t0;
-                tend = min(tcur + grab, pe);
-                tail_near = t0 + (uint32_t)TILE_TAIL >= pe - pb;
+        TileRec T;
+        bool got = false;
+        while (!got && stage <= TILE_PARTS) {
+            const uint32_t t0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)claim);
+            if (stage == 0) {
+                const uint32_t n_top = B.tile_counts[TN_HEAVIEST];
+                if (t0 < n_top + B.tile_counts[TN_HEAVY]) {
+                    T = B.tiles[B.heavy_list[t0 < n_top ? t0 : B.n_tiles - 1 - (t0 - n_top)]];
+                    got = true;
+                }
             } else {
-                part = (part + 1) % TILE_PARTS;
-                --parts_left;
-                tail_near = true;  // other partitions are in their tails too
+                const uint32_t part = (blockIdx.x + stage - 1) % TILE_PARTS, n_busy = B.tile_counts[TN_BUSY];
+                const uint32_t pb = (uint32_t)(((uint64_t)n_busy * part) / TILE_PARTS);
+                const uint32_t pe = (uint32_t)(((uint64_t)n_busy * (part + 1)) / TILE_PARTS);
+                if (t0 < pe - pb) {
+                    T = B.tiles[pb + t0];
+                    got = T.nruns <= B.tile_counts[TN_HEAVY_MIN];  // the heavy ones are drawn already
+                    if (!got) {
+                        take();
+                        continue;
+                    }
+                }
             }
+            if (!got && ++stage <= TILE_PARTS) take();
         }
-        if (tcur >= tend) break;
-        const uint32_t tile = B.tile_list[tcur++];
-        const uint32_t fi = B.tile_frame[tile];
+        if (!got) break;
+        const uint32_t tile = (uint32_t)__builtin_amdgcn_readfirstlane((int)T.tile);
+        const uint32_t fi = (uint32_t)__builtin_amdgcn_readfirstlane((int)T.frame);
         const FrameDesc F = B.frames[fi];
         const uint32_t lt = tile - F.tile_base;
         const uint32_t tx = lt % F.ntx, ty = lt / F.ntx;
         const uint32_t x0 = tx * TW, y0 = ty * TILE_H;
-        const uint32_t off = B.run_off[tile];
-        uint32_t nruns = B.run_off[tile + 1] - off;
+        const uint32_t off = (uint32_t)__builtin_amdgcn_readfirstlane((int)T.off);
+        uint32_t nruns = (uint32_t)__builtin_amdgcn_readfirstlane((int)T.nruns);
         if (off >= B.runs_cap) nruns = 0;
         else if (off + nruns > B.runs_cap) nruns = B.runs_cap - off;
         const bool has_depth = F.depth != nullptr;
@@ -1608,8 +1668,8 @@ __global__ __launch_bounds__(64, 2) void k_raster(BatchDesc B) {
         const bool vec = ncols == (uint32_t)TW && pixfmt_bytes(F.fmt) == 4u && ((uintptr_t)F.color & 15u) == 0 &&
                          (F.color_stride & 15u) == 0 && (!has_depth || (((uintptr_t)F.depth & 15u) == 0 &&
                                                                          (F.depth_stride & 3u) == 0));
-        if (nruns == 0) {
-            clear_tile<TW, TH>(F, tile, lane);
+        if (nruns == 0) {  // no room for its runs: the launch is done again
+            take();
             continue;
         }
 
@@ -2190,6 +2250,7 @@ __global__ __launch_bounds__(64, 2) void k_raster(BatchDesc B) {
                 }
         __syncthreads();
 
+        take();
         // write-back: fetch the texels, colour and depth to the target
         if (vec && (F.clear_color || F.color_write)) {
             // four pixels per lane; every load of a quad is issued before use
@@ -2463,7 +2524,7 @@ __global__ __launch_bounds__(256) void k_cull(BatchDesc B) {
 // Zeroes per-batch counters (a kernel, so it can live inside a captured graph).
 __global__ void k_reset(BatchDesc B) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < B.n_tiles) B.run_count[i] = 0;
+    if (i < B.n_tiles) B.run_count[run_slot(i)] = 0;
     // the draw of each group's first triangle
     if (i < B.n_groups) B.group_draw[i] = find_draw_tri(B.draws, B.n_draws, (uint64_t)i * WAVE);
     if (i < B.n_frames * PRIM_PARTS) {
@@ -2483,7 +2544,8 @@ __global__ void k_reset(BatchDesc B) {
         *B.extra_count = 0;
         *B.err = 0;
         if (B.fan_count) *B.fan_count = 0;
-        for (uint32_t k = 0; k < TILE_PARTS; ++k) B.tile_counter[k] = 0;
+        for (uint32_t k = 0; k < N_TILE_COUNTERS; ++k) B.tile_counter[k * TC_STRIDE] = 0;
+        for (uint32_t k = TN_BUSY; k <= TN_HEAVY_MIN; ++k) B.tile_counts[k] = 0;
     }
     if (B.fan_cnt && i < B.n_draws) B.fan_cnt[i] = 0;
 }
@@ -2493,9 +2555,6 @@ __global__ void k_reset(BatchDesc B) {
 // ---------------------------------------------------------------------------
 static hipError_t launch_impl(const BatchDesc& B0, hipStream_t s, uint32_t raster_grid, hipEvent_t* ev) {
     BatchDesc B = B0;
-    // the rasterizer's waves clear the tiles without runs at their end (faster,
-    // measured, than k_bin's extra blocks doing it beside the binning)
-    B.clear_in_raster = RF_CLEAR_IN_RASTER;
     B.small_tris = B.n_tris > (uint64_t)RF_SMALL_TRIS * B.n_tiles;
     uint32_t reset_n = B.n_tiles > B.n_frames * PRIM_PARTS ? B.n_tiles : B.n_frames * PRIM_PARTS;
     reset_n = reset_n > B.n_groups ? reset_n : B.n_groups;
@@ -2513,18 +2572,19 @@ static hipError_t launch_impl(const BatchDesc& B0, hipStream_t s, uint32_t raste
     if (B.n_groups) hipLaunchKernelGGL(k_setup, dim3((B.n_groups + 3) / 4), dim3(256), 0, s, B);
     mark(2);
     const uint32_t nb = (B.n_tiles + 1023) / 1024;
-    hipLaunchKernelGGL(k_scan_local, dim3(nb ? nb : 1), dim3(1024), 0, s, B);
-    hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(1024), 0, s, B);
-    hipLaunchKernelGGL(k_scan_add, dim3(nb ? nb : 1), dim3(1024), 0, s, B);
-    mark(3);
-    {
-        const uint32_t bin_blocks = (B.n_groups + 3) / 4;
-        const uint32_t clear_blocks = B.clear_in_raster ? 0u : (B.n_tiles + 4 * EMPTY_GRAB - 1) / (4 * EMPTY_GRAB);
-        if (bin_blocks + clear_blocks)
-            hipLaunchKernelGGL(k_bin, dim3(bin_blocks + clear_blocks), dim3(256), 0, s, B);
+    if (B.n_tiles <= SCAN_ONE) {
+        hipLaunchKernelGGL(k_scan, dim3(1), dim3(1024), 0, s, B);
+    } else {
+        hipLaunchKernelGGL(k_scan_local, dim3(nb), dim3(1024), 0, s, B);
+        hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(1024), 0, s, B);
+        hipLaunchKernelGGL(k_scan_add, dim3(nb), dim3(1024), 0, s, B);
     }
+    mark(3);
+    if (B.n_groups) hipLaunchKernelGGL(k_bin, dim3((B.n_groups + 3) / 4), dim3(256), 0, s, B);
     mark(4);
-    hipLaunchKernelGGL(k_binsort, dim3((B.n_tiles + sort_tpw(B) - 1) / sort_tpw(B)), dim3(WAVE), 0, s, B);
+    // no tile has more than 64 runs where there are no more groups
+    if (B.n_groups > (uint32_t)WAVE)
+        hipLaunchKernelGGL(k_binsort, dim3(B.n_tiles < 1024u ? B.n_tiles : 1024u), dim3(256), 0, s, B);
     mark(5);
     chk(hipGetLastError());
     chk(launch_raster(B, s, raster_grid));

@@ -516,7 +516,6 @@ static rf_status launch_lane_sorted(Serve& s, Lane& l) {
     B.tile_w = SERVE_TILE_W;
     B.tile_h = DEFAULT_TILE_H;
     B.chunk = RF_SERVE_CHUNK;
-    B.sort_tpw = 1;
     B.any_cull = any_cull;
     B.extra_cap = l.extra_cap;
     B.runs_cap = std::max<uint32_t>(4 * B.n_groups + B.n_tiles + 1024, l.runs_cap);
@@ -560,7 +559,6 @@ static rf_status launch_lane(Serve& s, Lane& l) {
     B.tile_w = SERVE_TILE_W;
     B.tile_h = DEFAULT_TILE_H;
     B.chunk = RF_SERVE_CHUNK;  // span chunk of served launches
-    B.sort_tpw = 1;            // few frames a launch: one tile per binsort wave
     B.extra_cap = l.extra_cap;
     B.runs_cap = l.runs_cap;
     const uint64_t sb = scratch_bytes(B);

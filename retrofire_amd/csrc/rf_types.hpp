@@ -145,6 +145,35 @@ struct Run {
     unsigned long long mask;
 };
 
+// A tile as the rasterizer takes it: all it needs to start, in one load.
+struct alignas(16) TileRec {
+    uint32_t tile, frame, off, nruns;  // its runs are runs[off .. off + nruns)
+};
+// Words of BatchDesc::tile_counts.
+enum TileCount : uint32_t {
+    TN_BUSY = 0,       // tiles with runs
+    TN_LONG = 1,       // entries of long_list from its front
+    TN_HUGE = 2,       // and from its end
+    TN_HEAVIEST = 3,   // entries of heavy_list from its front
+    TN_HEAVY = 4,      // and from its end
+    TN_HEAVY_MIN = 5,  // tiles of more runs than this are in heavy_list
+};
+constexpr uint32_t LONG_RUNS = 64, HUGE_RUNS = 1024;  // run lists longer than these (see k_binsort)
+// Work counters behind the partitions' (BatchDesc::tile_counter).
+constexpr uint32_t TC_EMPTY = TILE_PARTS, TC_HEAVY = TILE_PARTS + 1, TC_LONG = TILE_PARTS + 2, TC_HUGE = TILE_PARTS + 3;
+constexpr uint32_t N_TILE_COUNTERS = TILE_PARTS + 4;
+// Words between them: on one line, with the tile counts that every wave reads,
+// 22,000 atomics from eight dies made the rasterizer wait (32 crates1080 frames:
+// 0.62 ms, on lines of their own 0.46).
+constexpr uint32_t TC_STRIDE = 32;
+
+// Atomics on one line of memory wait for each other: four counters of
+// neighbouring tiles to a line of 128 bytes, where thirty-two took k_bin of 32
+// mixed frames 1.22 ms and these 0.74 (k_setup 3.03 -> 2.76; eight a line 0.77
+// and 2.83, one a line 0.70 and 2.75, but their scan 0.042 for 0.034).
+constexpr uint32_t RUN_STRIDE = 8;  // words
+__host__ __device__ inline uint64_t run_slot(uint32_t tile) { return (uint64_t)tile * RUN_STRIDE; }
+
 struct BatchDesc {
     const DrawDesc* draws;
     const FrameDesc* frames;
@@ -156,7 +185,6 @@ struct BatchDesc {
     uint32_t n_tiles;   // total tiles over all frames
     uint32_t tile_w, tile_h;  // rasterizer tile: 16, 32 or 64 columns x 16, 32 or 64 rows
     uint32_t chunk;     // rasterizer span chunk: 6 or 8 pixels (anything else: 8)
-    uint32_t sort_tpw;  // tiles per k_binsort wave (1..64; 0: the default, 8)
     // scratch
     float* sv;           // screen vertex (x, y, z, a0, a1, a2) per slot of the pre draws
     uint32_t* hdr;       // per triangle: surviving fan count | extra base << 3
@@ -166,19 +194,19 @@ struct BatchDesc {
     uint32_t extra_cap;
     uint32_t* rect;      // per triangle: pixel rect (c0 | r0 << 16, c1 | r1 << 16; all ones: none), 2 words
     float* zmax;         // per triangle: no fragment's z is above it (+inf: not known)
-    uint32_t* run_count; // per tile
+    uint32_t* run_count; // per tile (run_slot)
     uint32_t* run_off;   // per tile + 1 (exclusive scan)
-    uint32_t* run_cursor;
+    uint32_t* run_cursor;  // per tile (run_slot): where its next run goes
     uint32_t* scan_blk;  // per 1024 tiles: run total, then its offset
-    uint32_t* tile_frame;  // per tile: its frame
-    uint32_t* tile_list;   // tiles with runs, in tile order
-    uint32_t* busy_count;  // their number
+    TileRec* tiles;        // the tiles with runs in tile order, then, from the end down, the others in tile order
+    uint32_t* long_list;   // places in `tiles` of those with a long list of runs, from the front, and a huge one, from the end
+    uint32_t* heavy_list;  // places in `tiles` of the heaviest, from the front, and of the heavy ones, from the end
+    uint32_t* tile_counts; // TileCount words
     uint32_t small_tris;       // 1: k_setup counts and bounds the small triangles, the rasterizer passes over hidden ones
-    uint32_t clear_in_raster;  // 1: the rasterizer clears the tiles without runs itself
     uint32_t* group_draw;   // per 64-triangle group: the draw of its first triangle
     Run* runs;
     uint32_t runs_cap;
-    uint32_t* tile_counter;  // persistent raster work counters, one per tile partition (TILE_PARTS)
+    uint32_t* tile_counter;  // work counters: one per tile partition, TC_* (N_TILE_COUNTERS)
     uint32_t* err;
     unsigned long long* prims_part;  // per frame: PRIM_PARTS partial counters (prims.o, frags.i)
     uint32_t* draw_vis;  // per draw: 0 if the bounding-box test hid it, else 1

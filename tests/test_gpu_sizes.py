@@ -6,6 +6,7 @@ import pytest
 import oracle_lib as O
 import retrofire_amd as rf
 from retrofire_amd import batch as RB
+from retrofire_amd import mat as M
 from test_gpu_parity import random_soup
 
 pytestmark = pytest.mark.gpu
@@ -94,3 +95,76 @@ def test_tiles_of_many_draws(n):
     kinds = [3, 1, 3, 0]
     check_frame(40, 40, [(kinds[i % 4], 1 + i % 3) for i in range(n)], rf.Context(clear=True, face_cull=None),
                 (1, 0, 1, 1, 0))
+
+
+@pytest.mark.parametrize("runs", [63, 64, 65, 1023, 1024, 1025, 4096, 4097])
+def test_run_lists_of_every_length(runs):
+    """One tile of a 16 x 16 frame with about 64 triangles in each of `runs`
+    groups: lists are ordered in registers, by a wave, by a block and in global
+    memory, and a small triangle in front decides nothing about the others."""
+    w = h = 16
+    rng = np.random.default_rng(runs)
+    n = 64 * runs
+    # every triangle meets the frame, so every group has its run in the tile
+    pos = rng.uniform([-0.9, -0.9, 0.0], [0.9, 0.9, 4.0], size=(n, 1, 3)).astype(np.float32)
+    pos = (pos + rng.uniform(-0.3, 0.3, size=(n, 3, 3)).astype(np.float32)).reshape(-1, 3)
+    tris = np.arange(3 * n, dtype=np.uint32).reshape(n, 3)
+    attr = rng.uniform(0, 1, size=(3 * n, 3)).astype(np.float32)
+    mvp = M.then(M.translate3(0, 0, 2.0), M.perspective(1.2, np.float32(1.0), 0.1, 8.0))
+    vp = M.viewport(0, h, w, 0)
+    ocol, odep, ost = np.zeros((h, w, 4), np.uint8), np.zeros((h, w), np.float32), np.zeros(8, np.uint64)
+    ocol[...] = (0, 0, 0, 255)
+    err, _ = O.render(1, tris, pos, attr, mvp, vp, ocol, depth=odep, ctx=(1, 0, 1, 1, 0), stats=ost)
+    assert err == 0
+    fb, m = RB.DeviceFramebuf(w, h, 0, True), RB.Mesh(pos, tris, attr)
+    b = RB.Batch([(fb, rf.Context(clear=True, face_cull=None), [RB.mesh_draw(m, rf.shader.Gouraud(), mvp, vp)])],
+                 tile_w=16)
+    for _ in range(2):
+        b.run()
+        s = b.wait()[0]
+        gcol, gdep = fb.read()
+        assert np.array_equal(gcol, ocol)
+        assert np.array_equal(gdep.view(np.uint32), odep.view(np.uint32))
+        assert [s.prims_o, s.frags_i, s.frags_o] == [int(ost[2]), int(ost[5]), int(ost[6])]
+    b.free()
+    fb.free()
+    m.free()
+
+
+@pytest.mark.parametrize("frames", [1, 255, 256, 257, 600])
+def test_tile_counts_around_the_scan_kernels(frames):
+    """64 x 64 frames of 16 tiles each, 4,096 tiles being what one block scans:
+    empty frames, dense ones (whose tiles are heavy) and ordinary ones."""
+    rng = np.random.default_rng(frames)
+    w = h = 64
+    soups = [small_soup(rng, n, w, h, 1) for n in (3, 40, 1500)]
+    meshes = [RB.Mesh(p, t, a) for p, a, t, _, _ in soups]
+    want = []
+    for pos, attr, tris, mvp, vp in soups:
+        ocol, odep, ost = np.zeros((h, w, 4), np.uint8), np.zeros((h, w), np.float32), np.zeros(8, np.uint64)
+        ocol[...] = (0, 0, 0, 255)
+        err, _ = O.render(1, tris, pos, attr, mvp, vp, ocol, depth=odep, ctx=(1, 0, 1, 1, 0), stats=ost)
+        assert err == 0
+        want.append((ocol, odep, int(ost[5]), int(ost[6])))
+    dev = rf.default_device()
+    dev.set_tile_height(16)
+    try:
+        which = [None if i % 7 == 3 else 2 if i % 11 == 0 else i % 2 for i in range(frames)]
+        fbs = [RB.DeviceFramebuf(w, h, 0, True) for _ in range(frames)]
+        ctx = rf.Context(clear=True, face_cull=None)
+        b = RB.Batch([(fbs[i], ctx, [] if k is None else [RB.mesh_draw(meshes[k], rf.shader.Gouraud(), *soups[k][3:])])
+                      for i, k in enumerate(which)], tile_w=16)
+        b.run()
+        for fb, k, s in zip(fbs, which, b.wait()):
+            gcol, gdep = fb.read()
+            if k is None:
+                assert (gcol == (0, 0, 0, 255)).all() and (gdep == 0).all() and s.frags_i == 0
+            else:
+                assert np.array_equal(gcol, want[k][0])
+                assert np.array_equal(gdep.view(np.uint32), want[k][1].view(np.uint32))
+                assert (s.frags_i, s.frags_o) == want[k][2:]
+        b.free()
+    finally:
+        dev.set_tile_height(0)
+        for x in fbs + meshes:
+            x.free()
