@@ -255,9 +255,8 @@ def make_draw(prims, verts, shd, uniform, to_screen, keep: list) -> _ffi.RfDraw:
         keep.append(a)
     m = np.ascontiguousarray(uniform, dtype=np.float32).reshape(16)
     v = np.ascontiguousarray(to_screen, dtype=np.float32).reshape(16)
-    for i in range(16):
-        d.mvp[i] = m[i]
-        d.viewport[i] = v[i]
+    d.mvp[:] = m.tolist()
+    d.viewport[:] = v.tolist()
     if shd.kind == 0:
         for i in range(4):
             d.flat_color[i] = shd.color[i]

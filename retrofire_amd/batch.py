@@ -102,9 +102,8 @@ def mesh_draw(mesh: Mesh, shd, mvp, viewport, first_tri=0, n_tris=0, texture: Te
     d.kind = shd.kind
     m = np.ascontiguousarray(mvp, np.float32).reshape(16)
     v = np.ascontiguousarray(viewport, np.float32).reshape(16)
-    for i in range(16):
-        d.mvp[i] = m[i]
-        d.viewport[i] = v[i]
+    d.mvp[:] = m.tolist()
+    d.viewport[:] = v.tolist()
     if shd.kind == 0:
         for i in range(4):
             d.flat_color[i] = shd.color[i]

@@ -48,6 +48,23 @@ void DevBuf::release(uint64_t* counter) {
     cap = 0;
 }
 
+bool PinBuf::ensure(size_t bytes) {
+    if (bytes <= cap) return true;
+    release();
+    const size_t want = (bytes + bytes / 4 + 4095) & ~size_t(4095);
+    if (hipHostMalloc((void**)&p, want, 0)) {
+        p = nullptr;
+        return false;
+    }
+    cap = want;
+    return true;
+}
+void PinBuf::release() {
+    if (p) (void)hipHostFree(p);
+    p = nullptr;
+    cap = 0;
+}
+
 uint32_t bytes_per_pixel(uint32_t fmt) { return pixfmt_bytes(fmt); }
 
 uint32_t pack_clear(uint32_t fmt, const uint8_t* c) { return pack_pixel(fmt, c[0], c[1], c[2], c[3]); }
@@ -105,6 +122,7 @@ static void scratch_arrays(BatchDesc& B, Fn&& fn) {
     const uint64_t ntl = std::max<uint64_t>(B.n_tiles, 1), nf = std::max<uint64_t>(B.n_frames, 1);
     void* misc = nullptr;
     fn(MISC_BYTES, &misc);
+    fn(nf * sizeof(FrameStats), (void**)&B.stats);  // right behind: report_bytes
     fn(nv * 6 * sizeof(float), (void**)&B.sv);
     fn(nt * sizeof(uint32_t), (void**)&B.hdr);
     fn(nt * sizeof(ScrTri), (void**)&B.scr);
@@ -120,7 +138,6 @@ static void scratch_arrays(BatchDesc& B, Fn&& fn) {
     fn(ntl * sizeof(uint32_t), (void**)&B.long_list);
     fn(ntl * sizeof(uint32_t), (void**)&B.heavy_list);
     fn(std::max<uint64_t>(B.runs_cap, 1) * sizeof(Run), (void**)&B.runs);
-    fn(nf * sizeof(FrameStats), (void**)&B.stats);
     fn(std::max<uint64_t>(B.n_draws, 1) * sizeof(uint32_t), (void**)&B.draw_vis);
     fn(nf * PRIM_PARTS * PRIM_PART_STRIDE * 8, (void**)&B.prims_part);
     uint32_t* m = (uint32_t*)misc;
@@ -182,19 +199,14 @@ rf_status run_sized(Device& d, Scratch& sc, BatchDesc& B, hipStream_t s,
         if (sc.prepare(B, counter) != hipSuccess) return RF_E_DEVICE;
         if (pre && pre(B) != hipSuccess) return RF_E_DEVICE;
         if (launch_pipeline(B, s, raster_grid(d, B)) != hipSuccess) return RF_E_DEVICE;
-        uint32_t misc[3];
-        uint32_t total_runs = 0;
-        if (hipMemcpyAsync(misc, misc_words(B), sizeof(misc), hipMemcpyDeviceToHost, s) != hipSuccess)
+        std::vector<uint8_t> rep(report_bytes(B.n_frames));
+        if (hipMemcpyAsync(rep.data(), misc_words(B), rep.size(), hipMemcpyDeviceToHost, s) != hipSuccess ||
+            hipStreamSynchronize(s) != hipSuccess)
             return RF_E_DEVICE;
-        if (hipMemcpyAsync(&total_runs, B.run_off + B.n_tiles, 4, hipMemcpyDeviceToHost, s) !=
-            hipSuccess)
-            return RF_E_DEVICE;
+        uint32_t misc[RUNS_WORD + 1];
+        std::memcpy(misc, rep.data(), sizeof(misc));
         stats_out.resize(B.n_frames);
-        if (B.n_frames &&
-            hipMemcpyAsync(stats_out.data(), B.stats, B.n_frames * sizeof(FrameStats),
-                           hipMemcpyDeviceToHost, s) != hipSuccess)
-            return RF_E_DEVICE;
-        if (hipStreamSynchronize(s) != hipSuccess) return RF_E_DEVICE;
+        std::memcpy(stats_out.data(), rep.data() + STATS_OFF, B.n_frames * sizeof(FrameStats));
         const uint32_t err = misc[2];
         bool again = false;
         if (err & ERRB_EXTRA) {
@@ -205,7 +217,7 @@ rf_status run_sized(Device& d, Scratch& sc, BatchDesc& B, hipStream_t s,
         }
         if (err & ERRB_RUNS) {
             if (B.runs_cap >= 0xFFFFFF00u) return RF_E_UNSUPPORTED;
-            B.runs_cap = grow_runs_cap(total_runs);
+            B.runs_cap = grow_runs_cap(misc[RUNS_WORD]);
             again = true;
         }
         if (!again) {
@@ -219,6 +231,12 @@ rf_status run_sized(Device& d, Scratch& sc, BatchDesc& B, hipStream_t s,
 
 
 // ---- the plain path's pieces, shared by rf_render and rf_render_noalloc ----
+
+// Largest target read back, and largest upload, through pinned memory.
+constexpr size_t STAGE_DOWN_MAX = 256ull << 20, STAGE_UP_MAX = 128ull << 20;
+static size_t up256(size_t x) { return (x + 255) & ~size_t(255); }
+
+static void copy(const CopyRows& c) { copy_rows(c, 0, c.rows); }
 
 rf_status plain_check(const rf_draw* draw, const rf_target* target, const rf_ctx* ctx) {
     rf_status st = check_ctx(ctx);
@@ -265,6 +283,15 @@ PlainLayout plain_layout(const rf_draw* draw, const rf_target* target) {
     return L;
 }
 
+PlainLayout plain_layout_packed(const rf_draw* draw, const rf_target* target) {
+    PlainLayout L = plain_layout(draw, target);
+    L.col_pitch = (L.col_row + 15) & ~size_t(15);
+    L.col_b = L.col_pitch * target->height;
+    L.dep_pitch_f = (target->width + 3) & ~3u;
+    L.dep_b = target->depth ? L.dep_pitch_f * 4 * target->height : 0;
+    return L;
+}
+
 hipError_t plain_upload_inputs(const rf_draw* draw, const PlainLayout& L, const PlainBufs& P, hipStream_t s) {
     hipError_t e = hipSuccess;
     if (L.pos_b) e = hipMemcpyAsync(P.pos, draw->pos, L.pos_b, hipMemcpyHostToDevice, s);
@@ -281,55 +308,6 @@ hipError_t plain_upload_target(const rf_target* target, const rf_ctx* ctx, const
     if (!e && target->depth && !ctx->clear_depth)
         e = hipMemcpyAsync(P.depth, target->depth, L.dep_b, hipMemcpyHostToDevice, s);
     return e;
-}
-
-// Largest view read-back staged through pinned memory (colour and depth).
-constexpr size_t STAGE_MAX = 256ull << 20;
-
-hipError_t plain_download_sync(Device& d, const rf_target* target, const PlainLayout& L, const PlainBufs& P,
-                               hipStream_t s) {
-    const bool col_view = L.col_pitch != L.col_row;
-    const bool dep_view = target->depth && L.dep_pitch_f * 4 != L.dep_row;
-    const uint32_t h = target->height;
-    const size_t cb = col_view ? (size_t)h * L.col_row : 0, db = dep_view ? (size_t)h * L.dep_row : 0;
-    // Packed rows go straight into the caller's memory in one copy. A view's
-    // rows would be a 2D copy into pageable memory, which the runtime stages
-    // row by row (about 10x slower at 2048x2048); into pinned memory it is one
-    // DMA transfer, so they come into d.stage and then move on the host,
-    // writing only the view's bytes.
-    bool staged = (col_view || dep_view) && cb + db <= STAGE_MAX;
-    if (staged && cb + db > d.stage_cap) {
-        if (d.stage) (void)hipHostFree(d.stage);
-        d.stage = nullptr;
-        d.stage_cap = 0;
-        if (hipHostMalloc((void**)&d.stage, cb + db, 0)) {
-            d.stage = nullptr;
-            staged = false;
-        } else {
-            d.stage_cap = cb + db;
-        }
-    }
-    if (!staged) {
-        const hipError_t e = plain_download(target, L, P, s);
-        return e ? e : hipStreamSynchronize(s);
-    }
-    hipError_t e = col_view ? hipMemcpy2DAsync(d.stage, L.col_row, P.color, L.col_pitch, L.col_row, h,
-                                               hipMemcpyDeviceToHost, s)
-                            : hipMemcpyAsync(target->color, P.color, L.col_b, hipMemcpyDeviceToHost, s);
-    if (!e && target->depth)
-        e = dep_view ? hipMemcpy2DAsync(d.stage + cb, L.dep_row, P.depth, L.dep_pitch_f * 4, L.dep_row, h,
-                                        hipMemcpyDeviceToHost, s)
-                     : hipMemcpyAsync(target->depth, P.depth, L.dep_b, hipMemcpyDeviceToHost, s);
-    if (!e) e = hipStreamSynchronize(s);
-    if (e) return e;
-    uint8_t* const col = static_cast<uint8_t*>(target->color);
-    uint8_t* const dep = reinterpret_cast<uint8_t*>(target->depth);
-    for (uint32_t y = 0; y < h; ++y) {
-        if (col_view) std::memcpy(col + (size_t)y * L.col_pitch, d.stage + (size_t)y * L.col_row, L.col_row);
-        if (dep_view)
-            std::memcpy(dep + (size_t)y * L.dep_pitch_f * 4, d.stage + cb + (size_t)y * L.dep_row, L.dep_row);
-    }
-    return hipSuccess;
 }
 
 hipError_t plain_download(const rf_target* target, const PlainLayout& L, const PlainBufs& P, hipStream_t s) {
@@ -463,10 +441,11 @@ rf_status rf_device_close(rf_device* dev) {
     (void)hipStreamSynchronize(d->stream);
     d->plain.release(&d->bytes);
     sortpass_release(d->ds, &d->bytes);
-    for (DevBuf* b : {&d->up_pos, &d->up_attr, &d->up_tris, &d->up_tex, &d->up_color, &d->up_depth,
-                      &d->up_desc})
-        b->release(&d->bytes);
-    if (d->stage) (void)hipHostFree(d->stage);
+    d->up.release(&d->bytes);
+    d->stage_up.release();
+    d->stage_down.release();
+    for (hipEvent_t e : d->down_ev)
+        if (e) (void)hipEventDestroy(e);
     (void)hipStreamDestroy(d->stream);
     delete d;
     return RF_OK;
@@ -505,29 +484,73 @@ rf_status rf_render(rf_device* dev, const rf_draw* draw, rf_target* target, cons
     if (st) return st;
     if (hipSetDevice(d.ordinal) != hipSuccess) return RF_E_DEVICE;
     hipStream_t s = d.stream;
-    const PlainLayout L = plain_layout(draw, target);
-
-    // uploads
-    if (d.up_pos.ensure(std::max<size_t>(L.pos_b, 4), &d.bytes) ||
-        d.up_attr.ensure(std::max<size_t>(L.attr_b, 4), &d.bytes) ||
-        d.up_tris.ensure(std::max<size_t>(L.tri_b, 4), &d.bytes) ||
-        d.up_tex.ensure(std::max<size_t>(L.tex_b, 4), &d.bytes) || d.up_color.ensure(L.col_b, &d.bytes) ||
-        d.up_depth.ensure(std::max<size_t>(L.dep_b, 4), &d.bytes) ||
-        d.up_desc.ensure(PLAIN_DESC_BYTES, &d.bytes))
-        return RF_E_DEVICE;
-    PlainBufs P{d.up_pos.p, d.up_attr.p, d.up_tris.p, d.up_tex.p, d.up_color.p, d.up_depth.p, d.up_desc.p};
-    if (plain_upload_inputs(draw, L, P, s)) return RF_E_DEVICE;
-    auto upload_target = [&]() -> hipError_t { return plain_upload_target(target, ctx, L, P, s); };
-    if (upload_target()) return RF_E_DEVICE;
+    // Copies from and to pageable memory are staged by the runtime, one after
+    // another, each a wait: a two-triangle call spent 0.15 of 0.22 ms on eleven
+    // of them, a 1920x1080 frame's read-back ran at 17 GB/s. So what goes up is
+    // collected in pinned memory and goes as one copy; what comes down (the
+    // counters and, on the chance that they report no error, the target) comes
+    // into pinned memory in parts, and each part goes on into the caller's while
+    // the next arrives. Inputs and targets beyond the limits
+    // go directly, as do all if no pinned memory can be had.
+    PlainLayout L = plain_layout_packed(draw, target);
+    bool staged = L.col_b + L.dep_b <= STAGE_DOWN_MAX && d.stage_down.ensure(STATS_OFF + 4096 + L.col_b + L.dep_b);
+    if (!staged) L = plain_layout(draw, target);
+    // the device block, in upload order
+    struct Part {
+        const void* src;
+        size_t off, bytes;
+    };
+    const size_t o_pos = up256(PLAIN_DESC_BYTES), o_attr = o_pos + up256(L.pos_b), o_tris = o_attr + up256(L.attr_b),
+                 o_tex = o_tris + up256(L.tri_b), o_col = o_tex + up256(L.tex_b), o_dep = o_col + up256(L.col_b),
+                 end = o_dep + up256(L.dep_b);
+    if (d.up.ensure(end, &d.bytes)) return RF_E_DEVICE;
+    uint8_t* const up = (uint8_t*)d.up.p;
+    PlainBufs P{up + o_pos, up + o_attr, up + o_tris, up + o_tex, up + o_col, up + o_dep, up};
 
     DrawDesc dd;
     FrameDesc fd;
     BatchDesc B;
     plain_descs(draw, target, ctx, L, P, d.plain_tile_w, d.plain_tile_h, d.plain_chunk, dd, fd, B);
     uint8_t* desc = (uint8_t*)P.desc;
-    if (hipMemcpyAsync(desc, &dd, sizeof(dd), hipMemcpyHostToDevice, s) ||
-        hipMemcpyAsync((void*)B.frames, &fd, sizeof(fd), hipMemcpyHostToDevice, s))
+    const size_t o_fd = (const uint8_t*)B.frames - up;
+    const bool up_col = !ctx->clear_color, up_dep = target->depth && !ctx->clear_depth;
+    const size_t in_end = o_col, up_end = up_dep ? end : up_col ? o_dep : in_end;
+    const bool staged_up = staged && up_end <= STAGE_UP_MAX && d.stage_up.ensure(up_end);
+    // the target's own content, where it is not cleared (again before a rerun)
+    auto upload_target = [&]() -> hipError_t {
+        if (!staged) return plain_upload_target(target, ctx, L, P, s);
+        hipError_t e = hipSuccess;
+        uint8_t* const h = d.stage_up.p;
+        if (up_col)
+            e = staged_up ? hipMemcpyAsync(P.color, h + o_col, L.col_b, hipMemcpyHostToDevice, s)
+                          : hipMemcpy2DAsync(P.color, L.col_pitch, target->color, target->color_stride, L.col_row,
+                                             target->height, hipMemcpyHostToDevice, s);
+        if (!e && up_dep)
+            e = staged_up ? hipMemcpyAsync(P.depth, h + o_dep, L.dep_b, hipMemcpyHostToDevice, s)
+                          : hipMemcpy2DAsync(P.depth, L.dep_pitch_f * 4, target->depth,
+                                             (size_t)target->depth_stride * 4, L.dep_row, target->height,
+                                             hipMemcpyHostToDevice, s);
+        return e;
+    };
+    if (staged_up) {
+        uint8_t* const h = d.stage_up.p;
+        std::memcpy(h, &dd, sizeof(dd));
+        std::memcpy(h + o_fd, &fd, sizeof(fd));
+        for (const Part& p : {Part{draw->pos, o_pos, L.pos_b}, Part{draw->attr, o_attr, L.attr_b},
+                              Part{draw->tris, o_tris, L.tri_b}, Part{draw->tex, o_tex, L.tex_b}})
+            if (p.bytes) std::memcpy(h + p.off, p.src, p.bytes);
+        if (hipMemcpyAsync(up, h, in_end, hipMemcpyHostToDevice, s)) return RF_E_DEVICE;
+        if (up_col)
+            copy({h + o_col, (const uint8_t*)target->color, L.col_pitch, target->color_stride, L.col_row,
+                    target->height});
+        if (up_dep)
+            copy({h + o_dep, (const uint8_t*)target->depth, L.dep_pitch_f * 4, (size_t)target->depth_stride * 4,
+                    L.dep_row, target->height});
+    } else if (plain_upload_inputs(draw, L, P, s) || hipMemcpyAsync(desc, &dd, sizeof(dd), hipMemcpyHostToDevice, s) ||
+               hipMemcpyAsync((void*)B.frames, &fd, sizeof(fd), hipMemcpyHostToDevice, s)) {
         return RF_E_DEVICE;
+    }
+    if (upload_target()) return RF_E_DEVICE;
     B.extra_cap = std::max<uint32_t>(d.plain_extra_cap, 1024u);
     B.runs_cap = std::max<uint32_t>(d.plain_runs_cap, 4 * B.n_groups + B.n_tiles + 1024);
 
@@ -568,16 +591,83 @@ rf_status rf_render(rf_device* dev, const rf_draw* draw, rf_target* target, cons
         };
     }
 
-    std::vector<FrameStats> fs;
-    uint32_t err = 0;
-    st = run_sized(d, d.plain, B, s, pre, fs, &err, upload_target, &d.bytes);
-    if (st) return st;
+    if (!staged) {
+        std::vector<FrameStats> fs;
+        uint32_t err = 0;
+        st = run_sized(d, d.plain, B, s, pre, fs, &err, upload_target, &d.bytes);
+        if (st) return st;
+        d.plain_extra_cap = std::max(d.plain_extra_cap, B.extra_cap);
+        d.plain_runs_cap = std::max(d.plain_runs_cap, B.runs_cap);
+        if ((st = map_err(err))) return st;
+        if (plain_download(target, L, P, s) || hipStreamSynchronize(s)) return RF_E_DEVICE;
+        plain_stats(stats, draw, fs[0], t0);
+        return RF_OK;
+    }
+    for (hipEvent_t& e : d.down_ev)
+        if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming)) return RF_E_DEVICE;
+    uint8_t* const down = d.stage_down.p;
+    uint8_t* const pix = down + up256(report_bytes(1));
+    const size_t span = o_dep + L.dep_b - o_col;  // colour, then depth, as on the device
+    // parts of whole 64 KiB, at least 1 MiB
+    const size_t part = std::max<size_t>(1 << 20, (span / DOWN_CHUNKS + 0x10000) & ~size_t(0xFFFF));
+    uint32_t misc[RUNS_WORD + 1];
+    for (int attempt = 0;; ++attempt) {
+        if (attempt == 4) return RF_E_INTERNAL;
+        if (d.plain.prepare(B, &d.bytes) || (pre && pre(B)) || launch_pipeline(B, s, raster_grid(d, B)) ||
+            hipMemcpyAsync(down, misc_words(B), report_bytes(1), hipMemcpyDeviceToHost, s) ||
+            hipEventRecord(d.down_ev[0], s))
+            return RF_E_DEVICE;
+        uint32_t n = 0;
+        for (size_t at = 0; at < span; at += part, ++n)
+            if (hipMemcpyAsync(pix + at, up + o_col + at, std::min(part, span - at), hipMemcpyDeviceToHost, s) ||
+                hipEventRecord(d.down_ev[1 + n], s))
+                return RF_E_DEVICE;
+        if (hipEventSynchronize(d.down_ev[0])) return RF_E_DEVICE;
+        std::memcpy(misc, down, sizeof(misc));
+        const uint32_t err = misc[2];
+        if (!(err & (ERRB_EXTRA | ERRB_RUNS))) {
+            if (err) {
+                if (hipStreamSynchronize(s)) return RF_E_DEVICE;  // the staging is free again
+                return map_err(err);
+            }
+            break;
+        }
+        if (hipStreamSynchronize(s)) return RF_E_DEVICE;
+        if (err & ERRB_EXTRA) {
+            // more clip fans than a launch can index: refused, not wrapped
+            if (B.extra_cap >= MAX_LAUNCH_PRIMS) return RF_E_UNSUPPORTED;
+            B.extra_cap = grow_extra_cap(misc[0]);
+        }
+        if (err & ERRB_RUNS) {
+            if (B.runs_cap >= 0xFFFFFF00u) return RF_E_UNSUPPORTED;
+            B.runs_cap = grow_runs_cap(misc[RUNS_WORD]);
+        }
+        if (upload_target()) return RF_E_DEVICE;  // the aborted run may have drawn into it
+    }
     d.plain_extra_cap = std::max(d.plain_extra_cap, B.extra_cap);
     d.plain_runs_cap = std::max(d.plain_runs_cap, B.runs_cap);
-    if ((st = map_err(err))) return st;
-
-    if (plain_download_sync(d, target, L, P, s)) return RF_E_DEVICE;
-    plain_stats(stats, draw, fs[0], t0);
+    // rows of colour, then of depth, as far as the parts have arrived
+    size_t col_done = 0, dep_done = 0;
+    const size_t h = target->height, dep_at = o_dep - o_col, dep_pitch = L.dep_pitch_f * 4;
+    uint32_t n = 0;
+    for (size_t at = 0; at < span; at += part, ++n) {
+        if (hipEventSynchronize(d.down_ev[1 + n])) return RF_E_DEVICE;
+        const size_t have = std::min(at + part, span);
+        const size_t col = std::min(have / L.col_pitch, h);
+        if (col > col_done)
+            copy({(uint8_t*)target->color + col_done * target->color_stride, pix + col_done * L.col_pitch,
+                    target->color_stride, L.col_pitch, L.col_row, col - col_done});
+        col_done = col;
+        if (!target->depth || have <= dep_at) continue;
+        const size_t dep = std::min((have - dep_at) / dep_pitch, h), dst = (size_t)target->depth_stride * 4;
+        if (dep > dep_done)
+            copy({(uint8_t*)target->depth + dep_done * dst, pix + dep_at + dep_done * dep_pitch, dst, dep_pitch,
+                    L.dep_row, dep - dep_done});
+        dep_done = dep;
+    }
+    FrameStats fs;
+    std::memcpy(&fs, down + STATS_OFF, sizeof(fs));
+    plain_stats(stats, draw, fs, t0);
     return RF_OK;
 }
 

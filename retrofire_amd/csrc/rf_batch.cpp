@@ -34,8 +34,10 @@ struct Batch {
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
-    FrameStats* h_stats = nullptr;  // pinned
-    uint32_t* h_misc = nullptr;     // pinned
+    uint8_t* h_report = nullptr;    // pinned: the launch's report (report_bytes), then the sort pass's error word
+    const FrameStats* stats() const { return reinterpret_cast<const FrameStats*>(h_report + STATS_OFF); }
+    uint32_t* sort_err() const { return reinterpret_cast<uint32_t*>(h_report + report_bytes((uint32_t)frames.size())); }
+    uint32_t err() const { return reinterpret_cast<const uint32_t*>(h_report)[2] | *sort_err(); }
     bool pending = false;
     std::vector<rf_tune_entry> tune;  // the autotuner's timings (tile width, height, chunk, ms)
     // depth sort: the triangle draws of frames whose context asks for it
@@ -217,8 +219,7 @@ static void batch_release(Batch* b) {
     b->d_desc.release(&d.bytes);
     if (b->ev0) (void)hipEventDestroy(b->ev0);
     if (b->ev1) (void)hipEventDestroy(b->ev1);
-    if (b->h_stats) (void)hipHostFree(b->h_stats);
-    if (b->h_misc) (void)hipHostFree(b->h_misc);
+    if (b->h_report) (void)hipHostFree(b->h_report);
     if (b->stream) (void)hipStreamDestroy(b->stream);
     delete b;
 }
@@ -262,12 +263,11 @@ rf_status rf_batch_create(rf_device* dev, const rf_frame* frames, uint32_t n_fra
     }
     rf_status st = RF_OK;
     if (hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking) || hipEventCreate(&b->ev0) ||
-        hipEventCreate(&b->ev1) || hipHostMalloc((void**)&b->h_stats, n_frames * sizeof(FrameStats), 0) ||
-        hipHostMalloc((void**)&b->h_misc, 64, 0)) {
+        hipEventCreate(&b->ev1) || hipHostMalloc((void**)&b->h_report, report_bytes(n_frames) + 64, 0)) {
         batch_release(b);
         return RF_E_DEVICE;
     }
-    std::memset(b->h_misc, 0, 64);
+    std::memset(b->h_report, 0, report_bytes(n_frames) + 64);
     // Depth sort (render.rs:180-183): the triangle draws of frames that ask
     // for it go through the sort pass; its planning run gives their fan counts.
     for (uint32_t i = 0; i < n_frames; ++i)
@@ -349,13 +349,11 @@ rf_status rf_batch_run(rf_batch* bh, int sync) {
     if (hipSetDevice(b.dev->ordinal)) return RF_E_DEVICE;
     if (hipEventRecord(b.ev0, b.stream) || hipGraphLaunch(b.exec, b.stream) || hipEventRecord(b.ev1, b.stream))
         return RF_E_DEVICE;
-    if (hipMemcpyAsync(b.h_stats, b.B.stats, b.B.n_frames * sizeof(FrameStats), hipMemcpyDeviceToHost,
-                       b.stream) ||
-        hipMemcpyAsync(b.h_misc, misc_words(b.B), 16, hipMemcpyDeviceToHost, b.stream))
+    if (hipMemcpyAsync(b.h_report, misc_words(b.B), report_bytes(b.B.n_frames), hipMemcpyDeviceToHost, b.stream))
         return RF_E_DEVICE;
     // the sort pass's error bits (its own counters)
     if (!b.sp.draws.empty() &&
-        hipMemcpyAsync(b.h_misc + 8, misc_words(b.sp.P) + 2, 4, hipMemcpyDeviceToHost, b.stream))
+        hipMemcpyAsync(b.sort_err(), misc_words(b.sp.P) + 2, 4, hipMemcpyDeviceToHost, b.stream))
         return RF_E_DEVICE;
     b.pending = true;
     if (sync) return rf_batch_wait(bh, nullptr);
@@ -367,23 +365,23 @@ rf_status rf_batch_wait(rf_batch* bh, rf_stats* stats) {
     Batch& b = *reinterpret_cast<Batch*>(bh);
     if (hipStreamSynchronize(b.stream)) return RF_E_DEVICE;
     b.pending = false;
-    rf_status st = map_err(b.h_misc[2] | b.h_misc[8]);
+    rf_status st = map_err(b.err());
     if (st) return st;
     if (stats) {
         float ms = 0.0f;
         (void)hipEventElapsedTime(&ms, b.ev0, b.ev1);
         for (uint32_t i = 0; i < b.B.n_frames; ++i) {
             rf_stats& s = stats[i];
-            const FrameStats& h = b.h_stats[i];
+            const FrameStats& h = b.stats()[i];
             s.calls = b.frame_calls[i] - h.hidden_draws;
             s.prims_i = b.frame_prims_i[i] - h.hidden_prims;
             s.verts_i = b.frame_verts_i[i] - h.hidden_verts;
             s.objs_i = b.frame_objs[i];
             s.objs_o = b.frame_objs[i] - h.hidden_draws;
-            s.prims_o = b.h_stats[i].prims_o;
-            s.verts_o = b.h_stats[i].verts_o;
-            s.frags_i = b.h_stats[i].frags_i;
-            s.frags_o = b.h_stats[i].frags_o;
+            s.prims_o = h.prims_o;
+            s.verts_o = h.verts_o;
+            s.frags_i = h.frags_i;
+            s.frags_o = h.frags_o;
             s.seconds = ms * 1e-3;
         }
     }

@@ -3,8 +3,13 @@
 
 #include <hip/hip_runtime.h>
 
+#include <atomic>
+#include <condition_variable>
 #include <cstdint>
 #include <functional>
+#include <memory>
+#include <mutex>
+#include <thread>
 #include <vector>
 
 #include "../../include/retrofire_amd.h"
@@ -24,6 +29,7 @@ constexpr uint64_t MAX_LAUNCH_PRIMS = 1ull << 29;
 // Clip-fan and bin-run capacities grown by a rerun that needs more.
 uint32_t grow_extra_cap(uint32_t needed);
 uint32_t grow_runs_cap(uint32_t needed);
+constexpr uint32_t DOWN_CHUNKS = 12;  // parts of a read-back that are copied on while others arrive
 constexpr uint32_t DEFAULT_TILE_H = 32;  // rasterizer tile height of rf_render and served launches
 inline bool valid_tile_h(uint32_t th) { return th == 16 || th == 32 || th == 64; }
 
@@ -46,6 +52,12 @@ constexpr uint64_t MISC_BYTES = 512 + 4 * N_TILE_COUNTERS * TC_STRIDE;
 uint64_t scratch_bytes(const BatchDesc& B);
 void scratch_carve(BatchDesc& B, uint8_t* base);
 inline uint32_t* misc_words(const BatchDesc& B) { return B.extra_count; }
+// What a launch reports, in one copy from misc_words(B): the counters (word 0
+// the clip fans beyond the first, 2 the error bits, RUNS_WORD the bin runs) and,
+// from STATS_OFF, the frames' FrameStats.
+constexpr uint32_t RUNS_WORD = 3;
+constexpr uint64_t STATS_OFF = (MISC_BYTES + 255) & ~uint64_t(255);
+inline uint64_t report_bytes(uint32_t n_frames) { return STATS_OFF + n_frames * sizeof(FrameStats); }
 
 // A grow-only block holding a batch's scratch.
 struct Scratch {
@@ -79,13 +91,51 @@ struct SortPass {
 };
 
 
+// Rows of memory to copy.
+struct CopyRows {
+    uint8_t* dst;
+    const uint8_t* src;
+    size_t dst_pitch, src_pitch, row, rows;
+};
+void copy_rows(const CopyRows& c, size_t r0, size_t r1);  // rows [r0, r1)
+// A few threads that copy rows together with their caller (rf_copy.cpp). One
+// copy at a time: a second caller's is made by itself. Joined on destruction.
+class CopyPool {
+public:
+    CopyPool();
+    ~CopyPool();
+    void run(const CopyRows& c);
+
+private:
+    void worker();
+    void work();
+    std::vector<std::thread> threads;
+    std::mutex user;  // held by the caller whose copy it is
+    std::mutex m;     // guards job .. open
+    std::condition_variable cv;
+    CopyRows job{};
+    size_t rows_per_piece = 0, pieces = 0;
+    bool open = false, stop = false;
+    std::atomic<uint64_t> epoch{0};
+    std::atomic<size_t> next{0};
+    std::atomic<int> inside{0};  // threads at work on the job
+};
+
+// Pinned host memory, grow-only.
+struct PinBuf {
+    uint8_t* p = nullptr;
+    size_t cap = 0;
+    bool ensure(size_t bytes);  // false: none to be had (the old block is gone)
+    void release();
+};
+
 struct Device {
     int ordinal = 0;
     int num_cu = 256;
     hipStream_t stream = nullptr;
     uint64_t bytes = 0;  // device memory held
     Scratch plain;
-    DevBuf up_pos, up_attr, up_tris, up_tex, up_color, up_depth, up_desc;
+    DevBuf up;  // rf_render's descriptors, inputs and target
     SortPass ds;  // rf_render's depth sort
     uint32_t plain_tile_w = 32;  // rasterizer tile width of rf_render
     uint32_t plain_tile_h = DEFAULT_TILE_H;  // and its tile height
@@ -94,9 +144,10 @@ struct Device {
     // rf_render_noalloc's static device array on this GPU (from
     // hipGetSymbolAddress at rf_device_open; null if that failed)
     uint8_t* noalloc = nullptr;
-    // pinned host staging of rf_render's read-back into a view (grow-only)
-    uint8_t* stage = nullptr;
-    size_t stage_cap = 0;
+    // rf_render's pinned staging: descriptors, inputs and an uncleared target on
+    // their way up; counters, colour and depth on their way down
+    PinBuf stage_up, stage_down;
+    hipEvent_t down_ev[DOWN_CHUNKS + 1] = {};  // the counters', then a chunk's each
 };
 // Looks up the device address of rf_render_noalloc's array on the current
 // device (rf_noalloc.cpp).
@@ -145,8 +196,8 @@ rf_status run_sized(Device& d, Scratch& sc, BatchDesc& B, hipStream_t s,
 
 // The plain path (one render() call with host buffers): argument checks,
 // the device layout of its inputs and target, the host<->device copies, the
-// descriptors and the stats. rf_render keeps the buffers in grow-only device
-// allocations; rf_render_noalloc carves them from a fixed static array.
+// descriptors and the stats. rf_render keeps the buffers in a grow-only device
+// allocation; rf_render_noalloc carves them from a fixed static array.
 struct PlainLayout {
     int na = 0;          // attribute floats per vertex
     bool textured = false;
@@ -160,15 +211,12 @@ struct PlainBufs {
 constexpr size_t PLAIN_DESC_BYTES = 256 * ((sizeof(DrawDesc) + 255) / 256) + 256 * ((sizeof(FrameDesc) + 255) / 256);
 rf_status plain_check(const rf_draw* draw, const rf_target* target, const rf_ctx* ctx);
 PlainLayout plain_layout(const rf_draw* draw, const rf_target* target);
+// The same with the target's rows packed on the device, 16-byte aligned.
+PlainLayout plain_layout_packed(const rf_draw* draw, const rf_target* target);
 hipError_t plain_upload_inputs(const rf_draw* draw, const PlainLayout& L, const PlainBufs& P, hipStream_t s);
 hipError_t plain_upload_target(const rf_target* target, const rf_ctx* ctx, const PlainLayout& L, const PlainBufs& P,
                                hipStream_t s);
 hipError_t plain_download(const rf_target* target, const PlainLayout& L, const PlainBufs& P, hipStream_t s);
-// rf_render's read-back, synchronous: packed rows straight into the target;
-// a view's rows by one DMA transfer into d.stage (pinned, up to 256 MiB), then
-// on the host into the view (larger views, or no pinned memory: a 2D copy).
-hipError_t plain_download_sync(Device& d, const rf_target* target, const PlainLayout& L, const PlainBufs& P,
-                               hipStream_t s);
 void plain_descs(const rf_draw* draw, const rf_target* target, const rf_ctx* ctx, const PlainLayout& L,
                  const PlainBufs& P, uint32_t tile_w, uint32_t tile_h, uint32_t chunk, DrawDesc& dd, FrameDesc& fd,
                  BatchDesc& B);

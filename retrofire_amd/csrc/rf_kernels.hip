@@ -955,6 +955,7 @@ __device__ __forceinline__ void scan_totals(const BatchDesc& B, uint32_t runs, u
     }
     if (threadIdx.x == 0) {
         B.run_off[B.n_tiles] = runs;
+        B.extra_count[RUNS_WORD] = runs;
         B.tile_counts[TN_BUSY] = busy;
         B.tile_counts[TN_HEAVY_MIN] = h.heavy;
         if (runs > B.runs_cap) atomicOr(B.err, ERRB_RUNS);

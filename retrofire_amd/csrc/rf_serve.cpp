@@ -209,6 +209,7 @@ struct Serve {
     std::mutex pm;  // guards `pin`; never held across a HIP call (taken after `m`)
     void* pin_mem = nullptr;
     Arena pin;      // read-back buffers in the pinned block
+    std::unique_ptr<CopyPool> pool;  // copies results to the callers of rf_serve_poll
     uint64_t sort_bytes = 0;  // device memory of the lanes' depth-sort buffers (worker thread only)
 };
 
@@ -806,6 +807,7 @@ rf_status rf_serve_open(rf_device* dev, uint64_t budget_bytes, uint32_t max_batc
         return RF_E_DEVICE;
     }
     s->pin.init((uint8_t*)s->pin_mem, pin_bytes);
+    s->pool.reset(new (std::nothrow) CopyPool());
     const size_t stage = 2 * (align_up((size_t)max_batch * STAGE_DRAWS * sizeof(DrawDesc)) +
                               align_up((size_t)max_batch * sizeof(FrameDesc)));
     for (uint32_t i = 0; i < n_streams; ++i) {
@@ -868,19 +870,30 @@ rf_status rf_serve_poll(rf_serve* sh, rf_result* out, void** color, uint32_t max
     std::unique_lock<std::mutex> lk(s.m);
     if (s.done.empty() && timeout_ms)
         s.cv_done.wait_for(lk, std::chrono::milliseconds(timeout_ms), [&] { return !s.done.empty(); });
-    uint32_t n = 0;
-    while (n < max && !s.done.empty()) {
-        Done d = s.done.front();
+    std::vector<Done> got;
+    while (got.size() < max && !s.done.empty()) {
+        got.push_back(s.done.front());
         s.done.pop_front();
-        out[n] = d.res;
-        if (d.pixels) {
-            if (color && color[n]) std::memcpy(color[n], d.pixels, d.pix_bytes);
-            pin_put(s, d.pixels, d.pix_bytes);
+    }
+    lk.unlock();
+    // The pixels are copied without the lock (the worker admits and the waiters
+    // report meanwhile) and by several threads: one copies at about 20 GB/s, and
+    // a burst's frames come down the link at 57.
+    const uint32_t n = (uint32_t)got.size();
+    for (uint32_t i = 0; i < n; ++i) {
+        const Done& d = got[i];
+        out[i] = d.res;
+        if (!d.pixels) continue;
+        if (color && color[i]) {
+            uint8_t* const to = (uint8_t*)color[i];
+            const size_t rows = d.pix_bytes / 4096, rest = d.pix_bytes % 4096;
+            if (s.pool) s.pool->run({to, d.pixels, 4096, 4096, 4096, rows});
+            else std::memcpy(to, d.pixels, rows * 4096);
+            std::memcpy(to + rows * 4096, d.pixels + rows * 4096, rest);
         }
-        ++n;
+        pin_put(s, d.pixels, d.pix_bytes);
     }
     *n_out = n;
-    lk.unlock();
     if (n) s.cv_work.notify_all();  // admissions may wait for read-back space
     return RF_OK;
 }

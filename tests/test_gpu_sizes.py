@@ -168,3 +168,36 @@ def test_tile_counts_around_the_scan_kernels(frames):
         dev.set_tile_height(0)
         for x in fbs + meshes:
             x.free()
+
+
+@pytest.mark.parametrize("w,h", [(1, 1), (3, 700), (255, 257), (512, 512), (513, 511), (1031, 997)])
+@pytest.mark.parametrize("fmt", [rf.PIX_RGBA8, rf.PIX_RGB8, rf.PIX_RGB565])
+@pytest.mark.parametrize("pad,clear,depth", [(0, True, True), (0, False, True), (7, False, True), (7, True, False)])
+def test_plain_calls_into_targets_of_every_size(w, h, fmt, pad, clear, depth):
+    """rf_render's staged copies: packed targets and views, cleared and drawn
+    over, smaller than one part of the read-back and of several; the parent's
+    bytes around a view stay as they are."""
+    rng = np.random.default_rng([w, h, fmt, pad])
+    shape = (h + pad, w + pad) + ({0: (4,), 1: (3,)}.get(fmt, ()))
+    col = rng.integers(0, 250, size=shape).astype(np.uint16 if fmt == rf.PIX_RGB565 else np.uint8)
+    dep = rng.uniform(0.0, 0.2, size=(h + pad, w + pad)).astype(np.float32)
+    gcol, gdep = col.copy(), dep.copy()
+    cut = (slice(pad // 2, pad // 2 + h), slice(pad // 2, pad // 2 + w))
+    ocol, odep = np.ascontiguousarray(col[cut]), np.ascontiguousarray(dep[cut])
+    if clear:
+        ocol[...] = 0 if fmt == rf.PIX_RGB565 else np.array([0, 0, 0, 255][:ocol.shape[2]], np.uint8)
+        odep[...] = 0.0
+    pos, attr, tris, mvp, vp = random_soup(rng, 40, w, h, 1)
+    ost = np.zeros(8, np.uint64)
+    err, _ = O.render(1, tris, pos, attr, mvp, vp, ocol, depth=odep if depth else None, fmt=fmt, ctx=(1, 0, 1, 1, 0),
+                      stats=ost)
+    assert err == 0
+    ctx = rf.Context(clear=clear, face_cull=None)
+    target = rf.Framebuf(gcol[cut], gdep[cut], fmt) if depth else rf.Colorbuf(gcol[cut], fmt)
+    rf.render(tris, (pos, attr), rf.shader.Gouraud(), mvp, vp, target, ctx)
+    assert np.array_equal(gcol[cut], ocol)
+    assert [ctx.stats.prims_o, ctx.stats.frags_i, ctx.stats.frags_o] == [int(ost[2]), int(ost[5]), int(ost[6])]
+    if depth:
+        assert np.array_equal(gdep[cut].view(np.uint32), odep.view(np.uint32))
+    gcol[cut], gdep[cut] = col[cut], dep[cut]
+    assert np.array_equal(gcol, col) and np.array_equal(gdep, dep)
