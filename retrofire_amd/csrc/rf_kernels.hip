@@ -2494,32 +2494,53 @@ __global__ __launch_bounds__(256) void k_fan_gather(BatchDesc P, BatchDesc M, co
 // (clip.rs:245-267) — all corners outside one same plane. What the skipped
 // render() call would have counted is added to the frame's hidden totals.
 // ---------------------------------------------------------------------------
+// Bound by those totals when every hidden draw adds its own (4 frames of 1,000
+// draws: 54 us): a wave whose hidden draws are of one frame adds once.
 __global__ __launch_bounds__(256) void k_cull(BatchDesc B) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= B.n_draws) return;
-    const DrawDesc* D = &B.draws[i];
-    uint32_t vis = 1;
-    if (D->cull) {
-        const float* m = D->mvp;
-        uint32_t all_out = ~0u;
-        for (int c = 0; c < 8; ++c) {
-            const float px = D->bbox[(c & 4) ? 3 : 0], py = D->bbox[(c & 2) ? 4 : 1], pz = D->bbox[(c & 1) ? 5 : 2];
-            const float x = dot4(m + 0, px, py, pz, 1.0f);
-            const float y = dot4(m + 4, px, py, pz, 1.0f);
-            const float z = dot4(m + 8, px, py, pz, 1.0f);
-            const float w = dot4(m + 12, px, py, pz, 1.0f);
-            all_out &= outcode(x, y, z, w);
+    bool hidden = false;
+    uint32_t frame = 0;
+    unsigned long long prims = 0, verts = 0;
+    if (i < B.n_draws) {
+        const DrawDesc* D = &B.draws[i];
+        if (D->cull) {
+            const float* m = D->mvp;
+            uint32_t all_out = ~0u;
+            for (int c = 0; c < 8; ++c) {
+                const float px = D->bbox[(c & 4) ? 3 : 0], py = D->bbox[(c & 2) ? 4 : 1], pz = D->bbox[(c & 1) ? 5 : 2];
+                const float x = dot4(m + 0, px, py, pz, 1.0f);
+                const float y = dot4(m + 4, px, py, pz, 1.0f);
+                const float z = dot4(m + 8, px, py, pz, 1.0f);
+                const float w = dot4(m + 12, px, py, pz, 1.0f);
+                all_out &= outcode(x, y, z, w);
+            }
+            if (all_out != 0) {
+                hidden = true;
+                frame = D->frame;
+                // a depth-sorted draw holds its fans: its render() call's own counts
+                prims = D->pre ? D->in_tris : D->n_tris;
+                verts = D->pre ? D->in_verts : D->n_verts;
+            }
         }
-        if (all_out != 0) {
-            vis = 0;
-            FrameStats& st = B.stats[D->frame];
-            atomicAdd(&st.hidden_draws, 1ull);
-            // a depth-sorted draw holds its fans: its render() call's own counts
-            atomicAdd(&st.hidden_prims, (unsigned long long)(D->pre ? D->in_tris : D->n_tris));
-            atomicAdd(&st.hidden_verts, (unsigned long long)(D->pre ? D->in_verts : D->n_verts));
-        }
+        B.draw_vis[i] = hidden ? 0u : 1u;
     }
-    B.draw_vis[i] = vis;
+    const uint32_t f0 = wave_min_u32(hidden ? frame : 0xFFFFFFFFu), f1 = ~wave_min_u32(hidden ? ~frame : 0xFFFFFFFFu);
+    if (f0 == f1) {
+        const uint32_t n = (uint32_t)__popcll(__ballot(hidden));
+        prims = wave_sum_u64(prims);
+        verts = wave_sum_u64(verts);
+        if (lane_id() == 0) {
+            FrameStats& st = B.stats[f0];
+            atomicAdd(&st.hidden_draws, (unsigned long long)n);
+            atomicAdd(&st.hidden_prims, prims);
+            atomicAdd(&st.hidden_verts, verts);
+        }
+    } else if (hidden) {
+        FrameStats& st = B.stats[frame];
+        atomicAdd(&st.hidden_draws, 1ull);
+        atomicAdd(&st.hidden_prims, prims);
+        atomicAdd(&st.hidden_verts, verts);
+    }
 }
 
 // Zeroes per-batch counters (a kernel, so it can live inside a captured graph).

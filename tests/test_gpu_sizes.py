@@ -201,3 +201,42 @@ def test_plain_calls_into_targets_of_every_size(w, h, fmt, pad, clear, depth):
         assert np.array_equal(gdep[cut].view(np.uint32), odep.view(np.uint32))
     gcol[cut], gdep[cut] = col[cut], dep[cut]
     assert np.array_equal(gcol, col) and np.array_equal(gdep, dep)
+
+
+@pytest.mark.parametrize("counts", [(1, 2), (63, 1, 64), (65, 130), (300, 5)])
+def test_culled_draws_of_several_frames_in_a_wave(counts):
+    """Frames of `counts` draws, half of them hidden whole by their bounding
+    boxes: the hidden calls, primitives and vertices are each frame's own."""
+    rng = np.random.default_rng(counts)
+    pos = rng.uniform(-0.2, 0.2, size=(30, 3)).astype(np.float32)
+    tris = np.arange(30, dtype=np.uint32).reshape(10, 3)
+    m = RB.Mesh(pos, tris)
+    vp, proj = M.viewport(0, 48, 64, 0), M.perspective(1.2, np.float32(64 / 48), 0.1, 8.0)
+    frames, want = [], []
+    for n in counts:
+        draws, ocol, ost = [], np.zeros((48, 64, 4), np.uint8), np.zeros(8, np.uint64)
+        ocol[...] = (0, 0, 0, 255)
+        hidden = 0
+        for k in range(n):
+            x = 40.0 if rng.random() < 0.5 else float(rng.uniform(-0.5, 0.5))
+            mvp = M.then(M.translate3(x, 0.0, 2.0), proj)
+            draws.append(RB.mesh_draw(m, rf.shader.Flat((k % 256, 9, 200, 255)), mvp, vp, cull=True))
+            if O.bbox_visibility(O.bbox_of(pos), mvp) == O.HIDDEN:
+                hidden += 1
+                continue
+            err, _ = O.render(0, tris, pos, None, mvp, vp, ocol, flat=(k % 256, 9, 200, 255), ctx=(0, 0, 1, 1, 0),
+                              stats=ost)
+            assert err == 0
+        frames.append((RB.DeviceFramebuf(64, 48, 0, False), rf.Context(clear=True, face_cull=None), draws))
+        want.append((ocol, [n, n - hidden] + [int(x) for x in ost[:7]]))
+    b = RB.Batch(frames, tile_w=32)
+    for _ in range(2):
+        b.run()
+        for s, (fb, _, _), (ocol, counts_) in zip(b.wait(), frames, want):
+            assert np.array_equal(fb.read()[0], ocol)
+            assert [s.objs_i, s.objs_o, s.calls, s.prims_i, s.prims_o, s.verts_i, s.verts_o, s.frags_i,
+                    s.frags_o] == counts_
+    b.free()
+    m.free()
+    for fb, _, _ in frames:
+        fb.free()
