@@ -145,6 +145,10 @@ struct Run {
     unsigned long long mask;
 };
 
+// Runs of a group that k_setup keeps for k_bin; a group of more is walked again.
+constexpr uint32_t PRE_RUNS = 32;
+constexpr uint32_t RUNS_MULTI = 1u << 31;  // n_runs bit: Run::multi
+
 // A tile as the rasterizer takes it: all it needs to start, in one load.
 struct alignas(16) TileRec {
     uint32_t tile, frame, off, nruns;  // its runs are runs[off .. off + nruns)
@@ -194,6 +198,9 @@ struct BatchDesc {
     uint32_t extra_cap;
     uint32_t* rect;      // per triangle: pixel rect (c0 | r0 << 16, c1 | r1 << 16; all ones: none), 2 words
     float* zmax;         // per triangle: no fragment's z is above it (+inf: not known)
+    uint32_t* tile_of;   // per group, PRE_RUNS: its runs' tiles, and
+    unsigned long long* mask_of;  // masks, as k_setup has met them
+    uint32_t* n_runs;    // per group: their number | RUNS_MULTI
     uint32_t* run_count; // per tile (run_slot)
     uint32_t* run_off;   // per tile + 1 (exclusive scan)
     uint32_t* run_cursor;  // per tile (run_slot): where its next run goes

@@ -240,3 +240,13 @@ def test_culled_draws_of_several_frames_in_a_wave(counts):
     m.free()
     for fb, _, _ in frames:
         fb.free()
+
+
+@pytest.mark.parametrize("n", [1, 31, 32, 33, 63, 64, 65, 130])
+@pytest.mark.parametrize("draws", [1, 3])
+def test_groups_of_many_tiles(n, draws):
+    """One group of 64 triangles (and, with more draws, several and the end of
+    one) meets n tiles of a row: what k_setup keeps of its runs, what k_bin walks
+    again, and lists of exactly 64."""
+    check_frame(16 * n, 16, [(1, 64), (3, 64), (0, 40)][:draws], rf.Context(clear=True, face_cull=None), (1, 0, 1, 1, 0),
+                random_soup, 16)
