@@ -574,14 +574,13 @@ rf_status rf_render(rf_device* dev, const rf_draw* draw, rf_target* target, cons
         if (e & ERRB_INDEX) return RF_E_INDEX;
         if (e & ERRB_CLIP) return RF_E_INTERNAL;
         if (sortpass_map(S, s)) return RF_E_DEVICE;
-        // the sorted fans as vertex slots and index triples of one draw
+        // the sorted fans as vertex slots of one draw
         const uint32_t n_f = S.n_f;
         dd.pre = 1;
         dd.in_tris = dd.n_tris;
         dd.in_verts = dd.n_verts;
         dd.n_verts = 3 * n_f;
         dd.n_tris = n_f;
-        dd.tris = sortpass_idx(S, 0);
         if (hipMemcpyAsync(desc, &dd, sizeof(dd), hipMemcpyHostToDevice, s)) return RF_E_DEVICE;
         B.n_verts = 3ull * n_f;
         B.n_tris = n_f;

@@ -118,7 +118,6 @@ static rf_status build_descs(Batch& b, uint32_t tile_w, uint32_t tile_h, uint32_
                 dd.in_verts = dd.n_verts;
                 dd.n_tris = nf;
                 dd.n_verts = 3 * nf;
-                dd.tris = sortpass_idx(b.sp, b.sp.off[si]);
                 b.sp.main_of[si] = (uint32_t)b.h_draws.size();
             }
             dd.vert_base = vbase;

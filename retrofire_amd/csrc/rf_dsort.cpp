@@ -50,6 +50,14 @@ rf_status sortpass_plan(Device& d, SortPass& S, hipStream_t s, uint64_t* counter
     P.tile_w = 32;
     P.tile_h = DEFAULT_TILE_H;
     P.chunk = 8;
+    // the key's fields: draw, depth (32 bits), triangle << 3 | fan
+    uint32_t draw_bits = 0, idx_bits = 4;
+    while (nd > 1 && (1u << draw_bits) < nd) ++draw_bits;
+    while ((1ull << idx_bits) < 8 * nt) ++idx_bits;
+    P.fan_draw_keyed = nd > 1 && draw_bits + 32 + idx_bits <= 64;
+    P.fan_bits = idx_bits;
+    S.key_bits = 32 + idx_bits + (P.fan_draw_keyed ? draw_bits : 0);
+    S.sort_bits = P.fan_draw_keyed ? 0 : draw_bits;
     uint32_t cap = std::max<uint32_t>(S.cap, (uint32_t)std::min<uint64_t>(2 * nt + 1024, MAX_LAUNCH_PRIMS));
     std::vector<uint32_t> misc(33);
     for (int attempt = 0;; ++attempt) {
@@ -83,20 +91,17 @@ rf_status sortpass_plan(Device& d, SortPass& S, hipStream_t s, uint64_t* counter
         S.off[i] = acc;
         acc += S.cnt[i];
     }
-    S.sort_bits = 0;
-    while (nd > 1 && (1u << S.sort_bits) < nd) ++S.sort_bits;
     // sort scratch: the larger of the two sorts' needs
     size_t t64 = 0, t32 = 0;
     unsigned long long* k = (unsigned long long*)S.keys.p;
     uint32_t* v = (uint32_t*)S.vals.p;
-    if (sort_pairs_u64(nullptr, t64, k, k + S.cap, v, v + S.cap, S.n_f, s)) return RF_E_DEVICE;
+    if (sort_pairs_u64(nullptr, t64, k, k + S.cap, v, v + S.cap, S.n_f, S.key_bits, s)) return RF_E_DEVICE;
     if (S.sort_bits &&
         sort_pairs_u32(nullptr, t32, v, v, v, v, S.n_f, S.sort_bits, s))
         return RF_E_DEVICE;
     S.tmp_bytes = std::max(t64, t32);
     if (S.tmp.ensure(std::max<size_t>(S.tmp_bytes, 4), counter) ||
-        S.key2.ensure(std::max<size_t>((size_t)S.n_f * 8, 4), counter) ||
-        S.idx.ensure(std::max<size_t>((size_t)S.n_f * 12, 4), counter) ||
+        S.key2.ensure(std::max<size_t>(S.sort_bits ? (size_t)S.n_f * 8 : 0, 4), counter) ||
         S.map.ensure(std::max<size_t>(nd, 1) * 8, counter))
         return RF_E_DEVICE;
     return RF_OK;
@@ -122,7 +127,7 @@ hipError_t sortpass_sort_gather(const SortPass& S, const BatchDesc& M, hipStream
     uint32_t* v = (uint32_t*)S.vals.p;
     uint32_t* k2 = (uint32_t*)S.key2.p;
     size_t tb = S.tmp_bytes;
-    hipError_t e = sort_pairs_u64(S.tmp.p, tb, k, k + S.cap, v, v + S.cap, S.n_f, s);
+    hipError_t e = sort_pairs_u64(S.tmp.p, tb, k, k + S.cap, v, v + S.cap, S.n_f, S.key_bits, s);
     const uint32_t* order = v + S.cap;
     const uint32_t* draws_of = nullptr;
     if (!e && S.sort_bits) {
@@ -133,13 +138,13 @@ hipError_t sortpass_sort_gather(const SortPass& S, const BatchDesc& M, hipStream
         order = v;
         draws_of = k2 + S.n_f;
     }
-    if (!e) e = launch_fan_gather(S.P, M, order, draws_of, (const uint32_t*)S.map.p, S.n_f, (uint32_t*)S.idx.p, s);
+    if (!e) e = launch_fan_gather(S.P, M, order, draws_of, (const uint32_t*)S.map.p, S.n_f, s);
     return e;
 }
 
 void sortpass_release(SortPass& S, uint64_t* counter) {
     S.sc.release(counter);
-    for (DevBuf* b : {&S.desc, &S.fans, &S.keys, &S.vals, &S.fdraw, &S.fcnt, &S.key2, &S.tmp, &S.idx, &S.map})
+    for (DevBuf* b : {&S.desc, &S.fans, &S.keys, &S.vals, &S.fdraw, &S.fcnt, &S.key2, &S.tmp, &S.map})
         b->release(counter);
 }
 

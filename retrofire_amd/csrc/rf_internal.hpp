@@ -69,10 +69,11 @@ struct Scratch {
 // Depth sort of some render() calls of a batch (render.rs:180-183,
 // 209-219; rf_dsort.cpp). Their draws, over their own meshes, form a batch P
 // of their own: P's pass clips every triangle into clip fans with depth keys,
-// a radix sort orders the fans by depth (then triangle and fan, so equal
-// depths keep submission order), a second stable sort groups them by draw,
-// and the gather writes each draw's fans, in that order, as the vertex slots
-// and index triples of the corresponding pre draw of the main batch. The
+// a radix sort orders the fans by draw and depth (then triangle and fan, so
+// equal depths keep submission order; where that exceeds a 64-bit key, by depth,
+// and a second stable sort groups them by draw), and the gather writes each
+// draw's fans, in that order, as the vertex slots of the corresponding pre draw
+// of the main batch. The
 // planning run learns each draw's fan count (fixed for fixed inputs), which
 // sizes the main batch's pre draws.
 struct SortPass {
@@ -81,11 +82,12 @@ struct SortPass {
     std::vector<uint32_t> cnt, off;   // per P draw: fans, first position in the sorted order
     uint32_t n_f = 0;                 // fans in all
     uint32_t cap = 0;                 // fan capacity of P's pass
-    uint32_t sort_bits = 0;           // key bits of the second sort (0: one draw, none)
+    uint32_t sort_bits = 0;           // key bits of the second sort (0: none)
+    uint32_t key_bits = 64;           // key bits of the first
     size_t tmp_bytes = 0;
     BatchDesc P{};
     Scratch sc;
-    DevBuf desc, fans, keys, vals, fdraw, fcnt, key2, tmp, idx, map;
+    DevBuf desc, fans, keys, vals, fdraw, fcnt, key2, tmp, map;
     uint32_t frames_n = 0;            // main frames (P's draws keep their frame indices)
     const FrameDesc* frames = nullptr;
 };
@@ -225,20 +227,20 @@ void plain_stats(rf_stats* stats, const rf_draw* draw, const FrameStats& fs, dou
 // Depth sort kernels (rf_kernels.hip, rf_sort.hip): the clip fans of B's
 // draws and their keys (B.fan_*); the radix sorts of (key, fan) pairs; the
 // draw of each fan in an order; the sorted fans written as vertex slots of
-// the main batch M's depth-sorted draws, with their index triples.
+// the main batch M's depth-sorted draws.
 hipError_t launch_fans(const BatchDesc& B, hipStream_t s);
 hipError_t sort_pairs_u64(void* tmp, size_t& tmp_bytes, const unsigned long long* keys_in,
                           unsigned long long* keys_out, const uint32_t* vals_in, uint32_t* vals_out, uint32_t n,
-                          hipStream_t s);
+                          uint32_t end_bit, hipStream_t s);
 hipError_t sort_pairs_u32(void* tmp, size_t& tmp_bytes, const uint32_t* keys_in, uint32_t* keys_out,
                           const uint32_t* vals_in, uint32_t* vals_out, uint32_t n, uint32_t end_bit, hipStream_t s);
 hipError_t launch_fan_draw_keys(const uint32_t* order, const uint32_t* fan_draw, uint32_t n, uint32_t* keys,
                                 hipStream_t s);
 hipError_t launch_fan_gather(const BatchDesc& P, const BatchDesc& M, const uint32_t* order, const uint32_t* draws_of,
-                             const uint32_t* map, uint32_t n_fans, uint32_t* idx, hipStream_t s);
+                             const uint32_t* map, uint32_t n_fans, hipStream_t s);
 
 // Uploads P's draws, runs P's pass eagerly (growing the fan capacity as
-// needed) and sizes the sorts and the index triples from the fan counts.
+// needed) and sizes the sorts from the fan counts.
 // *err_out receives P's error bits.
 rf_status sortpass_plan(Device& d, SortPass& S, hipStream_t s, uint64_t* counter, uint32_t* err_out);
 // Uploads the (first position, main draw) table once main_of is set.
@@ -248,11 +250,6 @@ hipError_t sortpass_fans(const SortPass& S, hipStream_t s);
 // The sorts and the gather into M (whose pre draws and scratch are in place).
 hipError_t sortpass_sort_gather(const SortPass& S, const BatchDesc& M, hipStream_t s);
 void sortpass_release(SortPass& S, uint64_t* counter);
-// Device pointer to index triple `first_fan` of the sorted order.
-inline const uint32_t* sortpass_idx(const SortPass& S, uint32_t first_fan) {
-    return (const uint32_t*)S.idx.p + 3ull * first_fan;
-}
-
 // Enqueues the whole pipeline for batch `B` on stream `s` (rf_kernels.hip).
 hipError_t launch_pipeline(const BatchDesc& B, hipStream_t s, uint32_t raster_grid);
 // Same, with an event recorded after each stage (for per-kernel timing);

@@ -713,11 +713,14 @@ __global__ __launch_bounds__(256) void k_setup(BatchDesc B) {
             // the caller skips a hidden object before render() (crates.rs:118-122)
         } else if (D->prim == PRIM_EDGE) {
             nf = edge_setup(B, D, F, di, g, t, rect, has_rect);
-        } else if (D->tris[3 * t] >= D->n_verts || D->tris[3 * t + 1] >= D->n_verts ||
-                   D->tris[3 * t + 2] >= D->n_verts) {
+        } else if (!D->pre && (D->tris[3 * t] >= D->n_verts || D->tris[3 * t + 1] >= D->n_verts ||
+                               D->tris[3 * t + 2] >= D->n_verts)) {
             atomicOr(B.err, ERRB_INDEX);
         } else {
-            const uint32_t ix[3] = {D->tris[3 * t], D->tris[3 * t + 1], D->tris[3 * t + 2]};
+            uint32_t ix[3] = {(uint32_t)(3 * t), (uint32_t)(3 * t + 1), (uint32_t)(3 * t + 2)};
+            if (!D->pre)
+#pragma unroll
+                for (int k = 0; k < 3; ++k) ix[k] = D->tris[3 * t + k];
             float p[3][4], sp[3][3];
             uint32_t oc[3] = {0, 0, 0};
             if (!D->pre) {
@@ -2385,13 +2388,14 @@ uint32_t raster_wg_per_cu(uint32_t tile_w, uint32_t chunk, uint32_t tile_h) {
 //                 Render::depth, (a.z + b.z + c.z) / 3 (prim.rs:21-23), as a
 //                 total_cmp order key, then the triangle and fan index, so
 //                 equal depths keep submission order;
-//   radix sort of (key, fan) pairs; with several sorted draws, a second,
-//                 stable sort by draw, so each draw's fans are contiguous and
-//                 in order (each render() call sorts its own primitives);
-//   k_fan_gather  fan i of the sorted order becomes vertex slots
-//                 3i'..3i'+2 of its draw, i' its rank in the draw (screen
+//   radix sort of (key, fan) pairs, the draw first in the key, so that each
+//                 draw's fans are contiguous and in order (each render() call
+//                 sorts its own primitives); where draw, depth and index exceed
+//                 64 bits, a second, stable sort by draw;
+//   k_fan_gather  vertex q of fan i of the sorted order becomes vertex slot
+//                 3i' + q of its draw, i' its rank in the draw (screen
 //                 vertices): the main pipeline then draws them as unclipped
-//                 triangles.
+//                 triangles, whose indices follow from their number.
 // The sorted draws form a batch of their own (their original meshes); the
 // gather writes into the main batch, whose descriptors of these draws hold
 // the fan counts the planning run found.
@@ -2402,7 +2406,9 @@ __device__ __forceinline__ void put_fan(const BatchDesc& B, const DrawDesc* D, u
     const float z = ((a.p[2] + b.p[2]) + c.p[2]) / 3.0f;
     uint32_t k = (uint32_t)total_key(z) ^ 0x80000000u;  // ascending total order as unsigned
     if (D->sort == 2) k = ~k;                           // back to front
-    B.fan_keys[f] = ((unsigned long long)k << 32) | (g << 3) | j;
+    unsigned long long key = ((unsigned long long)k << B.fan_bits) | (g << 3) | j;
+    if (B.fan_draw_keyed) key |= (unsigned long long)di << (32 + B.fan_bits);
+    B.fan_keys[f] = key;
     B.fan_vals[f] = f;
     if (B.fan_draw) B.fan_draw[f] = di;
     float* o = B.fans + (uint64_t)f * FAN_FLOATS;
@@ -2481,27 +2487,27 @@ __global__ __launch_bounds__(256) void k_fan_draw_keys(const uint32_t* order, co
     if (i < n) keys[i] = fan_draw[order[i]];
 }
 
-// Fan i of the final order (its draw d = draws_of[i], 0 if null) becomes
-// vertex slots of main draw map[2d + 1] at rank i - map[2d] (the draw's first
-// position) and index triples idx[3i..3i+2] (relative to that draw).
+// Vertex q of fan i of the final order (of draw d: draws_of[i], else the fan's
+// own where there are several) becomes vertex slot 3 rank + q of main draw
+// map[2d + 1], rank = i - map[2d] (the draw's first position). A thread a
+// vertex: the fans lie anywhere, and a thread that reads a fan's 84 bytes alone
+// waits for them three times as long (290,000 fans: 0.112 ms).
 __global__ __launch_bounds__(256) void k_fan_gather(BatchDesc P, BatchDesc M, const uint32_t* order,
-                                                    const uint32_t* draws_of, const uint32_t* map, uint32_t n_fans,
-                                                    uint32_t* idx) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+                                                    const uint32_t* draws_of, const uint32_t* map, uint32_t n_fans) {
+    const uint64_t v = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t i = (uint32_t)(v / 3), q = (uint32_t)(v - 3ull * i);
     if (i >= n_fans) return;
-    const uint32_t d = draws_of ? draws_of[i] : 0u;
+    const uint32_t f = order[i];
+    const uint32_t d = P.n_draws < 2 ? 0u : draws_of ? draws_of[i] : P.fan_draw[f];
     const uint32_t rank = i - map[2 * d];
     const DrawDesc* D = &M.draws[map[2 * d + 1]];
-    const float* src = P.fans + (uint64_t)order[i] * FAN_FLOATS;
-    const bool persp = kind_persp(D->kind);
-    for (int q = 0; q < 3; ++q) {
-        const uint64_t slot = D->vert_base + 3ull * rank + q;
-        CV c;
-        for (int e = 0; e < 4; ++e) c.p[e] = src[7 * q + e];
-        for (int e = 0; e < 3; ++e) c.a[e] = src[7 * q + 4 + e];
-        to_screen(c, D->vp, persp, M.sv + 6 * slot);
-        idx[3ull * i + q] = 3u * rank + (uint32_t)q;
-    }
+    const float* src = P.fans + (uint64_t)f * FAN_FLOATS + 7 * q;
+    CV c;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) c.p[e] = src[e];
+#pragma unroll
+    for (int e = 0; e < 3; ++e) c.a[e] = src[4 + e];
+    to_screen(c, D->vp, kind_persp(D->kind), M.sv + 6 * (D->vert_base + 3ull * rank + q));
 }
 
 // ---------------------------------------------------------------------------
@@ -2647,11 +2653,11 @@ hipError_t launch_fan_draw_keys(const uint32_t* order, const uint32_t* fan_draw,
     return hipGetLastError();
 }
 hipError_t launch_fan_gather(const BatchDesc& P, const BatchDesc& M, const uint32_t* order, const uint32_t* draws_of,
-                             const uint32_t* map, uint32_t n_fans, uint32_t* idx, hipStream_t s) {
-    if (n_fans && (!P.fans || !order || !map || !idx || !M.sv)) return hipErrorInvalidValue;
+                             const uint32_t* map, uint32_t n_fans, hipStream_t s) {
+    if (n_fans && (!P.fans || !order || !map || !M.sv)) return hipErrorInvalidValue;
     if (n_fans)
-        hipLaunchKernelGGL(k_fan_gather, dim3((n_fans + 255) / 256), dim3(256), 0, s, P, M, order, draws_of, map,
-                           n_fans, idx);
+        hipLaunchKernelGGL(k_fan_gather, dim3((uint32_t)((3ull * n_fans + 255) / 256)), dim3(256), 0, s, P, M, order, draws_of,
+                           map, n_fans);
     return hipGetLastError();
 }
 hipError_t launch_pipeline(const BatchDesc& B, hipStream_t s, uint32_t raster_grid) {

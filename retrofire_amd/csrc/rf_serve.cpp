@@ -474,8 +474,7 @@ static rf_status launch_lane_sorted(Serve& s, Lane& l) {
     rf_status st = sortpass_plan(d, S, l.stream, &s.sort_bytes, &e);
     if (!st) st = map_err(e);
     if (st) return st;
-    // the main draws: the sorted fans of each triangle draw as its vertex
-    // slots and index triples
+    // the main draws: the sorted fans of each triangle draw as its vertex slots
     std::vector<DrawDesc> dds;
     uint64_t vbase = 0, tbase = 0;
     uint32_t any_cull = 0;
@@ -489,7 +488,6 @@ static rf_status launch_lane_sorted(Serve& s, Lane& l) {
             dd.in_verts = dd.n_verts;
             dd.n_tris = nf;
             dd.n_verts = 3 * nf;
-            dd.tris = sortpass_idx(S, S.off[si]);
             S.main_of[si] = (uint32_t)k;
         }
         dd.vert_base = vbase;

@@ -9,12 +9,13 @@
 
 namespace rf {
 
-// With tmp == nullptr only sets tmp_bytes (the scratch the sort needs).
+// With tmp == nullptr only sets tmp_bytes (the scratch the sort needs). Only
+// key bits [0, end_bit) are compared.
 hipError_t sort_pairs_u64(void* tmp, size_t& tmp_bytes, const unsigned long long* keys_in,
                           unsigned long long* keys_out, const uint32_t* vals_in, uint32_t* vals_out, uint32_t n,
-                          hipStream_t s) {
-    return hipcub::DeviceRadixSort::SortPairs(tmp, tmp_bytes, keys_in, keys_out, vals_in, vals_out, (int)n, 0, 64,
-                                              s);
+                          uint32_t end_bit, hipStream_t s) {
+    return hipcub::DeviceRadixSort::SortPairs(tmp, tmp_bytes, keys_in, keys_out, vals_in, vals_out, (int)n, 0,
+                                              (int)end_bit, s);
 }
 
 // 32-bit keys (only bits [0, end_bit) compared), 32-bit values; stable.

@@ -82,7 +82,7 @@ enum ErrBits : uint32_t {
 struct DrawDesc {
     const float* pos;       // n_verts x (x, y, z)
     const float* attr;      // n_verts x kind_attrs(kind)
-    const uint32_t* tris;   // n_tris x (i0, i1, i2), or x (i0, i1) for edges
+    const uint32_t* tris;   // n_tris x (i0, i1, i2), or x (i0, i1) for edges; a pre draw's are 3t, 3t + 1, 3t + 2
     const uint8_t* tex;     // Color4 texels (textured kinds)
     uint32_t n_verts, n_tris;
     uint32_t kind, frame;
@@ -222,7 +222,9 @@ struct BatchDesc {
     uint32_t depth_sort;              // 0 none, 1 front to back, 2 back to front
     uint32_t fan_cap;
     float* fans;                      // per fan: 3 x (x, y, z, w, a0, a1, a2)
-    unsigned long long* fan_keys;     // per fan: order key << 32 | triangle << 3 | fan
+    unsigned long long* fan_keys;     // per fan: draw (if it fits) | order key | triangle << 3 | fan
+    uint32_t fan_bits;                // bits of the key's last field
+    uint32_t fan_draw_keyed;          // 1: the draw is the key's first field
     uint32_t* fan_vals;               // per fan: its index in `fans`
     uint32_t* fan_count;
     uint32_t* fan_draw;               // per fan: its draw

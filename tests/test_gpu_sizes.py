@@ -250,3 +250,33 @@ def test_groups_of_many_tiles(n, draws):
     again, and lists of exactly 64."""
     check_frame(16 * n, 16, [(1, 64), (3, 64), (0, 40)][:draws], rf.Context(clear=True, face_cull=None), (1, 0, 1, 1, 0),
                 random_soup, 16)
+
+
+@pytest.mark.parametrize("n,per", [(2, 3), (64, 17), (3000, 3), (9000, 21)])
+def test_many_depth_sorted_draws(n, per):
+    """So many sorted render() calls that draw, depth and index still fit one
+    sort key, or (9,000 calls of 21 triangles) do not: each sorts its own."""
+    rng = np.random.default_rng(n)
+    w = h = 24
+    kinds = [small_soup(rng, per, w, h, 1) for _ in range(min(n, 50))]
+    meshes = [RB.Mesh(p, t, a) for p, a, t, _, _ in kinds]
+    fb = RB.DeviceFramebuf(w, h, 0, False)
+    ocol, ost = np.zeros((h, w, 4), np.uint8), np.zeros(8, np.uint64)
+    ocol[...] = (0, 0, 0, 255)
+    draws = []
+    for k in range(n):
+        pos, attr, tris, mvp, vp = kinds[k % len(kinds)]
+        draws.append(RB.mesh_draw(meshes[k % len(kinds)], rf.shader.Gouraud(), mvp, vp))
+        err, _ = O.render(1, tris, pos, attr, mvp, vp, ocol, ctx=(0, 0, 1, 1, 2), stats=ost)
+        assert err == 0
+    ctx = rf.Context(clear=True, face_cull=None, depth_test=None, depth_sort="back_to_front")
+    b = RB.Batch([(fb, ctx, draws)], tile_w=16)
+    for _ in range(2):
+        b.run()
+        s = b.wait()[0]
+        assert np.array_equal(fb.read()[0], ocol)
+        assert [s.calls, s.prims_i, s.prims_o, s.verts_i, s.verts_o, s.frags_i, s.frags_o] == [int(x) for x in ost[:7]]
+    b.free()
+    fb.free()
+    for m in meshes:
+        m.free()
