@@ -130,6 +130,7 @@ static void scratch_arrays(BatchDesc& B, Fn&& fn) {
     fn(nt * 2 * sizeof(uint32_t), (void**)&B.rect);
     fn(nt * sizeof(float), (void**)&B.zmax);
     fn((nt / 64 + 1) * sizeof(uint32_t), (void**)&B.group_draw);
+    fn((nt / 64 + 1) * sizeof(GroupBound), (void**)&B.group_max);
     fn((nt / 64 + 1) * PRE_RUNS * sizeof(uint32_t), (void**)&B.tile_of);
     fn((nt / 64 + 1) * PRE_RUNS * 8, (void**)&B.mask_of);
     fn((nt / 64 + 1) * sizeof(uint32_t), (void**)&B.n_runs);

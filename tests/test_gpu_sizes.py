@@ -280,3 +280,26 @@ def test_many_depth_sorted_draws(n, per):
     fb.free()
     for m in meshes:
         m.free()
+
+
+def coherent_soup(rng, n, w, h, kind):
+    """Small triangles whose 64 of a group lie together, the groups at depths of
+    their own; every fifth group has one triangle through the near plane or one
+    as large as the frame among them."""
+    pos, attr, tris, _, vp = random_soup(rng, n, w, h, kind)
+    g = -(-n // 64)
+    mid = np.repeat(rng.uniform([-0.8, -0.8, 0.0], [0.8, 0.8, 5.0], size=(g, 3)), 64, axis=0)[:n, None]
+    pos = mid + rng.uniform(-1, 1, size=(n, 3, 3)) * [0.15, 0.15, 0.02]
+    odd = np.arange(7, n, 320)
+    pos[odd[0::2], 2, 2] = -3.0
+    pos[odd[1::2]] = mid[odd[1::2]] + rng.uniform(-1, 1, size=(len(odd[1::2]), 3, 3)) * [3.0, 3.0, 0.5]
+    mvp = M.then(M.translate3(0, 0, 2.0), M.perspective(1.2, np.float32(w / h), 0.1, 8.0))
+    return pos.reshape(-1, 3).astype(np.float32), attr, tris, mvp, vp
+
+
+@pytest.mark.parametrize("w,h,tw", [(16, 16, 16), (37, 29, 32)])
+@pytest.mark.parametrize("groups", [64, 65, 128, 129, 300])
+def test_whole_groups_behind(groups, w, h, tw):
+    """Run lists around multiples of 64, most of whose groups are hidden as a whole."""
+    check_frame(w, h, [(1, 64 * groups - 5), (3, 130)], rf.Context(clear=True, face_cull=None), (1, 0, 1, 1, 0),
+                coherent_soup, tw)
