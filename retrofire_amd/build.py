@@ -12,12 +12,15 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "librfamd.so")
-# (object name, source, extra flags). rf_kernels.hip builds twice: the pipeline
-# kernels, and k_raster alone under the max-ilp scheduler (shorter dependent
-# chains in the rasterizer; the same scheduler makes k_setup slower).
+# (object name, source, extra flags). rf_kernels.hip builds three times: the
+# pipeline kernels, and k_raster alone, without and with edges, under the max-ilp
+# scheduler (shorter dependent chains in the rasterizer; the same scheduler makes
+# k_setup slower).
+ILP = ["-mllvm", "-amdgpu-sched-strategy=max-ilp"]
 SOURCES = [
     ("rf_kernels", "rf_kernels.hip", []),
-    ("rf_raster", "rf_kernels.hip", ["-DRF_RASTER_TU", "-mllvm", "-amdgpu-sched-strategy=max-ilp"]),
+    ("rf_raster", "rf_kernels.hip", ["-DRF_RASTER_TU=0"] + ILP),
+    ("rf_raster_lines", "rf_kernels.hip", ["-DRF_RASTER_TU=1"] + ILP),
     ("rf_sort", "rf_sort.hip", []),
     ("rf_api", "rf_api.cpp", []),
     ("rf_batch", "rf_batch.cpp", []),

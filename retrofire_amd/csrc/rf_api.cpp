@@ -186,7 +186,8 @@ uint32_t grow_runs_cap(uint32_t needed) {
 }
 
 uint32_t raster_grid(const Device& d, const BatchDesc& B) {
-    const uint32_t g = (uint32_t)d.num_cu * raster_wg_per_cu(B.tile_w, B.chunk, B.tile_h);
+    const uint32_t g = (uint32_t)d.num_cu * (B.any_lines ? raster_wg_per_cu_lines(B.tile_w, B.chunk, B.tile_h)
+                                                         : raster_wg_per_cu_tris(B.tile_w, B.chunk, B.tile_h));
     return std::max(1u, std::min(B.n_tiles, g));
 }
 
@@ -372,6 +373,7 @@ void plain_descs(const rf_draw* draw, const rf_target* target, const rf_ctx* ctx
     B.n_tris = draw->n_tris;
     B.n_groups = (uint32_t)((draw->n_tris + WAVE_SIZE - 1) / WAVE_SIZE);
     B.n_tiles = tile_base;
+    B.any_lines = draw->prim == PRIM_EDGE;
     B.tile_w = tile_w;
     B.chunk = chunk;
     B.tile_h = tile_h;

@@ -83,7 +83,7 @@ static rf_status build_descs(Batch& b, uint32_t tile_w, uint32_t tile_h, uint32_
     b.frame_verts_i.assign(b.frames.size(), 0);
     b.frame_calls.assign(b.frames.size(), 0);
     b.frame_objs.assign(b.frames.size(), 0);
-    uint32_t any_cull = 0;
+    uint32_t any_cull = 0, any_lines = 0;
     uint64_t vbase = 0, tbase = 0;
     uint32_t tile_base = 0;
     for (size_t fi = 0; fi < b.frames.size(); ++fi) {
@@ -123,6 +123,7 @@ static rf_status build_descs(Batch& b, uint32_t tile_w, uint32_t tile_h, uint32_
             dd.vert_base = vbase;
             dd.tri_base = tbase;
             any_cull |= md.cull;
+            any_lines |= dd.prim == PRIM_EDGE;
             vbase += dd.pre ? dd.n_verts : 0;
             tbase += dd.n_tris;
             b.frame_calls[fi] += 1;
@@ -148,6 +149,7 @@ static rf_status build_descs(Batch& b, uint32_t tile_w, uint32_t tile_h, uint32_
     B.n_groups = (uint32_t)((tbase + WAVE_SIZE - 1) / WAVE_SIZE);
     B.n_tiles = tile_base;
     B.any_cull = any_cull;
+    B.any_lines = any_lines;
     B.tile_w = tile_w;
     B.tile_h = tile_h;
     B.chunk = chunk;

@@ -188,7 +188,8 @@ void set_grid(FrameDesc& f, uint32_t tile_w, uint32_t tile_h, uint32_t& tile_bas
 // its instance, times the CUs, at most one per tile).
 uint32_t raster_grid(const Device& d, const BatchDesc& B);
 // Resident one-wave rasterizer workgroups per CU of an instance (rf_kernels.hip).
-uint32_t raster_wg_per_cu(uint32_t tile_w, uint32_t chunk, uint32_t tile_h);
+uint32_t raster_wg_per_cu_tris(uint32_t tile_w, uint32_t chunk, uint32_t tile_h);
+uint32_t raster_wg_per_cu_lines(uint32_t tile_w, uint32_t chunk, uint32_t tile_h);
 // Runs B's pipeline on `s` synchronously, growing B's clip-fan and bin-run
 // capacities (and the scratch, counted in *counter) until they suffice;
 // `pre` runs before each attempt's pipeline, `restore` before each retry.
@@ -256,7 +257,9 @@ hipError_t launch_pipeline(const BatchDesc& B, hipStream_t s, uint32_t raster_gr
 // `ev` holds 8 events.
 hipError_t launch_pipeline_timed(const BatchDesc& B, hipStream_t s, uint32_t raster_grid, hipEvent_t* ev);
 // The rasterizer's launch alone: rf_kernels.hip compiled with RF_RASTER_TU
-// (its own object, scheduled for instruction-level parallelism).
-hipError_t launch_raster(const BatchDesc& B, hipStream_t s, uint32_t raster_grid);
+// (objects of their own, scheduled for instruction-level parallelism), for
+// launches without and with edges.
+hipError_t launch_raster_tris(const BatchDesc& B, hipStream_t s, uint32_t raster_grid);
+hipError_t launch_raster_lines(const BatchDesc& B, hipStream_t s, uint32_t raster_grid);
 
 }  // namespace rf

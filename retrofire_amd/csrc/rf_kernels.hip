@@ -19,17 +19,19 @@
 //              rasterize_fb target.rs:163-198); the tile is written to HBM
 //              once.
 //
-// The file is compiled twice: as the pipeline (every kernel but k_raster, and
-// the launchers), and with RF_RASTER_TU defined as k_raster alone, under the
-// max-ilp scheduler. That scheduling shortens k_raster's dependent chains
-// (1.145 -> 1.131 ms per 64 crates1080 frames) and would lengthen k_setup's
-// (0.092 -> 0.096 ms), so it applies to k_raster only.
+// The file is compiled three times: as the pipeline (every kernel but k_raster,
+// and the launchers), and with RF_RASTER_TU defined as k_raster alone, for
+// launches without (0) and with (1) edges, under the max-ilp scheduler. That
+// scheduling shortens k_raster's dependent chains (1.145 -> 1.131 ms per 64
+// crates1080 frames) and would lengthen k_setup's (0.092 -> 0.096 ms), so it
+// applies to k_raster only.
 //
 // Exactness: the serial recurrences of the reference (edge stepping per row,
 // varying stepping per pixel) are reproduced as serial sums; no closed forms.
 #include <hip/hip_runtime.h>
 
 #include <cstddef>
+#include <type_traits>
 
 #include "rf_ff.hpp"
 #include "rf_math.hpp"
@@ -1541,7 +1543,10 @@ __device__ __forceinline__ bool depth_pass_u(int32_t dt, float nz, float cur) {
 // TW: tile width (16, 32, 64); CH: pixels per lane applied together in a span
 // round (6 or 8: short spans waste fewer lanes' slots and registers at 6,
 // long spans take fewer rounds at 8).
-template <int TW, int CH, int TH>
+// LINES: the launch draws edges. The others carry neither the lines' set-up nor
+// the one-pixel copy of a round (8 icosphere frames: 1.97 ms as one instance for
+// both, 2.02 with that copy in it, 1.92 apart).
+template <int TW, int CH, int TH, bool LINES>
 __global__ __launch_bounds__(64, 2) void k_raster(BatchDesc B) {
     constexpr int TILE_H = TH;  // tile rows
     constexpr int REC_CAP = rec_cap(TW, TH);
@@ -1912,7 +1917,7 @@ __global__ __launch_bounds__(64, 2) void k_raster(BatchDesc B) {
                     }
                     di = st->draw;
                     kind = st->kind & 0xFFu;
-                    is_line = (st->kind & KIND_LINE) != 0u;
+                    is_line = LINES && (st->kind & KIND_LINE) != 0u;
                     counted = (st->kind & KIND_COUNTED) != 0u;
                     na = kind_attrs(kind);
                     if (is_line) {
@@ -2087,7 +2092,7 @@ __global__ __launch_bounds__(64, 2) void k_raster(BatchDesc B) {
                 if (valid) {
                     const EdgeRec R = s_rec[k];
                     const SlotP& P = s_slot[f];
-                    if (P.kind_tag & LINE_TAG) {
+                    if (LINES && (P.kind_tag & LINE_TAG)) {
                         // a line pixel (Scanline x..x + 1 with the first end's
                         // single varying value); only the tile holding it draws it
                         const uint32_t px = cvt_u32(R.lx), py = cvt_u32(R.rx);
@@ -2203,13 +2208,15 @@ __global__ __launch_bounds__(64, 2) void k_raster(BatchDesc B) {
 #pragma unroll
             for (int32_t c = 0; c < NCG; ++c)
                 if (c >= cl0 && c <= cw1) win = win && cells[c] == key;
-            if (win) {
+            // the next N pixels of the winners' records
+            auto apply = [&](auto n_px) {
+                constexpr int N = decltype(n_px)::value;
                 const int32_t rem = j1 - jc;
                 const uint32_t li = (uint32_t)(xs + jc - (int32_t)x0) * LD + row;
-                float zz[CH], v0[CH], v1[CH], v2[CH], cur[CH];
-                bool ps[CH];
+                float zz[N], v0[N], v1[N], v2[N], cur[N];
+                bool ps[N];
 #pragma unroll
-                for (int p = 0; p < CH; ++p) {
+                for (int p = 0; p < N; ++p) {
                     zz[p] = z;
                     v0[p] = c0;
                     v1[p] = c1;
@@ -2222,14 +2229,14 @@ __global__ __launch_bounds__(64, 2) void k_raster(BatchDesc B) {
                 // the pixels of one chunk are distinct: read all depths first
                 if (has_depth) {
 #pragma unroll
-                    for (int p = 0; p < CH; ++p) cur[p] = s_px[li + p * LD];  // p >= rem: unused
+                    for (int p = 0; p < N; ++p) cur[p] = s_px[li + p * LD];  // p >= rem: unused
                 } else {
 #pragma unroll
-                    for (int p = 0; p < CH; ++p) cur[p] = 0.0f;
+                    for (int p = 0; p < N; ++p) cur[p] = 0.0f;
                 }
                 uint32_t npass = 0;
 #pragma unroll
-                for (int p = 0; p < CH; ++p) {
+                for (int p = 0; p < N; ++p) {
                     ps[p] = (p < rem) & depth_pass_u(dtest, zz[p], cur[p]);
                     npass += ps[p] ? 1u : 0u;
                 }
@@ -2237,7 +2244,7 @@ __global__ __launch_bounds__(64, 2) void k_raster(BatchDesc B) {
                     // the shader runs for every passing fragment, colour write or not
                     const float tw = (float)ip0, th = (float)ip1;
 #pragma unroll
-                    for (int p = 0; p < CH; ++p)
+                    for (int p = 0; p < N; ++p)
                         if (ps[p] && (cvt_u32(tw * (v0[p] / zz[p])) >= ip0 || cvt_u32(th * (v1[p] / zz[p])) >= ip1))
                             errs |= ERRB_TEXEL;
                 }
@@ -2245,16 +2252,16 @@ __global__ __launch_bounds__(64, 2) void k_raster(BatchDesc B) {
                     fo_acc += npass;
                     // colour sources of the chunk's pixels (the shader kind is
                     // decided once per chunk)
-                    uint32_t pay[CH];
+                    uint32_t pay[N];
                     uint32_t tg;
                     if (ikind == KIND_FLAT) {
                         tg = TAG_COLOR;
 #pragma unroll
-                        for (int p = 0; p < CH; ++p) pay[p] = ip0;
+                        for (int p = 0; p < N; ++p) pay[p] = ip0;
                     } else if (ikind == KIND_GOURAUD) {  // Color3f::to_color4 (color.rs:253-263)
                         tg = TAG_COLOR;
 #pragma unroll
-                        for (int p = 0; p < CH; ++p)
+                        for (int p = 0; p < N; ++p)
                             pay[p] = pack_pixel(F.fmt, cvt_u8(256.0f * v0[p]), cvt_u8(256.0f * v1[p]),
                                                 cvt_u8(256.0f * v2[p]), 0xFF);
                     } else {
@@ -2263,7 +2270,7 @@ __global__ __launch_bounds__(64, 2) void k_raster(BatchDesc B) {
                         if (ikind == KIND_TEX_CLAMP) {  // SamplerClamp (tex.rs:280-303)
                             const float mu = tw - 1.0f, mv = th - 1.0f;
 #pragma unroll
-                            for (int p = 0; p < CH; ++p) {
+                            for (int p = 0; p < N; ++p) {
                                 // Scanline::fragments z_div (raster.rs:61-68, vec.rs:666-676)
                                 float su = (v0[p] / zz[p]) * tw, sv = (v1[p] / zz[p]) * th;
                                 su = su < 0.0f ? 0.0f : su;
@@ -2274,14 +2281,14 @@ __global__ __launch_bounds__(64, 2) void k_raster(BatchDesc B) {
                             }
                         } else if (ikind == KIND_TEX_REPEAT_POT) {  // SamplerRepeatPot (tex.rs:240-266)
 #pragma unroll
-                            for (int p = 0; p < CH; ++p) {
+                            for (int p = 0; p < N; ++p) {
                                 const uint32_t ui = (uint32_t)cvt_i32(floorf(tw * (v0[p] / zz[p]))) & (ip0 - 1);
                                 const uint32_t vi = (uint32_t)cvt_i32(floorf(th * (v1[p] / zz[p]))) & (ip1 - 1);
                                 pay[p] = vi * ip2 + ui;
                             }
                         } else {  // SamplerOnce (tex.rs:343-357): `as u32`, no wrap
 #pragma unroll
-                            for (int p = 0; p < CH; ++p) {
+                            for (int p = 0; p < N; ++p) {
                                 const uint32_t ui = cvt_u32(tw * (v0[p] / zz[p]));
                                 const uint32_t vi = cvt_u32(th * (v1[p] / zz[p]));
                                 // outside the texture the reference panics (checked
@@ -2291,7 +2298,7 @@ __global__ __launch_bounds__(64, 2) void k_raster(BatchDesc B) {
                         }
                     }
 #pragma unroll
-                    for (int p = 0; p < CH; ++p) {
+                    for (int p = 0; p < N; ++p) {
                         if (ps[p]) {
                             s_tag[li + p * LD] = (uint8_t)tg;
                             s_pay[li + p * LD] = pay[p];
@@ -2300,11 +2307,19 @@ __global__ __launch_bounds__(64, 2) void k_raster(BatchDesc B) {
                 }
                 if (dwrite) {
 #pragma unroll
-                    for (int p = 0; p < CH; ++p)
+                    for (int p = 0; p < N; ++p)
                         if (ps[p]) s_dep[li + p * LD] = zz[p];
                 }
-                jc += CH;
+                jc += N;
                 if (jc >= j1) have = false;
+            };
+            // lines' records are single pixels: rounds of them alone apply no
+            // more (8 frames of 500 crates' edges over their fill: 0.264 ->
+            // 0.225 ms; at two pixels 0.240)
+            if (LINES && __ballot(win && j1 - jc > 1) == 0ull) {
+                if (win) apply(std::integral_constant<int, 1>{});
+            } else if (win) {
+                apply(std::integral_constant<int, CH>{});
             }
             // release the claims: every lane frees its whole row (one vector
             // write). Every claimed cell lies in a claimant's row, so all
@@ -2387,7 +2402,9 @@ __global__ __launch_bounds__(64, 2) void k_raster(BatchDesc B) {
 // The rasterizer's instances: tile width {16, 32, 64} x span chunk {6, 8}
 // x tile height {16, 32, 64}.
 using RasterFn = void (*)(BatchDesc);
-#define RF_K3(TW, CH) {k_raster<TW, CH, 16>, k_raster<TW, CH, 32>, k_raster<TW, CH, 64>}
+constexpr bool TU_LINES = RF_RASTER_TU != 0;
+#define RF_K3(TW, CH) \
+    {k_raster<TW, CH, 16, TU_LINES>, k_raster<TW, CH, 32, TU_LINES>, k_raster<TW, CH, 64, TU_LINES>}
 static const RasterFn RASTER_FNS[3][2][3] = {
     {RF_K3(16, 6), RF_K3(16, 8)}, {RF_K3(32, 6), RF_K3(32, 8)}, {RF_K3(64, 6), RF_K3(64, 8)}};
 #undef RF_K3
@@ -2398,14 +2415,19 @@ static int raster_index(uint32_t tw, uint32_t ch, uint32_t th, int* i, int* j, i
     return 0;
 }
 
-hipError_t launch_raster(const BatchDesc& B, hipStream_t s, uint32_t raster_grid) {
+#if RF_RASTER_TU
+#define RF_TU(name) name##_lines
+#else
+#define RF_TU(name) name##_tris
+#endif
+hipError_t RF_TU(launch_raster)(const BatchDesc& B, hipStream_t s, uint32_t raster_grid) {
     int i, j, k;
     raster_index(B.tile_w, B.chunk, B.tile_h, &i, &j, &k);
     hipLaunchKernelGGL(RASTER_FNS[i][j][k], dim3(raster_grid), dim3(64), 0, s, B);
     return hipGetLastError();
 }
 
-uint32_t raster_wg_per_cu(uint32_t tile_w, uint32_t chunk, uint32_t tile_h) {
+uint32_t RF_TU(raster_wg_per_cu)(uint32_t tile_w, uint32_t chunk, uint32_t tile_h) {
     // resident one-wave workgroups per CU of each instance (registers and
     // LDS decide), asked of the runtime once
     static int occ[3][2][3] = {};
@@ -2675,7 +2697,7 @@ static hipError_t launch_impl(const BatchDesc& B0, hipStream_t s, uint32_t raste
         hipLaunchKernelGGL(k_binsort, dim3(B.n_tiles < 1024u ? B.n_tiles : 1024u), dim3(256), 0, s, B);
     mark(5);
     chk(hipGetLastError());
-    chk(launch_raster(B, s, raster_grid));
+    chk(B.any_lines ? launch_raster_lines(B, s, raster_grid) : launch_raster_tris(B, s, raster_grid));
     mark(6);
     chk(hipGetLastError());
     return e;

@@ -477,7 +477,7 @@ static rf_status launch_lane_sorted(Serve& s, Lane& l) {
     // the main draws: the sorted fans of each triangle draw as its vertex slots
     std::vector<DrawDesc> dds;
     uint64_t vbase = 0, tbase = 0;
-    uint32_t any_cull = 0;
+    uint32_t any_cull = 0, any_lines = 0;
     for (size_t k = 0; k < q.draws.size(); ++k) {
         DrawDesc dd = draw_desc(q.draws[k], 0);
         if (const int32_t si = sort_of[k]; si >= 0) {
@@ -493,6 +493,7 @@ static rf_status launch_lane_sorted(Serve& s, Lane& l) {
         dd.vert_base = vbase;
         dd.tri_base = tbase;
         any_cull |= dd.cull;
+        any_lines |= dd.prim == PRIM_EDGE;
         vbase += dd.pre ? dd.n_verts : 0;
         tbase += dd.n_tris;
         dds.push_back(dd);
@@ -516,6 +517,7 @@ static rf_status launch_lane_sorted(Serve& s, Lane& l) {
     B.tile_h = DEFAULT_TILE_H;
     B.chunk = RF_SERVE_CHUNK;
     B.any_cull = any_cull;
+    B.any_lines = any_lines;
     B.extra_cap = l.extra_cap;
     B.runs_cap = std::max<uint32_t>(4 * B.n_groups + B.n_tiles + 1024, l.runs_cap);
     std::vector<FrameStats> fs;
@@ -569,7 +571,7 @@ static rf_status launch_lane(Serve& s, Lane& l) {
     dds.reserve(p.n_draws);
     fds.reserve(p.n_frames);
     uint64_t tbase = 0;
-    uint32_t tile_base = 0, any_cull = 0;
+    uint32_t tile_base = 0, any_cull = 0, any_lines = 0;
     for (size_t i = 0; i < l.reqs.size(); ++i) {
         Req& q = l.reqs[i];
         fds.push_back(frame_desc(q, tgt, tile_base));
@@ -577,11 +579,13 @@ static rf_status launch_lane(Serve& s, Lane& l) {
             DrawDesc dd = draw_desc(md, (uint32_t)i);
             dd.tri_base = tbase;
             any_cull |= md.cull;
+            any_lines |= dd.prim == PRIM_EDGE;
             tbase += dd.n_tris;
             dds.push_back(dd);
         }
     }
     B.any_cull = any_cull;
+    B.any_lines = any_lines;
     const size_t total = db + fb;
     if (rf_status st = stage_room(l, total, (uint32_t)fds.size())) return st;
     std::memcpy(l.h_desc, dds.data(), dds.size() * sizeof(DrawDesc));

@@ -226,6 +226,7 @@ struct BatchDesc {
     unsigned long long* prims_part;  // per frame: PRIM_PARTS partial counters (prims.o, frags.i)
     uint32_t* draw_vis;  // per draw: 0 if the bounding-box test hid it, else 1
     uint32_t any_cull;   // some draw asks for the bounding-box test
+    uint32_t any_lines;  // some draw is of edges
     // depth sort (render.rs:180-183, 209-219): clip fans in clip space, their keys
     uint32_t depth_sort;              // 0 none, 1 front to back, 2 back to front
     uint32_t fan_cap;

@@ -171,3 +171,33 @@ def test_edges_pixel_formats(fmt):
     for ctx, with_depth in ((rf.Context(clear=True, face_cull=None), True), (rf.Context(clear=False), False)):
         o, g = run_both(1, edges, pos, attr, mvp, vp, w, h, fmt=fmt, with_depth=with_depth, ctx=ctx)
         assert_same(o, g)
+
+
+@pytest.mark.parametrize("at", [0, 1, 2])
+def test_edges_in_one_draw_of_several(at):
+    """A batch of three one-draw frames, one of them of edges: the rasterizer
+    that the launch takes draws the lines and the triangles alike."""
+    rng = np.random.default_rng(at)
+    w, h = 83, 61
+    frames, meshes, fbs, want = [], [], [], []
+    for i in range(3):
+        pos, attr, edges, mvp, vp = edge_soup(rng, 90, w, h, 1)
+        prims = edges if i == at else np.arange(180, dtype=np.uint32).reshape(60, 3)
+        ocol, odep, ost = np.zeros((h, w, 4), np.uint8), np.zeros((h, w), np.float32), np.zeros(8, np.uint64)
+        ocol[...] = (0, 0, 0, 255)
+        err, _ = O.render(1, prims, pos, attr, mvp, vp, ocol, depth=odep, stats=ost, prim=int(i == at))
+        assert err == 0
+        meshes.append(RB.Mesh(pos, prims, attr))
+        fbs.append(RB.DeviceFramebuf(w, h, 0, True))
+        frames.append((fbs[i], rf.Context(clear=True), [RB.mesh_draw(meshes[i], rf.shader.Gouraud(), mvp, vp)]))
+        want.append((ocol, odep, ost))
+    b = RB.Batch(frames)
+    b.run()
+    for s, fb, (ocol, odep, ost) in zip(b.wait(), fbs, want):
+        gcol, gdep = fb.read()
+        assert np.array_equal(gcol, ocol)
+        assert np.array_equal(gdep.view(np.uint32), odep.view(np.uint32))
+        assert [s.prims_o, s.frags_i, s.frags_o] == [int(ost[2]), int(ost[5]), int(ost[6])]
+    b.free()
+    for o in fbs + meshes:
+        o.free()
