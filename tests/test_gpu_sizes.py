@@ -303,3 +303,16 @@ def test_whole_groups_behind(groups, w, h, tw):
     """Run lists around multiples of 64, most of whose groups are hidden as a whole."""
     check_frame(w, h, [(1, 64 * groups - 5), (3, 130)], rf.Context(clear=True, face_cull=None), (1, 0, 1, 1, 0),
                 coherent_soup, tw)
+
+
+@pytest.mark.parametrize("w,h", [(128, 128), (144, 128), (1024, 16), (1040, 16), (16, 1040)])
+@pytest.mark.parametrize("sizes", [(64,), (200,), (33, 31, 70)])
+def test_groups_over_a_block_of_tiles(w, h, sizes):
+    """Groups whose triangles span 64 tiles (of 16 x 16) and more, of one draw
+    and of several."""
+    dev = rf.default_device()
+    dev.set_tile_height(16)
+    try:
+        check_frame(w, h, [(1, n) for n in sizes], rf.Context(clear=True, face_cull=None), (1, 0, 1, 1, 0), tile_w=16)
+    finally:
+        dev.set_tile_height(0)
