@@ -200,7 +200,7 @@ rf_status rf_render(rf_device* dev, const rf_draw* draw, rf_target* target, cons
  * capture, tight serving loops, harnesses that forbid hipMalloc). Same
  * arguments, results and errors as rf_render, but every device buffer (the
  * draw's vertices, indices and texels, the target, descriptors and pipeline
- * scratch) comes from one static device array of 64 MiB per GPU, held from
+ * scratch) comes from one static device array of 80 MiB per GPU, held from
  * the first rf_device_open until the process ends; the call makes no
  * hipMalloc or hipFree. A draw whose buffers do not fit the array returns
  * RF_E_BUDGET before any device work (a 1920x1080 RGBA8 target with depth
@@ -297,7 +297,7 @@ uint32_t rf_batch_tune_results(const rf_batch* b, rf_tune_entry* out, uint32_t m
 rf_status rf_batch_last_ms(const rf_batch* b, float* total_ms, float* raster_ms);
 /* Runs the pipeline `iters` times outside the graph with an event after each
  * stage on the batch stream; ms[0..5] receive the mean milliseconds of:
- * vertex (with counter reset), setup, scan, bin, bin sort, raster. */
+ * counter reset (with culling), setup, scan, bin, bin sort, raster. */
 rf_status rf_batch_profile(rf_batch* b, int iters, float* ms);
 
 /* ---- serving ------------------------------------------------------------

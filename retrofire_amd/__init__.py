@@ -273,7 +273,7 @@ def make_draw(prims, verts, shd, uniform, to_screen, keep: list) -> _ffi.RfDraw:
 
 def render_noalloc(prims, verts, shd, uniform, to_screen, target, ctx: Context, device: Device | None = None):
     """render() through rf_render_noalloc: the same call and result, with
-    every device buffer taken from the library's fixed 64 MiB array per GPU
+    every device buffer taken from the library's fixed 80 MiB array per GPU
     instead of device allocations (for callers that cannot allocate). A call
     whose buffers do not fit raises RenderError(-9)."""
     _render(prims, verts, shd, uniform, to_screen, target, ctx, device, "rf_render_noalloc")

@@ -23,7 +23,10 @@
 
 namespace rf {
 
-constexpr uint64_t NOALLOC_BYTES = 64ull << 20;  // the largest layout rf_render_noalloc takes
+// The largest layout rf_render_noalloc takes. A triangle's share of it is 114
+// bytes (its indices, its scratch, its group's runs and bound), and a draw of
+// 600,000 triangles over a few vertices should fit.
+constexpr uint64_t NOALLOC_BYTES = 80ull << 20;
 
 // In host code `scratch` names a host-side stand-in of the array, not its
 // device address: only the address hipGetSymbolAddress returns for the

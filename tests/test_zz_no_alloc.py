@@ -6,6 +6,7 @@ import numpy as np
 import pytest
 
 import retrofire_amd as rf
+from retrofire_amd import mat as M
 from retrofire_amd import scenes as S
 
 pytestmark = pytest.mark.gpu
@@ -55,3 +56,23 @@ def test_noalloc_refuses_what_does_not_fit():
         rf.render_noalloc(sc.tris, (sc.pos, sc.attr), rf.shader.Gouraud(), sc.mvp, sc.viewport,
                           rf.Framebuf(col[:480, :640], dep[:480, :640]), rf.Context(depth_sort="back_to_front"))
     assert e.value.status == -5
+
+
+def test_noalloc_takes_many_triangles_of_few_vertices():
+    """600,000 triangles over 60 vertices: nearly all of the array is the
+    triangles' own scratch."""
+    rng = np.random.default_rng(5)
+    pos = rng.uniform(-0.3, 0.3, size=(60, 3)).astype(np.float32)
+    tris = rng.integers(0, 60, size=(600000, 3)).astype(np.uint32)
+    attr = rng.uniform(0, 1, size=(60, 3)).astype(np.float32)
+    out = []
+    for fn in (rf.render, rf.render_noalloc):
+        col, dep = np.zeros((16, 16, 4), np.uint8), np.zeros((16, 16), np.float32)
+        ctx = rf.Context()
+        fn(tris, (pos, attr), rf.shader.Gouraud(), M.identity(),
+           M.viewport(0, 16, 16, 0), rf.Framebuf(col, dep), ctx)
+        s = ctx.stats
+        out.append((col, dep.view(np.uint32), [s.prims_o, s.frags_i, s.frags_o]))
+    assert np.array_equal(out[0][0], out[1][0]) and out[0][0].any()
+    assert np.array_equal(out[0][1], out[1][1])
+    assert out[0][2] == out[1][2]
