@@ -151,7 +151,7 @@ constexpr uint32_t RUNS_MULTI = 1u << 31;  // n_runs bit: Run::multi
 
 // Bounds of a group's binned triangles: the rasterizer drops a whole run by them.
 struct alignas(16) GroupBound {
-    float zmax;       // no fragment's z is above it (+inf: not known)
+    float zmax;       // no fragment's z is above it (NaN: not known)
     uint32_t r0, r1;  // the union of their BatchDesc::rect
     uint32_t pad;
 };
@@ -204,7 +204,7 @@ struct BatchDesc {
     uint32_t* extra_count;
     uint32_t extra_cap;
     uint32_t* rect;      // per triangle: pixel rect (c0 | r0 << 16, c1 | r1 << 16; all ones: none), 2 words
-    float* zmax;         // per triangle: no fragment's z is above it (+inf: not known)
+    float* zmax;         // per triangle: no fragment's z is above it (NaN: not known)
     GroupBound* group_max;  // per group; written where small_tris is set
     uint32_t* tile_of;   // per group, PRE_RUNS: its runs' tiles, and
     unsigned long long* mask_of;  // masks, as k_setup has met them
