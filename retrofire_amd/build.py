@@ -29,7 +29,7 @@ SOURCES = [
     ("rf_noalloc", "rf_noalloc.cpp", []),
     ("rf_copy", "rf_copy.cpp", []),
 ]
-HEADERS = ["rf_types.hpp", "rf_math.hpp", "rf_internal.hpp"]
+HEADERS = ["rf_types.hpp", "rf_math.hpp", "rf_internal.hpp", "rf_handout.hpp"]
 ARCH = os.environ.get("RF_OFFLOAD_ARCH", "gfx950")
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")

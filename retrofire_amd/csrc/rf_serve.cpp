@@ -35,13 +35,13 @@
 #include <condition_variable>
 #include <cstring>
 #include <deque>
-#include <map>
 #include <mutex>
 #include <new>
 #include <thread>
 #include <vector>
 
 #include "../../include/retrofire_amd.h"
+#include "rf_handout.hpp"
 #include "rf_internal.hpp"
 
 #ifndef RF_SERVE_CHUNK
@@ -72,57 +72,6 @@ constexpr double COST_LAUNCH = 1.0e7;
 #endif
 constexpr double SERVE_SLOWDOWN = RF_SERVE_SLOWDOWN;
 constexpr size_t SERVE_SCAN = 256;  // pending requests looked at per launch
-constexpr uint64_t ALIGN = 256;
-inline uint64_t align_up(uint64_t x) { return (x + ALIGN - 1) & ~(ALIGN - 1); }
-
-// First-fit allocator over a byte range; free ranges coalesce. Not locked:
-// the device arena is used by the worker thread only, the pinned read-back
-// block under Serve::pm.
-struct Arena {
-    uint8_t* base = nullptr;
-    uint64_t size = 0, used = 0;
-    std::map<uint64_t, uint64_t> free_;  // offset -> bytes
-    void init(uint8_t* b, uint64_t n) {
-        base = b;
-        size = n;
-        used = 0;
-        free_.clear();
-        if (n) free_[0] = n;
-    }
-    uint64_t largest() const {
-        uint64_t m = 0;
-        for (const auto& kv : free_) m = std::max(m, kv.second);
-        return m;
-    }
-    bool alloc(uint64_t bytes, uint64_t& off) {
-        for (auto it = free_.begin(); it != free_.end(); ++it) {
-            if (it->second < bytes) continue;
-            off = it->first;
-            const uint64_t rest = it->second - bytes;
-            free_.erase(it);
-            if (rest) free_[off + bytes] = rest;
-            used += bytes;
-            return true;
-        }
-        return false;
-    }
-    void release(uint64_t off, uint64_t bytes) {
-        used -= bytes;
-        auto it = free_.emplace(off, bytes).first;
-        auto nx = std::next(it);
-        if (nx != free_.end() && it->first + it->second == nx->first) {
-            it->second += nx->second;
-            free_.erase(nx);
-        }
-        if (it != free_.begin()) {
-            auto pv = std::prev(it);
-            if (pv->first + pv->second == it->first) {
-                pv->second += it->second;
-                free_.erase(it);
-            }
-        }
-    }
-};
 
 struct Req {
     rf_request r;
@@ -132,11 +81,6 @@ struct Req {
     bool sorted = false;  // depth_sort with a triangle draw: launched alone, through the lane's sort pass
 };
 
-struct Done {
-    rf_result res;
-    uint8_t* pixels = nullptr;  // pinned, width * height * bpp
-    size_t pix_bytes = 0;
-};
 constexpr uint32_t STAGE_DRAWS = 8;  // draws per frame the staging is sized for at open
 
 // Counts of a launch: what its block must hold.
@@ -190,7 +134,7 @@ struct Lane {
 
 }  // namespace
 
-struct Serve {
+struct Serve : Handout {
     Device* dev = nullptr;
     void* arena_mem = nullptr;
     Arena arena;             // worker thread only
@@ -200,15 +144,10 @@ struct Serve {
     double extra_ratio = 1.0 / 16, runs_ratio = 8.0;
     std::vector<Lane*> lanes;
     std::thread worker;
-    std::mutex m;
-    std::condition_variable cv_work, cv_done;
     std::deque<Req> pending;
-    std::deque<Done> done;
     bool stop = false;
     bool stop_waiters = false;
-    std::mutex pm;  // guards `pin`; never held across a HIP call (taken after `m`)
-    void* pin_mem = nullptr;
-    Arena pin;      // read-back buffers in the pinned block
+    void* pin_mem = nullptr;  // the block that Handout::pin manages
     std::unique_ptr<CopyPool> pool;  // copies results to the callers of rf_serve_poll
     uint64_t sort_bytes = 0;  // device memory of the lanes' depth-sort buffers (worker thread only)
 };
@@ -229,29 +168,6 @@ static void waiter_main(Serve* sp, Lane* l) {
         l->done_s = t;
         l->finished.store(1);
         s.cv_work.notify_all();
-    }
-}
-
-// Read-back buffer of `bytes` from the pinned block (nullptr if it does not
-// fit now). Called with `m` held.
-static uint8_t* pin_take(Serve& s, size_t bytes) {
-    std::lock_guard<std::mutex> g(s.pm);
-    uint64_t off = 0;
-    if (!s.pin.alloc(align_up(bytes), off)) return nullptr;
-    return s.pin.base + off;
-}
-static bool pin_in_block(const Serve& s, const uint8_t* p) {
-    return p >= s.pin.base && p < s.pin.base + s.pin.size;
-}
-// Returns a read-back buffer: to the pinned block, or (a frame larger than
-// the block) to the host.
-static void pin_put(Serve& s, uint8_t* p, size_t bytes) {
-    if (!p) return;
-    if (pin_in_block(s, p)) {
-        std::lock_guard<std::mutex> g(s.pm);
-        s.pin.release((uint64_t)(p - s.pin.base), align_up(bytes));
-    } else {
-        (void)hipHostFree(p);
     }
 }
 
@@ -709,7 +625,7 @@ static void worker_main(Serve* sp) {
                 // whole pinned block) allocated at launch
                 const size_t pb = (size_t)q.r.width * q.r.height * bytes_per_pixel(q.r.fmt);
                 uint8_t* pin = nullptr;
-                if (align_up(pb) <= s.pin.size && !(pin = pin_take(s, pb))) break;  // wait for polls
+                if (align_up(pb) <= s.pin.size && !(pin = s.pin_take(pb))) break;  // wait for polls
                 l->pix.push_back(pin);
                 l->pix_bytes.push_back(pb);
                 p = p2;
@@ -727,7 +643,7 @@ static void worker_main(Serve* sp) {
             if (!take_block(s, *l)) {  // cannot happen: the block fits `room`
                 for (auto it = l->reqs.rbegin(); it != l->reqs.rend(); ++it) s.pending.push_front(std::move(*it));
                 l->reqs.clear();
-                for (size_t k = 0; k < l->pix.size(); ++k) pin_put(s, l->pix[k], l->pix_bytes[k]);
+                for (size_t k = 0; k < l->pix.size(); ++k) s.pin_put(l->pix[k], l->pix_bytes[k]);
                 l->pix.clear();
                 l->pix_bytes.clear();
                 continue;
@@ -796,7 +712,7 @@ rf_status rf_serve_open(rf_device* dev, uint64_t budget_bytes, uint32_t max_batc
     if (!s) return RF_E_DEVICE;
     s->dev = &d;
     s->max_batch = max_batch;
-    budget_bytes &= ~(ALIGN - 1);
+    budget_bytes &= ~(ARENA_ALIGN - 1);
     if (!budget_bytes || hipMalloc(&s->arena_mem, budget_bytes)) {
         delete s;
         return RF_E_DEVICE;
@@ -869,23 +785,11 @@ rf_status rf_serve_poll(rf_serve* sh, rf_result* out, void** color, uint32_t max
                         uint32_t timeout_ms) {
     if (!sh || !out || !n_out) return RF_E_ARG;
     Serve& s = *reinterpret_cast<Serve*>(sh);
-    std::unique_lock<std::mutex> lk(s.m);
-    if (s.done.empty() && timeout_ms)
-        s.cv_done.wait_for(lk, std::chrono::milliseconds(timeout_ms), [&] { return !s.done.empty(); });
-    std::vector<Done> got;
-    while (got.size() < max && !s.done.empty()) {
-        got.push_back(s.done.front());
-        s.done.pop_front();
-    }
-    lk.unlock();
-    // The pixels are copied without the lock (the worker admits and the waiters
-    // report meanwhile) and by several threads: one copies at about 20 GB/s, and
+    // The pixels are copied by several threads: one copies at about 20 GB/s, and
     // a burst's frames come down the link at 57.
-    const uint32_t n = (uint32_t)got.size();
-    for (uint32_t i = 0; i < n; ++i) {
-        const Done& d = got[i];
+    *n_out = s.hand_out(max, timeout_ms, [&](uint32_t i, const Done& d) {
         out[i] = d.res;
-        if (!d.pixels) continue;
+        if (!d.pixels) return;
         if (color && color[i]) {
             uint8_t* const to = (uint8_t*)color[i];
             const size_t rows = d.pix_bytes / 4096, rest = d.pix_bytes % 4096;
@@ -893,10 +797,8 @@ rf_status rf_serve_poll(rf_serve* sh, rf_result* out, void** color, uint32_t max
             else std::memcpy(to, d.pixels, rows * 4096);
             std::memcpy(to + rows * 4096, d.pixels + rows * 4096, rest);
         }
-        pin_put(s, d.pixels, d.pix_bytes);
-    }
-    *n_out = n;
-    if (n) s.cv_work.notify_all();  // admissions may wait for read-back space
+        if (!s.pin_in_block(d.pixels)) (void)hipHostFree(d.pixels);  // a frame larger than the block
+    });
     return RF_OK;
 }
 
@@ -932,7 +834,7 @@ rf_status rf_serve_close(rf_serve* sh) {
     }
     if (s->arena_mem) (void)hipFree(s->arena_mem);
     for (auto& d2 : s->done)
-        if (d2.pixels && !pin_in_block(*s, d2.pixels)) (void)hipHostFree(d2.pixels);
+        if (d2.pixels && !s->pin_in_block(d2.pixels)) (void)hipHostFree(d2.pixels);
     if (s->pin_mem) (void)hipHostFree(s->pin_mem);
     delete s;
     return RF_OK;
