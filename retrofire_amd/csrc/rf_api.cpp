@@ -237,7 +237,7 @@ rf_status run_sized(Device& d, Scratch& sc, BatchDesc& B, hipStream_t s,
 
 // ---- the plain path's pieces, shared by rf_render and rf_render_noalloc ----
 
-// Largest target read back, and largest upload, through pinned memory.
+// Largest target, and largest inputs, that go through pinned memory.
 constexpr size_t STAGE_DOWN_MAX = 256ull << 20, STAGE_UP_MAX = 128ull << 20;
 static size_t up256(size_t x) { return (x + 255) & ~size_t(255); }
 
@@ -492,12 +492,13 @@ rf_status rf_render(rf_device* dev, const rf_draw* draw, rf_target* target, cons
     hipStream_t s = d.stream;
     // Copies from and to pageable memory are staged by the runtime, one after
     // another, each a wait: a two-triangle call spent 0.15 of 0.22 ms on eleven
-    // of them, a 1920x1080 frame's read-back ran at 17 GB/s. So what goes up is
-    // collected in pinned memory and goes as one copy; what comes down (the
+    // of them, a 1920x1080 frame's read-back ran at 17 GB/s. So the inputs are
+    // collected in pinned memory and go up as one copy; what comes down (the
     // counters and, on the chance that they report no error, the target) comes
     // into pinned memory in parts, and each part goes on into the caller's while
-    // the next arrives. Inputs and targets beyond the limits
-    // go directly, as do all if no pinned memory can be had.
+    // the next arrives. A target that is not cleared goes up through the memory
+    // it comes down through. Larger inputs and targets go directly, as do all if
+    // no pinned memory can be had.
     PlainLayout L = plain_layout_packed(draw, target);
     bool staged = L.col_b + L.dep_b <= STAGE_DOWN_MAX && d.stage_down.ensure(STATS_OFF + 4096 + L.col_b + L.dep_b);
     if (!staged) L = plain_layout(draw, target);
@@ -519,39 +520,33 @@ rf_status rf_render(rf_device* dev, const rf_draw* draw, rf_target* target, cons
     plain_descs(draw, target, ctx, L, P, d.plain_tile_w, d.plain_tile_h, d.plain_chunk, dd, fd, B);
     uint8_t* desc = (uint8_t*)P.desc;
     const size_t o_fd = (const uint8_t*)B.frames - up;
-    const bool up_col = !ctx->clear_color, up_dep = target->depth && !ctx->clear_depth;
-    const size_t in_end = o_col, up_end = up_dep ? end : up_col ? o_dep : in_end;
-    const bool staged_up = staged && up_end <= STAGE_UP_MAX && d.stage_up.ensure(up_end);
-    // the target's own content, where it is not cleared (again before a rerun)
+    const bool staged_in = staged && o_col <= STAGE_UP_MAX && d.stage_up.ensure(o_col);
+    uint8_t* const down = d.stage_down.p;
+    uint8_t* const pix = staged ? down + up256(report_bytes(1)) : nullptr;  // colour, then depth, as on the device
+    // the target's own content, where it is not cleared (again before a rerun,
+    // whose aborted run has been read back over it)
     auto upload_target = [&]() -> hipError_t {
         if (!staged) return plain_upload_target(target, ctx, L, P, s);
         hipError_t e = hipSuccess;
-        uint8_t* const h = d.stage_up.p;
-        if (up_col)
-            e = staged_up ? hipMemcpyAsync(P.color, h + o_col, L.col_b, hipMemcpyHostToDevice, s)
-                          : hipMemcpy2DAsync(P.color, L.col_pitch, target->color, target->color_stride, L.col_row,
-                                             target->height, hipMemcpyHostToDevice, s);
-        if (!e && up_dep)
-            e = staged_up ? hipMemcpyAsync(P.depth, h + o_dep, L.dep_b, hipMemcpyHostToDevice, s)
-                          : hipMemcpy2DAsync(P.depth, L.dep_pitch_f * 4, target->depth,
-                                             (size_t)target->depth_stride * 4, L.dep_row, target->height,
-                                             hipMemcpyHostToDevice, s);
+        if (!ctx->clear_color) {
+            copy({pix, (const uint8_t*)target->color, L.col_pitch, target->color_stride, L.col_row, target->height});
+            e = hipMemcpyAsync(P.color, pix, L.col_b, hipMemcpyHostToDevice, s);
+        }
+        if (!e && target->depth && !ctx->clear_depth) {
+            copy({pix + (o_dep - o_col), (const uint8_t*)target->depth, L.dep_pitch_f * 4,
+                  (size_t)target->depth_stride * 4, L.dep_row, target->height});
+            e = hipMemcpyAsync(P.depth, pix + (o_dep - o_col), L.dep_b, hipMemcpyHostToDevice, s);
+        }
         return e;
     };
-    if (staged_up) {
+    if (staged_in) {
         uint8_t* const h = d.stage_up.p;
         std::memcpy(h, &dd, sizeof(dd));
         std::memcpy(h + o_fd, &fd, sizeof(fd));
         for (const Part& p : {Part{draw->pos, o_pos, L.pos_b}, Part{draw->attr, o_attr, L.attr_b},
                               Part{draw->tris, o_tris, L.tri_b}, Part{draw->tex, o_tex, L.tex_b}})
             if (p.bytes) std::memcpy(h + p.off, p.src, p.bytes);
-        if (hipMemcpyAsync(up, h, in_end, hipMemcpyHostToDevice, s)) return RF_E_DEVICE;
-        if (up_col)
-            copy({h + o_col, (const uint8_t*)target->color, L.col_pitch, target->color_stride, L.col_row,
-                    target->height});
-        if (up_dep)
-            copy({h + o_dep, (const uint8_t*)target->depth, L.dep_pitch_f * 4, (size_t)target->depth_stride * 4,
-                    L.dep_row, target->height});
+        if (hipMemcpyAsync(up, h, o_col, hipMemcpyHostToDevice, s)) return RF_E_DEVICE;
     } else if (plain_upload_inputs(draw, L, P, s) || hipMemcpyAsync(desc, &dd, sizeof(dd), hipMemcpyHostToDevice, s) ||
                hipMemcpyAsync((void*)B.frames, &fd, sizeof(fd), hipMemcpyHostToDevice, s)) {
         return RF_E_DEVICE;
@@ -610,9 +605,7 @@ rf_status rf_render(rf_device* dev, const rf_draw* draw, rf_target* target, cons
     }
     for (hipEvent_t& e : d.down_ev)
         if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming)) return RF_E_DEVICE;
-    uint8_t* const down = d.stage_down.p;
-    uint8_t* const pix = down + up256(report_bytes(1));
-    const size_t span = o_dep + L.dep_b - o_col;  // colour, then depth, as on the device
+    const size_t span = o_dep + L.dep_b - o_col;
     // parts of whole 64 KiB, at least 1 MiB
     const size_t part = std::max<size_t>(1 << 20, (span / DOWN_CHUNKS + 0x10000) & ~size_t(0xFFFF));
     uint32_t misc[RUNS_WORD + 1];
