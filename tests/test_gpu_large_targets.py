@@ -48,7 +48,10 @@ def seconds(draw, col, dep, clear):
 
 # (width, height, columns around the colour view, around the depth view, cleared)
 CASES = {"kept, 131 MiB, rows of no 16 bytes": (4099, 4200, 0, 0, False),
-         "kept view, 131 MiB": (4099, 4200, 5, 3, False)}
+         "kept view, 131 MiB": (4099, 4200, 5, 3, False),
+         "view of 281 MiB": (16001, 2300, 6, 2, True),
+         "colour view of 281 MiB, kept": (16001, 2300, 6, 0, False),
+         "depth view of 281 MiB, kept": (16001, 2300, 0, 2, False)}
 
 
 @pytest.mark.parametrize("case", CASES)
