@@ -165,7 +165,11 @@ typedef struct rf_serve rf_serve;
 rf_status rf_device_open(int ordinal, rf_device** out);
 rf_status rf_device_close(rf_device* dev);
 const char* rf_status_str(rf_status s);
-/* Bytes of device memory the library holds for scratch and residency. */
+/* Bytes of device memory the library holds for scratch and residency. Not in
+ * it: the pinned host memory that rf_render copies through, kept from call to
+ * call until rf_device_close. That is the size of the largest target so far (of
+ * those up to 256 MiB) and of the largest inputs (of those up to 128 MiB), each
+ * with a quarter more, at most 16 MiB. */
 uint64_t rf_device_bytes(const rf_device* dev);
 /* Rasterizer tile width (16, 32 or 64 pixel columns; 0 = the default, 32) used by
  * rf_render on this device. No counterpart in the reference (a tuning knob of

@@ -28,6 +28,7 @@ SOURCES = [
     ("rf_dsort", "rf_dsort.cpp", []),
     ("rf_noalloc", "rf_noalloc.cpp", []),
     ("rf_copy", "rf_copy.cpp", []),
+    ("rf_pin", "rf_pin.cpp", []),
 ]
 HEADERS = ["rf_types.hpp", "rf_math.hpp", "rf_internal.hpp", "rf_handout.hpp"]
 ARCH = os.environ.get("RF_OFFLOAD_ARCH", "gfx950")

@@ -48,23 +48,6 @@ void DevBuf::release(uint64_t* counter) {
     cap = 0;
 }
 
-bool PinBuf::ensure(size_t bytes) {
-    if (bytes <= cap) return true;
-    release();
-    const size_t want = (bytes + bytes / 4 + 4095) & ~size_t(4095);
-    if (hipHostMalloc((void**)&p, want, 0)) {
-        p = nullptr;
-        return false;
-    }
-    cap = want;
-    return true;
-}
-void PinBuf::release() {
-    if (p) (void)hipHostFree(p);
-    p = nullptr;
-    cap = 0;
-}
-
 uint32_t bytes_per_pixel(uint32_t fmt) { return pixfmt_bytes(fmt); }
 
 uint32_t pack_clear(uint32_t fmt, const uint8_t* c) { return pack_pixel(fmt, c[0], c[1], c[2], c[3]); }

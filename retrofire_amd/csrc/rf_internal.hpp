@@ -123,11 +123,13 @@ private:
     std::atomic<int> inside{0};  // threads at work on the job
 };
 
-// Pinned host memory, grow-only.
+// Pinned host memory, grow-only (rf_pin.cpp): a quarter more than asked for, at
+// most PIN_SLACK.
+constexpr size_t PIN_SLACK = 16ull << 20;
 struct PinBuf {
     uint8_t* p = nullptr;
     size_t cap = 0;
-    bool ensure(size_t bytes);  // false: none to be had (the old block is gone)
+    bool ensure(size_t bytes);  // false: none to be had; what was held still is
     void release();
 };
 
