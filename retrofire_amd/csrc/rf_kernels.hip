@@ -1550,11 +1550,14 @@ constexpr int CELL_W = RF_CELL_W;    // pixel columns per ordering cell
 // workgroups a CU holds (registers allow eight), so a tile's batch takes what
 // its pixels leave of the smallest share that holds 128 records: 1/8 of the
 // CU's 160 KB, else 1/6, 1/5, 1/4 or 1/3 (in the allocation's 1,280-byte
-// steps); tiles of 64 rows, whose triangles are taller, hold 384. Longer batches start fewer half-empty rounds: at 32 x 32 tiles, 8
-// icospheres1080 frames, 128 records and 32 triangles 2.63 ms, 192 and 64
-// 2.55, 256 and 32 2.35. (A batch's first triangle has at most th rows in a
-// tile, unless rows above the target fold onto row 0.)
+// steps). Tiles of 64 rows, whose triangles are taller, ask for 384 (and hold
+// 448, 480 and, of the third that is the largest share, 320). Longer batches
+// start fewer half-empty rounds: at 32 x 32 tiles, 8 icospheres1080 frames, 128
+// records and 32 triangles 2.63 ms, 192 and 64 2.55, 256 and 32 2.35. (A batch's
+// first triangle has at most th rows in a tile, unless rows above the target
+// fold onto row 0.)
 constexpr int REC_BYTES = 25;  // an EdgeRec and its owner
+constexpr int LDS_THIRD = 53760;
 __host__ __device__ constexpr int lds_fixed(int tw, int th, int slots) {
     return 9 * tw * (th + 1) + 4 * th * (tw / CELL_W) + 4 * (FQ_CAP + 64) + 4 * (slots + WAVE) + 64 * slots;
 }
@@ -1563,7 +1566,7 @@ __host__ __device__ constexpr int n_slot(int tw, int th) {
 }
 __host__ __device__ constexpr int rec_cap(int tw, int th) {
     const int f = lds_fixed(tw, th, n_slot(tw, th)), min = f + (th > 32 ? 384 : 128) * REC_BYTES;
-    const int share = min <= 20480 ? 20480 : min <= 26880 ? 26880 : min <= 32000 ? 32000 : min <= 40960 ? 40960 : 53760;
+    const int share = min <= 20480 ? 20480 : min <= 26880 ? 26880 : min <= 32000 ? 32000 : min <= 40960 ? 40960 : LDS_THIRD;
     const int r = (share - f) / REC_BYTES / 32 * 32;
     return r < 480 ? r : 480;
 }
@@ -1678,6 +1681,8 @@ __global__ __launch_bounds__(64, 2) void k_raster(BatchDesc B) {
     constexpr int REC_CAP = rec_cap(TW, TH);
     constexpr int NSLOT = n_slot(TW, TH);
     constexpr int DQ_CAP = NSLOT + WAVE;
+    static_assert(REC_CAP >= TILE_H, "a batch's first triangle fits");
+    static_assert(lds_fixed(TW, TH, NSLOT) + REC_CAP * REC_BYTES <= LDS_THIRD, "three workgroups a CU at least");
     constexpr int LD = TILE_H + 1;  // padded column stride in LDS (bank spread)
     constexpr int NPX = TW * LD;
     constexpr int CW = CELL_W < TW ? CELL_W : TW;  // ordering cell width in this tile
