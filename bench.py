@@ -146,7 +146,7 @@ def main():
 
     # per-kernel durations (HIP events on the batch stream, eager launches)
     prof = batch.profile(iters=max(3, min(10, a.steps)))
-    names = ["vertex", "setup", "scan", "bin", "binsort", "raster"]
+    names = ["reset", "setup", "scan", "bin", "binsort", "raster"]
     raster_ms = prof[5]
     bytes_per_frame_raster = W * H * (4 + 4) + tex.nbytes  # colour + depth written once, texture once
     alg_bytes = bytes_per_frame_raster * a.frames
@@ -425,7 +425,7 @@ def c3_run(rf, RB, a, W_steps):
            "frags_o_per_step": int(sum(s.frags_o for s in stats)),
            "tile_w": b.tile_w, "tile_h": b.tile_h, "chunk": b.chunk, "plan_s": round(plan_s, 2),
            "autotune_ms": [list(t) for t in b.tune_results()],
-           "stage_ms": {n: round(x, 4) for n, x in zip(["vertex", "setup", "scan", "bin", "binsort", "raster"], prof)},
+           "stage_ms": {n: round(x, 4) for n, x in zip(["reset", "setup", "scan", "bin", "binsort", "raster"], prof)},
            "raster_roofline": {"alg_bytes_per_launch": alg, "launch_ms": round(prof[5], 4),
                                "achieved_GBs": round(alg / (prof[5] * 1e-3) / 1e9, 1),
                                "frac": round(alg / (prof[5] * 1e-3) / 1e9 / HBM_PEAK_GBS, 4)}}
@@ -461,7 +461,7 @@ def c2_run(rf, RB, a, W_steps, n_frames=8):
            "mfrag_per_s": round(sum(s.frags_i for s in stats) * W_steps / el / 1e6, 1),
            "tile_w": b.tile_w, "tile_h": b.tile_h, "chunk": b.chunk,
            "autotune_ms": [list(t) for t in b.tune_results()],
-           "stage_ms": {n: round(x, 4) for n, x in zip(["vertex", "setup", "scan", "bin", "binsort", "raster"], prof)},
+           "stage_ms": {n: round(x, 4) for n, x in zip(["reset", "setup", "scan", "bin", "binsort", "raster"], prof)},
            "raster_roofline": {"alg_bytes_per_launch": alg, "launch_ms": round(prof[5], 4),
                                "achieved_GBs": round(alg / (prof[5] * 1e-3) / 1e9, 1),
                                "frac": round(alg / (prof[5] * 1e-3) / 1e9 / HBM_PEAK_GBS, 4)}}

@@ -173,8 +173,8 @@ class Batch:
         return t.value
 
     def profile(self, iters=5):
-        """Mean ms of vertex, setup, scan, bin, binsort, raster (eager run with
-        HIP events on the batch stream)."""
+        """Mean ms of counter reset (with culling), setup, scan, bin, binsort,
+        raster (eager run with HIP events on the batch stream)."""
         ms = (C.c_float * 6)()
         check(_ffi.lib().rf_batch_profile(self.h, iters, ms))
         return list(ms)

@@ -43,7 +43,7 @@ constexpr auto LINGER = std::chrono::microseconds(200);
 
 CopyPool::CopyPool() {
     const unsigned cores = std::thread::hardware_concurrency();
-        const unsigned n = std::min(4u, cores > 1 ? cores - 1 : 0u);
+    const unsigned n = std::min(4u, cores > 1 ? cores - 1 : 0u);
     try {
         for (unsigned i = 0; i < n; ++i) threads.emplace_back([this] { worker(); });
     } catch (...) {  // fewer threads, or none: the caller copies what they do not

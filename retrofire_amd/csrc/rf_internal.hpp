@@ -248,7 +248,7 @@ hipError_t launch_fan_gather(const BatchDesc& P, const BatchDesc& M, const uint3
 rf_status sortpass_plan(Device& d, SortPass& S, hipStream_t s, uint64_t* counter, uint32_t* err_out);
 // Uploads the (first position, main draw) table once main_of is set.
 hipError_t sortpass_map(SortPass& S, hipStream_t s);
-// P's pass (reset, culling, vertex shader, clip fans and keys).
+// P's pass (reset, culling, clip fans and keys).
 hipError_t sortpass_fans(const SortPass& S, hipStream_t s);
 // The sorts and the gather into M (whose pre draws and scratch are in place).
 hipError_t sortpass_sort_gather(const SortPass& S, const BatchDesc& M, hipStream_t s);

@@ -968,7 +968,7 @@ __global__ __launch_bounds__(256, 6) void k_setup(BatchDesc B) {
         if (lane == 0) B.group_max[group] = gb;
     }
     // prims.o (render.rs:195; verts.o is 3 per primitive, derived in
-    // k_scan_top) and the small triangles' frags.i: one atomic each per wave
+    // scan_totals) and the small triangles' frags.i: one atomic each per wave
     // when the wave's triangles all belong to one frame, else one per lane,
     // into the group's partial counters
     {
